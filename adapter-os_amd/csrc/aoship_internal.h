@@ -559,6 +559,7 @@ typedef struct {
 
 /* ---- full decoder step (embedding, norms, RoPE + KV cache, attention) ---- */
 #define AOS_ATTN_MAX_HD 256
+#define AOS_ATTN_PREFILL_ROWS 2048 /* (token, head) rows from which a prompt's attention runs on the matrix cores */
 typedef struct {
   const int32_t *ids; /* [T] */
   int T, H, vocab;
@@ -568,6 +569,7 @@ typedef struct {
   const uint16_t *bf16;   /* [vocab][H] bfloat16 rows when q4 is NULL */
   float *hidden;          /* [T][H] float32 */
   int32_t *status;        /* set to 1 when an id is out of range (that row is zero) */
+  uint32_t *clear;        /* a word set to 0 (a fresh cache's nonfinite flag), or NULL */
 } aos_embed_params;
 
 typedef struct {
@@ -586,6 +588,7 @@ typedef struct {
   int T, nh, nkv, hd, offset, max_seq;
   float *qr;                 /* [T][nh][hd] float32, rotated */
   uint16_t *kc, *vc;         /* [nkv][max_seq][hd] bf16 caches of this layer */
+  uint32_t *nonfinite;       /* set to 1 when an infinity or NaN enters the cache */
 } aos_rope_params;
 
 typedef struct {
@@ -606,6 +609,9 @@ typedef struct {
   const uint16_t *qb, *kb, *vb;
   const float *bq, *bk, *bv;
   const float *inv_freq;
+  /* set to 1 (rope_fused) when an infinity or NaN enters the cache; the prompt kernel reads it */
+  uint32_t *nonfinite;
+  int prefill; /* 1: the prompt kernel (head_dim 64 or 128, rotated queries, no splits) */
 } aos_attn_params;
 
 #define AOS_LAUNCH(ctx, kernel, grid, block, lds, ...)                                            \
@@ -650,6 +656,7 @@ int aos_launch_route(const aos_route_params *p, const aos_launch_ctx *ctx);
 int aos_launch_embed(const aos_embed_params *p, const aos_launch_ctx *ctx);
 int aos_launch_norm(const aos_norm_params *p, const aos_launch_ctx *ctx);
 int aos_launch_rope(const aos_rope_params *p, const aos_launch_ctx *ctx);
+int aos_attn_prefill_fits(int hd, int max_seq); /* 1: the prompt kernel takes this head_dim and cache */
 int aos_launch_attention(const aos_attn_params *p, const aos_launch_ctx *ctx);
 int aos_launch_shrink(const aos_shrink_params *p, const aos_launch_ctx *ctx);
 int aos_launch_gemv(const aos_gemv_params *p, int swiglu, const aos_launch_ctx *ctx);

@@ -11,9 +11,10 @@
  *                             inv_freq_i = 1 / theta^(-2i / hd), angle = position * inv_freq_i;
  *                             K and V appended to a bf16 cache laid out [kv head][position][hd]
  *   attention                 causal scaled dot-product attention over the cache, GQA by head
- *                             group (…real.cpp:3282-3327): one wave per (split of positions,
- *                             head, token) with an online softmax in float32, then a fixed-order
- *                             merge of the splits
+ *                             group (…real.cpp:3282-3327), with an online softmax in float32:
+ *                             decode and short prompts by one wave per (split of positions, head,
+ *                             token) and a fixed-order merge of the splits; prompts by 128-token
+ *                             tiles on the matrix cores
  *
  * Every reduction has a fixed order, so results are bit-identical run to run.
  */
@@ -29,6 +30,7 @@ namespace {
  * the launch is in flight at once. */
 __global__ void __launch_bounds__(256) aos_embed_kernel(aos_embed_params p) {
   const int t = blockIdx.y, g = blockIdx.x * 256 + threadIdx.x;
+  if (t == 0 && g == 0 && p.clear) *p.clear = 0u;
   if (8 * g >= p.H) return;
   const int id = p.ids[t];
   float4 *dst = (float4 *)(p.hidden + (size_t)t * p.H + 8 * g);
@@ -124,6 +126,9 @@ __global__ void __launch_bounds__(1024) aos_norm_kernel(aos_norm_params p) {
 
 /* ---- RoPE, biases, KV cache append ---------------------------------------------------------- */
 
+/* A bfloat16 infinity or NaN. */
+__device__ __forceinline__ bool bf16_nonfinite(uint32_t b) { return (b & 0x7f80u) == 0x7f80u; }
+
 /* One thread per rotated pair of q or k, or per element of v. */
 __global__ void __launch_bounds__(256) aos_rope_kernel(aos_rope_params p) {
   const int t = blockIdx.y, half = p.hd / 2;
@@ -153,15 +158,19 @@ __global__ void __launch_bounds__(256) aos_rope_kernel(aos_rope_params p) {
       dst[i + half] = r2;
     } else {
       uint16_t *dst = p.kc + ((size_t)h * p.max_seq + pos) * p.hd;
-      dst[i] = aos_f32_to_bf16(r1);
-      dst[i + half] = aos_f32_to_bf16(r2);
+      const uint16_t b1 = aos_f32_to_bf16(r1), b2 = aos_f32_to_bf16(r2);
+      dst[i] = b1;
+      dst[i + half] = b2;
+      if (bf16_nonfinite(b1) || bf16_nonfinite(b2)) *p.nonfinite = 1u;
     }
   } else {
     const int idx = w - nq - nk;
     const int h = idx / p.hd, d = idx - h * p.hd;
     float v = aos_bf16_to_f32(p.v[(size_t)t * nv + idx]);
     if (p.bv) v = v + p.bv[idx];
-    p.vc[((size_t)h * p.max_seq + pos) * p.hd + d] = aos_f32_to_bf16(v);
+    const uint16_t b = aos_f32_to_bf16(v);
+    p.vc[((size_t)h * p.max_seq + pos) * p.hd + d] = b;
+    if (bf16_nonfinite(b)) *p.nonfinite = 1u;
   }
 }
 
@@ -307,6 +316,8 @@ __global__ void __launch_bounds__(64) aos_attn_kernel(aos_attn_params p) {
                 kdst[i] = b1;
                 kdst[i + hw] = b2;
                 vdst[i] = o;
+                if (bf16_nonfinite(b1) || bf16_nonfinite(b2) || bf16_nonfinite(o) || bf16_nonfinite(o >> 16))
+                  *p.nonfinite = 1u;
               }
             }
           }
@@ -498,6 +509,285 @@ __global__ void __launch_bounds__(64) aos_attn_merge_kernel(aos_attn_params p) {
   attn_merge<DPL>(p, blockIdx.x, blockIdx.y, threadIdx.x, fs, lf);
 }
 
+/* ---- attention of a prompt on the matrix cores ------------------------------------------------ */
+
+/* Four waves cover 128 tokens of one head, each wave 32 (one per MFMA column); the keys and values of
+ * the causal range go by in tiles of 64 positions, straight from memory to a two-stage LDS ring the
+ * waves share (64 KB: two workgroups per CU, so one's softmax runs under the other's MFMAs).
+ *
+ * Scores: S^T[key][token] = K . Q^T. The keys are bfloat16; the float32 query is held as three
+ * bfloat16 pieces (the top 8, the next 8 and the last 8 bits of its significand, by truncation: the
+ * split is exact), so three MFMAs give the float32 products, summed in float32. The row of K on MFMA
+ * row r is key swap23(r) (bits 2 and 3 exchanged), which puts on lane (token, half c), register
+ * 8 s + e, the score of key 16 s + 8 c + e: the B operand layout of the second product, so the
+ * probabilities never cross lanes.
+ *
+ * Output: O^T[d][token] = V^T . P^T, the float32 probabilities split the same way (three MFMAs, P
+ * exact); V^T fragments come from the row-major value tile through ds_read_b64_tr_b16 (a 16-lane
+ * group reads 4 keys x 16 dimensions, lane l receiving column l of the 4 rows). Online softmax in
+ * float32, one token per lane pair; the output is rescaled only where a maximum grew.
+ *
+ * LDS chunks (16 bytes) are swizzled so that neither read conflicts: key rows by their row, value rows
+ * by the two row bits a transposed read spans.
+ *
+ * Bound by the matrix cores (three MFMAs for each of the plain bfloat16 products) and the float32
+ * exponentials and splits between them. One layer of 1900 tokens, 28 heads of 128, 4 key/value heads: 132 us
+ * (26 GFLOP of products over the causal half; 82 GFLOP executed, with the pieces and the masked parts of the
+ * edge tiles: 620 TFLOP/s) against 2452 us for the wave per (token, head), which reads every visible key and
+ * value row once per token. */
+constexpr int PA_BQ = 128; /* tokens per workgroup */
+constexpr int PA_BK = 64;  /* positions per tile */
+
+/* float32 pair -> its top 8, next 8 and last 8 significand bits as packed bfloat16 pairs */
+__device__ __forceinline__ void split3(float a, float b, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
+  const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
+  hi = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
+  const float ra = a - __builtin_bit_cast(float, ua & 0xffff0000u);
+  const float rb = b - __builtin_bit_cast(float, ub & 0xffff0000u);
+  const uint32_t va = __builtin_bit_cast(uint32_t, ra), vb = __builtin_bit_cast(uint32_t, rb);
+  mid = __builtin_amdgcn_perm(vb, va, 0x07060302u);
+  const float sa = ra - __builtin_bit_cast(float, va & 0xffff0000u);
+  const float sb = rb - __builtin_bit_cast(float, vb & 0xffff0000u);
+  lo = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, sb), __builtin_bit_cast(uint32_t, sa), 0x07060302u);
+}
+
+/* e^x for x <= 0 through the hardware's 2^t: t = x log2(e) rounded, its rounding error and the
+ * constant's low part put back to first order. x below -200 (and -infinity) gives 0; NaN stays NaN. */
+__device__ __forceinline__ float exp_neg(float x) {
+  const float L2E = 1.44269502f, L2E_LO = 1.92596303e-8f, LN2 = 0.693147182f;
+  x = x < -200.0f ? -200.0f : x;
+  const float t = x * L2E;
+  const float r = fmaf(x, L2E_LO, fmaf(x, L2E, -t));
+  const float e = __builtin_amdgcn_exp2f(t);
+  return fmaf(e, r * LN2, e);
+}
+
+/* Group of DMA loads of a tile: LDS bytes base + 1024 b + 16 lane of blocks b = 4 k + wave; v[k] is the
+ * lane's byte offset in the first tile. Positions past the resource's end read as zeros. */
+template <int N>
+__device__ __forceinline__ void pa_dma(const uint16_t *src, int bytes, unsigned char *dst, int wave, const int *v,
+                                       int tile_bytes) {
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)src, (short)0, bytes, 0x00020000);
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        rs, (__attribute__((address_space(3))) void *)(dst + (4 * k + wave) * 1024), 16, v[k], tile_bytes, 0, 0);
+}
+
+/* One token on one wave with plain float32 arithmetic: the path of a cache that holds an infinity or
+ * a NaN, whose products with the zero pieces of a split would be NaN where the float32 product is not. */
+template <int HD>
+__device__ void attn_token_plain(const aos_attn_params &p, int h, int t, int lane, float *ps) {
+  const int kvh = h / (p.nh / p.nkv), visible = p.offset + t + 1;
+  const float *q = p.q + ((size_t)t * p.nh + h) * HD;
+  const uint16_t *kb = p.kc + (size_t)kvh * p.max_seq * HD;
+  const uint16_t *vb = p.vc + (size_t)kvh * p.max_seq * HD;
+  float m = -__builtin_inff(), l = 0.0f, acc[HD / 64];
+#pragma unroll
+  for (int j = 0; j < HD / 64; ++j) acc[j] = 0.0f;
+  for (int base = 0; base < visible; base += 64) {
+    const int n = min(64, visible - base);
+    const bool valid = lane < n;
+    const uint16_t *kr = kb + (size_t)(base + (valid ? lane : 0)) * HD;
+    float dot = 0.0f;
+    for (int d = 0; d < HD; ++d) dot = dot + q[d] * aos_bf16_to_f32(kr[d]);
+    const float s = valid ? dot * p.scale : -__builtin_inff();
+    const float mn = fmaxf(m, wave_max(s));
+    const float alpha = expf(m - mn);
+    const float pv = valid ? expf(s - mn) : 0.0f;
+    l = l * alpha + wave_sum(pv);
+    ps[lane] = pv;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+#pragma unroll
+    for (int j = 0; j < HD / 64; ++j) acc[j] = acc[j] * alpha;
+    for (int jj = 0; jj < n; ++jj)
+#pragma unroll
+      for (int j = 0; j < HD / 64; ++j)
+        acc[j] = acc[j] + ps[jj] * aos_bf16_to_f32(vb[(size_t)(base + jj) * HD + lane + 64 * j]);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    m = mn;
+  }
+#pragma unroll
+  for (int j = 0; j < HD / 64; ++j)
+    p.out[((size_t)t * p.nh + h) * HD + lane + 64 * j] = aos_f32_to_bf16(acc[j] / l);
+}
+
+template <int HD>
+__global__ void __launch_bounds__(256, 2) aos_attn_prefill_kernel(aos_attn_params p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  constexpr int KS = HD / 16, DB = HD / 32, ROWB = HD * 2, TB = PA_BK * ROWB, NB = TB / 1024 / 4, CPR = HD / 8;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i = lane & 31, c = lane >> 5;
+  const int h = blockIdx.x, kvh = h / (p.nh / p.nkv);
+  const int q0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * PA_BQ; /* the longest ranges first */
+  if (*p.nonfinite) { /* uniform */
+    for (int j = 0; j < 32; ++j) {
+      const int t = q0 + 32 * wave + j;
+      if (t < p.T) attn_token_plain<HD>(p, h, t, lane, (float *)smem + 64 * wave);
+    }
+    return;
+  }
+  const int row = q0 + 32 * wave + i;
+  const int first = p.offset + q0 + 32 * wave; /* the wave's first position */
+  const int kend = p.offset + (q0 + PA_BQ < p.T ? q0 + PA_BQ : p.T);
+  const int ntiles = (kend + PA_BK - 1) / PA_BK;
+  const uint16_t *kb = p.kc + (size_t)kvh * p.max_seq * HD;
+  const uint16_t *vb = p.vc + (size_t)kvh * p.max_seq * HD;
+
+  /* LDS chunk slot of (row, chunk): keys slot = chunk ^ kx(row), values slot = chunk ^ vx(row) */
+  auto kx = [](int r) { return HD == 128 ? (r & 15) : ((r >> 1) & 7); };
+  auto vx = [](int r) {
+    return HD == 128 ? 2 * ((r & 3) | (((r >> 3) & 1) << 2)) : 2 * (((r >> 1) & 1) | (((r >> 3) & 1) << 1));
+  };
+  int kv_off[NB], vv_off[NB];
+#pragma unroll
+  for (int k = 0; k < NB; ++k) {
+    const int slot = (4 * k + wave) * 64 + lane, r = slot / CPR, sl = slot % CPR;
+    kv_off[k] = r * ROWB + ((sl ^ kx(r)) << 4);
+    vv_off[k] = r * ROWB + ((sl ^ vx(r)) << 4);
+  }
+  auto dma = [&](int kt) {
+    unsigned char *st = smem + (kt & 1) * 2 * TB;
+    pa_dma<NB>(kb, kend * ROWB, st, wave, kv_off, kt * TB);
+    pa_dma<NB>(vb, kend * ROWB, st + TB, wave, vv_off, kt * TB);
+  };
+  dma(0);
+
+  /* the token's query pieces: B operand, K elements 16 ks + 8 c .. +7 */
+  u32x4 qf[KS][3];
+  {
+    const float *q = p.q + ((size_t)(row < p.T ? row : p.T - 1) * p.nh + h) * HD + 8 * c;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const float4 a = *(const float4 *)(q + 16 * ks), b = *(const float4 *)(q + 16 * ks + 4);
+      const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        uint32_t hi, mid, lo;
+        split3(v[2 * e], v[2 * e + 1], hi, mid, lo);
+        qf[ks][0][e] = hi;
+        qf[ks][1][e] = mid;
+        qf[ks][2][e] = lo;
+      }
+    }
+  }
+  /* A operand row i of a 32-key block is key swap23(i) */
+  const int krow = (i & ~12) | ((i & 4) << 1) | ((i & 8) >> 1);
+  const int kbase = krow * ROWB + ((c ^ kx(krow)) << 4); /* chunk 2 ks + c: ^ (ks << 5) */
+  /* transposed value reads: 16-lane group (c, g) takes rows 8 c + 4 qq + w / 4 of a 16-key step,
+   * bytes 64 db + 32 g + 8 (w % 4) of the row */
+  const int w = lane & 15, g = (lane >> 4) & 1;
+  int vbase[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db) {
+    const int r = 8 * c + (w >> 2);
+    vbase[db] = TB + r * ROWB + (((4 * db + 2 * g + ((w & 3) >> 1)) ^ vx(r)) << 4) + 8 * (w & 1);
+  }
+
+  f32x16 o[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db) o[db] = f32x16{};
+  float m = -__builtin_inff(), l = 0.0f; /* l: this lane's half of the token's sum */
+  for (int kt = 0; kt < ntiles; ++kt) {
+    aos_mem_wait(); /* tile kt, issued a tile ago */
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); /* and every wave is past tile kt - 1 */
+    if (kt + 1 < ntiles) dma(kt + 1);
+    const int k0 = kt * PA_BK;
+    if (k0 > first + 31) continue; /* uniform: every key is later than the wave's tokens */
+    const unsigned char *st = smem + (kt & 1) * 2 * TB;
+    f32x16 s[2] = {f32x16{}, f32x16{}};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const u32x4 a0 = *(const u32x4 *)(st + (kbase ^ (ks << 5)));
+      const u32x4 a1 = *(const u32x4 *)(st + (kbase ^ (ks << 5)) + 32 * ROWB);
+#pragma unroll
+      for (int pc = 2; pc >= 0; --pc) {
+        s[0] = aos_mfma32(a0, qf[ks][pc], s[0]);
+        s[1] = aos_mfma32(a1, qf[ks][pc], s[1]);
+      }
+    }
+    const bool edge = k0 + PA_BK - 1 > first; /* uniform */
+    const int last = p.offset + row;          /* the token's own position */
+    float mx = m;
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        float x = s[b][v] * p.scale;
+        if (edge && k0 + 32 * b + 16 * (v >> 3) + 8 * c + (v & 7) > last) x = -__builtin_inff();
+        s[b][v] = x;
+        mx = fmaxf(mx, x);
+      }
+    mx = fmaxf(mx, aos_shfl_f(mx, lane ^ 32));
+    if (__ballot(mx > m)) {
+      const float alpha = m == mx ? 1.0f : exp_neg(m - mx);
+      l = l * alpha;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[db][v] = o[db][v] * alpha;
+      m = mx;
+    }
+#pragma unroll
+    for (int sp = 0; sp < 4; ++sp) {
+      u32x4 pf[3];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float pa = exp_neg(s[sp >> 1][8 * (sp & 1) + 2 * e] - m);
+        const float pb = exp_neg(s[sp >> 1][8 * (sp & 1) + 2 * e + 1] - m);
+        l = l + pa;
+        l = l + pb;
+        uint32_t hi, mid, lo;
+        split3(pa, pb, hi, mid, lo);
+        pf[0][e] = hi;
+        pf[1][e] = mid;
+        pf[2][e] = lo;
+      }
+      u32x4 a[DB];
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        const __attribute__((address_space(3))) unsigned char *vt =
+            (const __attribute__((address_space(3))) unsigned char *)(st + vbase[db] + 16 * sp * ROWB);
+        const s16x4 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)vt);
+        const s16x4 x1 =
+            __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(vt + 4 * ROWB));
+        const u32x2 y0 = __builtin_bit_cast(u32x2, x0), y1 = __builtin_bit_cast(u32x2, x1);
+        a[db] = u32x4{y0.x, y0.y, y1.x, y1.y};
+      }
+#pragma unroll
+      for (int pc = 2; pc >= 0; --pc)
+#pragma unroll
+        for (int db = 0; db < DB; ++db) o[db] = aos_mfma32(a[db], pf[pc], o[db]);
+    }
+  }
+  aos_mem_wait();
+  if (row >= p.T) return;
+  l = l + aos_shfl_f(l, lane ^ 32);
+  uint16_t *out = p.out + ((size_t)row * p.nh + h) * HD;
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      u32x2 r;
+      r.x = (uint32_t)aos_f32_to_bf16(o[db][4 * q] / l) | ((uint32_t)aos_f32_to_bf16(o[db][4 * q + 1] / l) << 16);
+      r.y = (uint32_t)aos_f32_to_bf16(o[db][4 * q + 2] / l) | ((uint32_t)aos_f32_to_bf16(o[db][4 * q + 3] / l) << 16);
+      *(u32x2 *)(out + 32 * db + 8 * q + 4 * c) = r;
+    }
+}
+
+template <int HD>
+int launch_attn_prefill(const aos_attn_params *p, const aos_launch_ctx *ctx) {
+  AOS_LAUNCH(ctx, aos_attn_prefill_kernel<HD>, dim3(p->nh, (p->T + PA_BQ - 1) / PA_BQ), dim3(256),
+             4 * PA_BK * HD * 2, *p);
+  return (int)hipGetLastError();
+}
+
 template <int DPL>
 int launch_attn(const aos_attn_params *p, const aos_launch_ctx *ctx) {
   AOS_LAUNCH(ctx, aos_attn_kernel<DPL>, dim3(p->splits, p->nh, p->T), dim3(64), 0, *p);
@@ -520,14 +810,26 @@ extern "C" int aos_launch_norm(const aos_norm_params *p, const aos_launch_ctx *c
 }
 
 extern "C" int aos_launch_rope(const aos_rope_params *p, const aos_launch_ctx *ctx) {
+  if (!p->nonfinite) return (int)hipErrorInvalidValue;
   const int items = p->nh * (p->hd / 2) + p->nkv * (p->hd / 2) + p->nkv * p->hd;
   AOS_LAUNCH(ctx, aos_rope_kernel, dim3((items + 255) / 256, p->T), dim3(256), 0, *p);
   return (int)hipGetLastError();
 }
 
+/* The prompt kernel's shapes: its head_dims, and a head's cache within a 32-bit byte offset (a tile past
+ * the end included). */
+extern "C" int aos_attn_prefill_fits(int hd, int max_seq) {
+  return (hd == 64 || hd == 128) && ((long long)max_seq + 2 * PA_BK) * hd * 2 < (1ll << 31);
+}
+
 extern "C" int aos_launch_attention(const aos_attn_params *p, const aos_launch_ctx *ctx) {
   if (p->hd % 8 || p->hd > AOS_ATTN_MAX_HD || p->splits < 1 || p->splits > ATTN_MAX_SPLITS || p->chunk % 64)
     return (int)hipErrorInvalidValue;
+  if (!p->nonfinite) return (int)hipErrorInvalidValue;
+  if (p->prefill) {
+    if (p->rope_fused || !aos_attn_prefill_fits(p->hd, p->max_seq)) return (int)hipErrorInvalidValue;
+    return p->hd == 64 ? launch_attn_prefill<64>(p, ctx) : launch_attn_prefill<128>(p, ctx);
+  }
   if (p->rope_fused && (p->T != 1 || !p->qb || !p->kb || !p->vb || !p->inv_freq)) return (int)hipErrorInvalidValue;
   if (p->hd <= 64) return launch_attn<1>(p, ctx);
   if (p->hd <= 128) return launch_attn<2>(p, ctx);
