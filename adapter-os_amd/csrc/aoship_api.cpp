@@ -640,6 +640,9 @@ enum {
   KS_PAMHR,
   KS_PXAML,
   KS_PXAM,
+  KS_GEMM_GUF,
+  KS_GEMM_DOWNF,
+  KS_GEMM_PROJF,
   KS_COUNT
 };
 static const char *kStatNames[KS_COUNT] = {
@@ -648,7 +651,7 @@ static const char *kStatNames[KS_COUNT] = {
     "lora_tile_shrink_x", "q4_gemm_gate_up", "lora_tile_shrink_h", "q4_gemm_down",   "q4_gemm_proj",
     "decode_mlp", "mlp1", "lora_tile_expand_gate_up", "lora_adapter_plan", "lora_adapter_shrink_x",
     "lora_adapter_reduce_x", "lora_adapter_shrink_h", "lora_adapter_reduce_h", "lora_adapter_expand_list",
-    "lora_adapter_expand_gate_up"};
+    "lora_adapter_expand_gate_up", "q4_gemm_gate_up_finish", "q4_gemm_down_finish", "q4_gemm_proj_finish"};
 
 struct aoship_layer {
   int layer_idx = 0;
@@ -1846,6 +1849,50 @@ static void plan_sk(aoship_layer *l, Carve &cv, aos_gemm_params &g, bool swiglu)
   g.timeout = l->wait_dev;
 }
 
+/* K pieces of each of a launch's `tasks` (token tile, weight block) tasks of G groups: as many as keep
+ * the launch in one round of the device's resident workgroups, at least AOS_SPLIT_MIN_GROUPS groups a
+ * piece, 1 below `least` pieces. A task runs its groups one after the other (1 to 1.5 us each however
+ * idle the chip is), so a launch of few tasks takes G times that: the 7B-shaped down GEMM of one token
+ * tile, 14 tasks of 296 groups, 284 us whole and 25 + 12 us in 18 pieces; gate/up, 148 tasks of 56
+ * groups, 83 us whole and 44 + 21 us in 3. least is 2, and 3 for a single matrix alone: stream-K
+ * serves two pieces as well (126 tasks on 256 slots) and moves fewer partial sums. */
+#define AOS_SPLIT_MIN_GROUPS 8
+static int gemm_pieces(long tasks, int G, bool swiglu, int least) {
+  const long slots = aos_gemm_sk_slots(swiglu ? 1 : 0);
+  if (tasks < 1) return 1;
+  const long s = std::min(slots / tasks, (long)(G / AOS_SPLIT_MIN_GROUPS));
+  return s < least ? 1 : (int)s;
+}
+
+/* Whether a down GEMM of these tasks leaves over 45% of its grid's last round idle and stream-K could
+ * share it: then its shrink takes a launch of its own rather than that round. The 7B-shaped MLP with
+ * the shrink in the launch and with stream-K: 700 tokens (84 tasks on 256 slots, in pieces) 554 and
+ * 439 us, 1100 tokens (126 tasks) 658 and 618 us, 1500 tokens (168 tasks) 731 and 768 us. */
+static bool down_mostly_idle(long tasks, int G) {
+  const long slots = aos_gemm_sk_slots(0);
+  if (slots < 1 || tasks * G / slots < AOS_SK_MIN_GROUPS) return false;
+  return tasks * 20 < (tasks + slots - 1) / slots * slots * 11;
+}
+
+static long gemm_tasks(int T, int RB, bool swiglu) {
+  const int wv = swiglu ? 4 : 8; /* the kernel shape's waves per workgroup */
+  return (long)ceil_div(T, AOS_GEMM_BM) * ceil_div(RB, wv);
+}
+
+/* The GEMMs gp[0, n) (planned, without shrink workgroups or stream-K) as one launch in S pieces; the
+ * pieces' partial sums from the workspace. */
+static void plan_multi(Carve &cv, const aos_gemm_params *gp, int n, int S, bool swiglu, aos_gemm_multi_params &q) {
+  memset(&q, 0, sizeof(q));
+  q.n = n;
+  q.S = S;
+  for (int i = 0; i < n; ++i) {
+    q.g[i] = gp[i];
+    if (S > 1)
+      q.g[i].sk_part = cv.b.take<float>((size_t)S * gemm_tasks(gp[i].T, gp[i].w0.RB, swiglu) *
+                                        aos_gemm_sk_slot_floats(swiglu ? 1 : 0));
+  }
+}
+
 /* The adapter-major shrink of sp (modules m0 .. of the plan's tables) over the users that plan A
  * lists: K slices for about 1024 workgroups, at least 8 groups a slice, at most 16 slices, and
  * the slices' partial sums within 256 MB. */
@@ -1901,6 +1948,7 @@ struct MlpPrefill {
   bool use_am_x = false, use_am_h = false; /* the x / h shrink's wide-union tiles run adapter-major */
   bool use_xam = false;                    /* ... and the gate/up expand of the widest */
   aos_gemm_params g1, g2;
+  aos_gemm_multi_params m1, m2; /* S > 1: the gate/up / down GEMM in K pieces */
   aos_xexp_params xe;
   bool fused_x = false, fused_h = false; /* the x / h shrink runs in the GEMM launch */
   bool use_xe = false;                   /* the gate/up expand launch runs (wide unions) */
@@ -1919,10 +1967,13 @@ static void plan_mlp_prefill(aoship_layer *l, int T, const uint16_t *x, const ao
   /* each shrink in its GEMM's launch when its workgroups fit in the idle slots of that grid's
    * last round, else a launch of its own (K split into slices) */
   M.fused_x = M.fused_h = false;
+  const int s1 = gemm_pieces(gemm_tasks(T, Wg.RB, true), Wg.G, true, 2);
+  const int s2 = gemm_pieces(gemm_tasks(T, Wd.RB, false), Wd.G, false, 3);
   if (M.P.lora && l->prefill_fused_shrink) {
     const int tc = M.P.tu_cap, rg = tall[0].rpad, ru = tall[1].rpad, rd = tall[2].rpad;
-    M.fused_x = aos_gemm_shrink_fits(T, Wg.RB, tc * (rg > ru ? rg : ru), 1) != 0;
-    M.fused_h = aos_gemm_shrink_fits(T, Wd.RB, tc * rd, 0) != 0;
+    M.fused_x = s1 == 1 && aos_gemm_shrink_fits(T, Wg.RB, tc * (rg > ru ? rg : ru), 1) != 0;
+    M.fused_h = s2 == 1 && !((l->prefill_sk & 2) && down_mostly_idle(gemm_tasks(T, Wd.RB, false), Wd.G)) &&
+                aos_gemm_shrink_fits(T, Wd.RB, tc * rd, 0) != 0;
   }
   plan_tshrink(l, cv, M.P, x, perm, T, H, 0, 2, M.sx, M.fused_x);
   plan_gemm(l, M.P, M.sx, Wg, &Wu, x, perm, nullptr, T, 0, 0, h, M.g1);
@@ -1930,8 +1981,8 @@ static void plan_mlp_prefill(aoship_layer *l, int T, const uint16_t *x, const ao
   plan_gemm(l, M.P, M.sh, Wd, nullptr, h, nullptr, perm, T, 2, 0, y, M.g2);
   if (M.fused_x) fuse_shrink(l, cv, M.P, M.sx, M.g1);
   if (M.fused_h) fuse_shrink(l, cv, M.P, M.sh, M.g2);
-  plan_sk(l, cv, M.g1, true);
-  plan_sk(l, cv, M.g2, false);
+  if (s1 == 1) plan_sk(l, cv, M.g1, true);
+  if (s2 == 1) plan_sk(l, cv, M.g2, false);
   /* the tiles whose union holds at least prefill_am_tu adapters: their shrinks adapter-major */
   const int n = (int)l->table.size();
   M.use_am_x = M.use_am_h = false;
@@ -2038,6 +2089,8 @@ static void plan_mlp_prefill(aoship_layer *l, int T, const uint16_t *x, const ao
     M.xe.xam_tu = xt;
     M.use_xam = true;
   }
+  plan_multi(cv, &M.g1, 1, s1, true, M.m1);
+  plan_multi(cv, &M.g2, 1, s2, false, M.m2);
   M.bytes = cv.b.off + 256;
   M.ctr = cv.coff + 64;
   M.flg = cv.foff + 64;
@@ -2073,6 +2126,16 @@ static int launch_amshrink(aoship_layer *l, const aos_amshrink_params &q, int sl
   return launch_err(aos_launch_amshrink(&r, &c1), "lora adapter-major shrink sum (prefill)");
 }
 
+/* Launch the GEMMs of q and, in pieces, the finish launch. */
+static int launch_multi(aoship_layer *l, const aos_gemm_multi_params &q, int swiglu, int slot, int finish_slot,
+                        const char *what) {
+  aos_launch_ctx c0 = launch_ctx(l, slot);
+  if (launch_err(aos_launch_gemm_multi(&q, swiglu, 0, &c0), what)) return -1;
+  if (q.S < 2) return 0;
+  aos_launch_ctx c1 = launch_ctx(l, finish_slot);
+  return launch_err(aos_launch_gemm_multi(&q, swiglu, 1, &c1), what);
+}
+
 static int chunk_prefill_t(int T) { return T < AOS_PREFILL_MAX_T ? T : AOS_PREFILL_MAX_T; }
 
 static void size_proj(aoship_layer *l, const int *mods, int nm, int max_tokens, size_t &bytes, size_t &ctr,
@@ -2099,9 +2162,12 @@ extern "C" int aoship_layer_reserve(aoship_layer_t *l, int max_tokens) {
     const size_t fw = mlp1_flag_words(l);
     if (fw > flg) flg = fw;
   }
-  if (mlp && max_tokens > AOS_DECODE_MAX_T) {
+  /* every number of token tiles up to the largest chunk's: fewer tiles are cut into more pieces */
+  for (int t0 = 0; mlp && t0 < chunk_prefill_t(max_tokens); t0 += AOS_GEMM_BM) {
+    const int T = std::min(t0 + AOS_GEMM_BM, chunk_prefill_t(max_tokens));
+    if (T <= AOS_DECODE_MAX_T) break;
     MlpPrefill M;
-    plan_mlp_prefill(l, chunk_prefill_t(max_tokens), nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, M);
+    plan_mlp_prefill(l, T, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, M);
     if (M.bytes > bytes) bytes = M.bytes;
     if (M.ctr > ctr) ctr = M.ctr;
     if (M.flg > flg) flg = M.flg;
@@ -2522,13 +2588,21 @@ extern "C" int aoship_mlp_forward(aoship_layer_t *l, const aoship_bf16_t *x, int
       }
       l->last_sk = (M.g1.sk_nwg ? 1 : 0) | (M.g2.sk_nwg ? 2 : 0);
       if (M.g1.s_cols || M.g1.sk_nwg) M.g1.gen = next_gen(&l->gen);
-      aos_launch_ctx c2 = launch_ctx(l, KS_GEMM_GU);
-      if (launch_err(aos_launch_gemm(&M.g1, 1, &c2), "q4 gemm gate/up")) return -1;
+      if (M.m1.S > 1) {
+        if (launch_multi(l, M.m1, 1, KS_GEMM_GU, KS_GEMM_GUF, "q4 gemm gate/up")) return -1;
+      } else {
+        aos_launch_ctx c2 = launch_ctx(l, KS_GEMM_GU);
+        if (launch_err(aos_launch_gemm(&M.g1, 1, &c2), "q4 gemm gate/up")) return -1;
+      }
       if (!M.fused_h && launch_tshrink(l, M.sh, KS_PSHRINK_H)) return -1;
       if (M.use_am_h && launch_amshrink(l, M.amh, KS_PAMH)) return -1;
       if (M.g2.s_cols || M.g2.sk_nwg) M.g2.gen = next_gen(&l->gen);
-      aos_launch_ctx c4 = launch_ctx(l, KS_GEMM_DOWN);
-      if (launch_err(aos_launch_gemm(&M.g2, 0, &c4), "q4 gemm down")) return -1;
+      if (M.m2.S > 1) {
+        if (launch_multi(l, M.m2, 0, KS_GEMM_DOWN, KS_GEMM_DOWNF, "q4 gemm down")) return -1;
+      } else {
+        aos_launch_ctx c4 = launch_ctx(l, KS_GEMM_DOWN);
+        if (launch_err(aos_launch_gemm(&M.g2, 0, &c4), "q4 gemm down")) return -1;
+      }
     }
     return 0;
   }
@@ -2596,11 +2670,15 @@ extern "C" int aoship_route_mlp_forward(aoship_router_t *r, const float *feature
 }
 
 /* Prefill chunk of projections sharing x: the group plan, one tile shrink over every module, one
- * GEMM per matrix. The same code sizes the workspace (a Carve over nullptr) and fills it. */
+ * launch over the matrices' GEMMs. The same code sizes the workspace (a Carve over nullptr) and fills
+ * it. The k and v GEMMs of grouped-query attention are a few tasks each, which take as long alone as
+ * q's: a 7B-shaped layer's q, k and v at 1531 tokens, 190 us as three launches. A single matrix
+ * whose grid leaves part of its last round idle runs as stream-K. */
 struct ProjPrefill {
   PrefillPlan P;
   aos_tshrink_params sp;
   aos_gemm_params gp[3];
+  aos_gemm_multi_params mu;
 };
 
 static void plan_proj_prefill(aoship_layer *l, Carve &cv, const int *mods, int nm, const uint16_t *xc, int Tc,
@@ -2611,8 +2689,13 @@ static void plan_proj_prefill(aoship_layer *l, Carve &cv, const int *mods, int n
   plan_prefill_common(l, cv, rc, Tc, tabs, nm, Q.P);
   const uint16_t *perm = Q.P.lora ? Q.P.gp.perm : nullptr;
   plan_tshrink(l, cv, Q.P, xc, perm, Tc, in, 0, nm, Q.sp);
+  long tasks = 0;
+  for (int i = 0; i < nm; ++i) tasks += gemm_tasks(Tc, l->mats[mods[i]].RB, false);
+  const int S = gemm_pieces(tasks, l->mats[mods[0]].G, false, nm > 1 ? 2 : 3);
   for (int i = 0; i < nm; ++i)
     plan_gemm(l, Q.P, Q.sp, l->mats[mods[i]], nullptr, xc, perm, perm, Tc, i, i, yc ? yc[i] : nullptr, Q.gp[i]);
+  if (S == 1 && nm == 1) plan_sk(l, cv, Q.gp[0], false);
+  plan_multi(cv, Q.gp, nm, S, false, Q.mu);
 }
 
 /* Decode chunk (T <= 32) of projections sharing x: the x shrink (and plan) and the GEMVs, whose
@@ -2656,7 +2739,7 @@ static void plan_proj_decode(aoship_layer *l, Carve &cv, const int *mods, int nm
 }
 
 /* Workspace of projections sharing x for calls of up to max_tokens tokens (decode chunks at every
- * power of two up to 32 tokens, and the largest prefill chunk). */
+ * power of two up to 32 tokens, and prefill chunks of every number of token tiles). */
 static void size_proj(aoship_layer *l, const int *mods, int nm, int max_tokens, size_t &bytes, size_t &ctr,
                       size_t &flg) {
   auto take = [&](const Carve &cv) {
@@ -2670,10 +2753,12 @@ static void size_proj(aoship_layer *l, const int *mods, int nm, int max_tokens, 
     plan_proj_decode(l, cv, mods, nm, nullptr, T, nullptr, nullptr, Q);
     take(cv);
   }
-  if (max_tokens > AOS_DECODE_MAX_T) {
+  for (int t0 = 0; t0 < chunk_prefill_t(max_tokens); t0 += AOS_GEMM_BM) {
+    const int T = std::min(t0 + AOS_GEMM_BM, chunk_prefill_t(max_tokens));
+    if (T <= AOS_DECODE_MAX_T) break;
     Carve cv(nullptr, nullptr, nullptr);
     ProjPrefill Q;
-    plan_proj_prefill(l, cv, mods, nm, nullptr, chunk_prefill_t(max_tokens), nullptr, nullptr, Q);
+    plan_proj_prefill(l, cv, mods, nm, nullptr, T, nullptr, nullptr, Q);
     take(cv);
   }
 }
@@ -2702,9 +2787,12 @@ static int proj_multi(aoship_layer *l, const int *mods, int nm, const uint16_t *
       plan_proj_prefill(l, cv, mods, nm, x + (size_t)t0 * in, Tc, rings + t0, yc, Q);
       if (launch_gplan(l, Q.P)) return -1;
       if (launch_tshrink(l, Q.sp, KS_PSHRINK_X)) return -1;
-      for (int i = 0; i < nm; ++i) {
+      if (nm == 1 && Q.mu.S == 1) {
+        if (Q.gp[0].sk_nwg) Q.gp[0].gen = next_gen(&l->gen);
         aos_launch_ctx cg = launch_ctx(l, KS_GEMM_PROJ);
-        if (launch_err(aos_launch_gemm(&Q.gp[i], 0, &cg), "q4 gemm")) return -1;
+        if (launch_err(aos_launch_gemm(&Q.gp[0], 0, &cg), "q4 gemm")) return -1;
+      } else if (launch_multi(l, Q.mu, 0, KS_GEMM_PROJ, KS_GEMM_PROJF, "q4 gemm")) {
+        return -1;
       }
     }
     return 0;

@@ -1829,7 +1829,8 @@ __device__ __forceinline__ void gemm_task(const aos_gemm_params &p, unsigned cha
 #pragma unroll
       for (int m = 0; m < NMAT; ++m)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+        for (int mt = 0; mt < MT; ++mt) {
+          if (!p.sk_lines && m0 + mt * 32 >= p.T) continue; /* rows the finish launch does not read */
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             const f32x16 &a = m ? acc1[mt] : acc0[mt];
@@ -1837,6 +1838,8 @@ __device__ __forceinline__ void gemm_task(const aos_gemm_params &p, unsigned cha
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, w4), rs,
                                                    base + (uint32_t)(((m * MT + mt) * 4 + q) * 64 * 16), 0, SC1);
           }
+        }
+      if (!p.sk_lines) return; /* the finish launch adds the pieces */
       aos_mem_wait();
       __syncthreads();
       if (tid == 0) aos_raise(p.sk_lines + (size_t)sk.v * 32, p.gen);
@@ -2027,6 +2030,153 @@ __global__ void __launch_bounds__(64 * WV, OCC) aos_gemm_sk_kernel(aos_gemm_para
     gemm_task<SW, D, DBT, APF, WV, OCC, LC, NS>(p, smem, (int)(t % (uint32_t)p.mb), (int)(t / (uint32_t)p.mb), (int)ga,
                                                 (int)gb, role, sk);
     it += gb - ga;
+  }
+}
+
+/* Up to three GEMMs in one launch, each task's K groups in q.S pieces (aos_gemm_multi_params).
+ * Workgroups of one GEMM that land on one XCD take consecutive (piece, weight block, token tile)
+ * triples, token tile fastest, so that a weight block's token tiles share an L2. */
+template <bool SW, int D, bool DBT, bool APF, int WV, int OCC, int LC, int NS>
+__global__ void __launch_bounds__(64 * WV, OCC) aos_gemm_multi_kernel(aos_gemm_multi_params q) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  static_assert(NS > 0, "pieces of K need the LDS-DMA token tiles");
+  int b = blockIdx.x, k = 0;
+  while (k < q.n - 1 && b >= q.wg_end[k]) ++k;
+  if (k > 0) b -= q.wg_end[k - 1];
+  const aos_gemm_params &p = q.g[k];
+  int mbi, nbk;
+  if (q.S == 1) {
+    gemm_tile_of(b, p.mb, p.nb, mbi, nbk);
+    gemm_task<SW, D, DBT, APF, WV, OCC, LC, NS>(p, smem, mbi, nbk, 0, p.w0.G, GEMM_WHOLE, SkCtx{0u, 0u, 0u});
+    return;
+  }
+  const int total = p.mb * p.nb * q.S, x = b & 7, rem = total & 7;
+  const int t = x * (total >> 3) + (x < rem ? x : rem) + (b >> 3);
+  mbi = t % p.mb;
+  nbk = t / p.mb % p.nb;
+  const int s = t / (p.mb * p.nb), G = p.w0.G;
+  gemm_task<SW, D, DBT, APF, WV, OCC, LC, NS>(p, smem, mbi, nbk, s * G / q.S, (s + 1) * G / q.S, GEMM_PART,
+                                              SkCtx{(uint32_t)((s * p.mb + mbi) * p.nb + nbk), 0u, 0u});
+}
+
+/* The finish launch of a split GEMM (q.S > 1): a wave per 32 x 32 block (row block rb, sub-tile mt
+ * of token tile mbi) adds the S pieces' sums in order, then the LoRA expand over the tile union (or
+ * the expand launch's sums) and runs the epilogue; a workgroup takes four consecutive row blocks.
+ * SA and B fragments come straight from memory: the expand is a few steps of 64 columns per block,
+ * each lane's loads of two steps in flight together and the next B pointers behind them. WV: the
+ * GEMM's waves per workgroup (its slot layout). */
+template <bool SW, int WV>
+__global__ void __launch_bounds__(256) aos_gemm_finish_kernel(aos_gemm_multi_params q) {
+  constexpr int MT = BM / 32, NMAT = SW ? 2 : 1, PW = NMAT * MT * 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = lane & 31, c = lane >> 5;
+  int b = blockIdx.x, kg = 0;
+  while (kg < q.n - 1 && b >= q.fin_end[kg]) ++kg;
+  if (kg > 0) b -= q.fin_end[kg - 1];
+  const aos_gemm_params &p = q.g[kg];
+  const int T = p.T, RB = p.w0.RB, mb = p.mb, nb = p.nb;
+  const int nst = (T + 31) >> 5;
+  const int st = b % nst, rb = b / nst * 4 + wave;
+  if (rb >= RB) return;
+  const int mbi = st >> 2, mt = st & 3, t0 = st * 32;
+  const int nbk = rb / WV, w = rb - nbk * WV;
+
+  f32x16 acc[NMAT];
+#pragma unroll
+  for (int m = 0; m < NMAT; ++m) acc[m] = f32x16{};
+  {
+    const size_t slot = (size_t)WV * PW * 64, step = (size_t)mb * nb * slot;
+    const f32x4 *src = (const f32x4 *)p.sk_part + ((size_t)mbi * nb + nbk) * slot + (w * PW + mt * 4) * 64 + lane;
+    constexpr int U = SW ? 2 : 4; /* pieces in flight */
+    for (int s0 = 0; s0 < q.S; s0 += U) {
+      f32x4 v[U][NMAT][4];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const f32x4 *sp = src + (size_t)(s0 + u < q.S ? s0 + u : q.S - 1) * step;
+#pragma unroll
+        for (int m = 0; m < NMAT; ++m)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[u][m][e] = sp[(m * MT * 4 + e) * 64];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (s0 + u < q.S) {
+#pragma unroll
+          for (int m = 0; m < NMAT; ++m)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[m][e] += v[u][m][e >> 2][e & 3];
+        }
+    }
+  }
+
+  const int TU = (p.tu && (p.rpad0 | (SW ? p.rpad1 : 0))) ? __builtin_amdgcn_readfirstlane(p.tu[mbi]) : 0;
+  const int rmax = SW && p.rpad1 > p.rpad0 ? p.rpad1 : p.rpad0;
+  if (SW && p.xd && TU * rmax >= p.xe_cols) { /* the expand launch's sums, in accumulator order */
+    const f32x4 *d = (const f32x4 *)p.xd + (((size_t)mbi * RB + rb) * MT + mt) * 256 + lane;
+    const size_t plane = (size_t)p.mtiles * RB * MT * 256;
+#pragma unroll
+    for (int m = 0; m < NMAT; ++m)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const f32x4 v = d[m * plane + e * 64];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) acc[m][4 * e + k] += v[k];
+      }
+  } else {
+    const int rowt = t0 + i < T ? t0 + i : T - 1; /* rows past the last token are never stored */
+    int off = 0;
+    for (int k = 0; k < p.sa_mod_before; ++k) off += TU * p.rpad_before[k];
+#pragma unroll
+    for (int m = 0; m < NMAT; ++m) {
+      const int rp = m ? p.rpad1 : p.rpad0;
+      const int n = TU * rp;
+      const uint16_t *sa = p.SA + (size_t)rowt * p.sa_stride + off;
+      const uint16_t *const *bpt = p.bp + ((size_t)(p.mod0 + m) * p.mtiles + mbi) * p.tu_cap;
+      /* two steps of 64 columns: pair h (columns k .. k + 15 of the lane, one union slot: rp is a
+       * multiple of 16) covers fragment words 2 h and 2 h + 1 */
+      auto col = [&](int k0, int h) { return k0 + (h >> 1) * 64 + 32 * c + (h & 1) * 16; };
+      auto ptrs = [&](int k0, const uint16_t *(&pb)[4]) {
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const int u = col(k0, h) / rp;
+          pb[h] = aos_gld_ptr(bpt + (u < TU ? u : TU - 1));
+        }
+      };
+      const uint16_t *pb[4];
+      if (n > 0) ptrs(0, pb);
+      for (int k0 = 0; k0 < n; k0 += 128) {
+        u32x4 a[8], f[8];
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const int k = col(k0, h), u = k / rp;
+          const bool in = k < n;
+          const uint16_t *bf = pb[h] + ((size_t)rb * (rp >> 3) + ((k - u * rp) >> 3)) * 256 + i * 8;
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            a[2 * h + e] = aos_gld16(in ? sa + k + 8 * e : p.zero);
+            f[2 * h + e] = aos_gld16(in && pb[h] ? bf + 256 * e : p.zero);
+          }
+        }
+        if (k0 + 128 < n) ptrs(k0 + 128, pb);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[m] = aos_mfma32(a[e], f[e], acc[m]);
+      }
+      off += n;
+    }
+  }
+
+  const int row = rb * 32 + i, out = p.w0.out;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int ps = t0 + aos_acc_m(v, lane);
+    if (ps >= T) continue;
+    const int tok = p.out_perm ? (int)p.out_perm[ps] : ps;
+    float r = acc[0][v];
+    if (SW) {
+      const float sg = 1.0f / (1.0f + expf(-acc[0][v]));
+      r = (acc[0][v] * sg) * acc[NMAT - 1][v];
+    }
+    p.y[(size_t)tok * out + row] = aos_f32_to_bf16(r);
   }
 }
 
@@ -2315,6 +2465,54 @@ extern "C" int aos_launch_gemm(const aos_gemm_params *p, int swiglu, const aos_l
     return (int)hipErrorInvalidValue;
   if (swiglu) return launch_gemm_cfg<true, 2, false, false, 4, 2, 2, AOS_GEMM_NS_SW>(p, ctx);
   return launch_gemm_cfg<false, 4, true, true, 8, 2, 4, AOS_GEMM_NS_ONE>(p, ctx);
+}
+
+/* Grids of a multi-GEMM launch and its finish launch for the kernel shape of WV waves. */
+template <int WV>
+static int multi_grids(const aos_gemm_multi_params *p, int swiglu, aos_gemm_multi_params &q) {
+  if (p->n < 1 || p->n > 3 || p->S < 1 || (swiglu && p->n != 1)) return (int)hipErrorInvalidValue;
+  q = *p;
+  int wg = 0, fin = 0;
+  for (int k = 0; k < 3; ++k) {
+    aos_gemm_params &g = q.g[k];
+    if (k < q.n) {
+      if (g.T < 1 || g.T > AOS_PREFILL_MAX_T || g.mtiles != (g.T + BM - 1) / BM || g.sa_mod_before < 0 ||
+          g.sa_mod_before > 2 || g.rpad0 % 16 || g.rpad1 % 16 || (swiglu && (!g.w1.qt || g.w1.RB != g.w0.RB)) ||
+          g.s_cols || g.sk_nwg || g.sk_lines || q.S > g.w0.G || (q.S > 1 && !g.sk_part))
+        return (int)hipErrorInvalidValue;
+      g.mb = g.mtiles;
+      g.nb = (g.w0.RB + WV - 1) / WV;
+      g.nbs = 0;
+      /* the pieces' slots are addressed with 32-bit byte offsets */
+      if ((uint64_t)g.mb * g.nb * q.S * aos_gemm_sk_slot_floats(swiglu) * 4 >= (1ull << 31) && q.S > 1)
+        return (int)hipErrorInvalidValue;
+      wg += g.mb * g.nb * q.S;
+      fin += (g.T + 31) / 32 * ((g.w0.RB + 3) / 4);
+    }
+    q.wg_end[k] = wg;
+    q.fin_end[k] = fin;
+  }
+  return 0;
+}
+
+template <bool SW, int D, bool DBT, bool APF, int WV, int OCC, int LC, int NS>
+static int launch_multi_cfg(const aos_gemm_multi_params *p, int finish, const aos_launch_ctx *ctx) {
+  aos_gemm_multi_params q;
+  const int e = multi_grids<WV>(p, SW, q);
+  if (e) return e;
+  if (finish) {
+    AOS_LAUNCH(ctx, (aos_gemm_finish_kernel<SW, WV>), dim3(q.fin_end[2]), dim3(256), 0, q);
+    return (int)hipGetLastError();
+  }
+  const size_t lds = (size_t)gemm_ntile<NS, LC>() * BM * 128 + gemm_aux();
+  AOS_LAUNCH(ctx, (aos_gemm_multi_kernel<SW, D, DBT, APF, WV, OCC, LC, NS>), dim3(q.wg_end[2]), dim3(64 * WV), lds, q);
+  return (int)hipGetLastError();
+}
+
+extern "C" int aos_launch_gemm_multi(const aos_gemm_multi_params *p, int swiglu, int finish,
+                                     const aos_launch_ctx *ctx) {
+  if (swiglu) return launch_multi_cfg<true, 2, false, false, 4, 2, 2, AOS_GEMM_NS_SW>(p, finish, ctx);
+  return launch_multi_cfg<false, 4, true, true, 8, 2, 4, AOS_GEMM_NS_ONE>(p, finish, ctx);
 }
 
 AOS_DEFINE_SPIN_SETTER(aos_spin_setter_gemm)

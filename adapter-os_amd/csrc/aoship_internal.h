@@ -539,6 +539,17 @@ typedef struct {
   int xe_cols;
 } aos_gemm_params;
 
+/* One launch over up to three GEMMs of one kernel shape (SwiGLU or single-matrix; n > 1: the
+ * projections that share x), each task's K groups cut into S pieces. S = 1: every task runs whole,
+ * expand and epilogue included. S > 1: piece s of a task stores its partial sums in slot
+ * (s * mb + mbi) * nb + nbk of its GEMM's sk_part (a slot: aos_gemm_sk_slot_floats floats), and the
+ * finish launch adds the pieces in order, then the expand, and writes y. */
+typedef struct {
+  aos_gemm_params g[3]; /* s_cols = sk_nwg = 0, sk_lines NULL; mb, nb, nbs set by the launcher */
+  int n, S;
+  int wg_end[3], fin_end[3]; /* workgroups through GEMM i of the two launches (set by the launcher) */
+} aos_gemm_multi_params;
+
 /* The expand launch of a SwiGLU prefill GEMM: for each tile with tu * rmax >= xe_cols and each
  * module m (0 gate, 1 up), xd[m] = SA . B^T over the tile's union columns of that module (g[m]
  * describes module m as the only module of a single-matrix expand), in the layout the GEMM reads. */
@@ -679,6 +690,8 @@ int aos_launch_mlp1(const aos_mlp1_params *p, const aos_launch_ctx *ctx);
 /* The prefill GEMM's stream-K shape on the current device (swiglu: the gate/up kernel, else the
  * single-matrix one): workgroups resident at once, and floats of partial sums per workgroup. */
 int aos_gemm_sk_slots(int swiglu);
+/* finish 0: the GEMMs' tasks (whole, or in S pieces); 1: the finish launch of S > 1 pieces. */
+int aos_launch_gemm_multi(const aos_gemm_multi_params *p, int swiglu, int finish, const aos_launch_ctx *ctx);
 int aos_gemm_sk_slot_floats(int swiglu);
 int aos_spin_setter_mlp1(uint32_t polls);
 /* The wait bound of each translation unit's kernels on the current device (polls; hipError_t). */
