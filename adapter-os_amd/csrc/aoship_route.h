@@ -232,10 +232,11 @@ __device__ __forceinline__ void decision_empty(aoship_decision_t *decisions, int
 
 /* X: the extras (scope, adaptive keys, decision policy, ring mapping, decision hashes) are
  * compiled in; the X = false instance is the plain router, launched when none is set. first: the
- * lane's RouteMeta for adapter `lane`, loaded ahead (NULL: loaded here). */
-template <bool LDS, bool X>
+ * lane's RouteMeta for adapter `lane`, loaded ahead (NULL: loaded here). NR waves of the workgroup
+ * may route at once, each with its own rw < NR. */
+template <bool LDS, bool X, int NR = 1>
 __device__ __forceinline__ void route_one(const aos_route_params &p, const float *priors, int t, int lane,
-                                          const RouteMeta *first = nullptr) {
+                                          const RouteMeta *first = nullptr, int rw = 0) {
   const int n = p.n;
   const uint8_t *scope = X ? p.scope : nullptr;
   const uint64_t *tie_key = X ? p.tie_key : nullptr;
@@ -275,8 +276,9 @@ __device__ __forceinline__ void route_one(const aos_route_params &p, const float
     if (n <= AOS_WAVE) {
       /* n <= 64: rank selection. Keys are unique (they end in the index), so lane i's rank is
        * the number of smaller keys; the 8 smallest are scattered to lanes 0..7 through LDS. */
-      __shared__ uint64_t keys[2 * AOS_WAVE];
-      __shared__ uint64_t top[2 * 8];
+      __shared__ uint64_t keys_s[NR][2 * AOS_WAVE];
+      __shared__ uint64_t top_s[NR][2 * 8];
+      uint64_t *keys = keys_s[NR > 1 ? rw : 0], *top = top_s[NR > 1 ? rw : 0];
       keys[2 * lane] = ka;
       keys[2 * lane + 1] = kb;
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");

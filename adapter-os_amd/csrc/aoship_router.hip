@@ -74,6 +74,121 @@ __global__ void __launch_bounds__(1024) aos_route_features_kernel(aos_route_para
   route_features_block<X>(p, blockIdx.x, lds);
 }
 
+/* The xor butterflies of W values (step o, then o / 2, ... 1) folded into each other: afterwards the
+ * 64 / NV lanes whose upper bits spell v hold value v's sum in acc[0]. */
+template <int W, int O, int NV>
+__device__ __forceinline__ void fold_sums(float (&acc)[NV], int lane) {
+  if constexpr (O >= 1) {
+    if constexpr (W > 1) {
+#pragma unroll
+      for (int v = 0; v < W / 2; ++v) {
+        const float lo = acc[v], hi = acc[v + W / 2];
+        acc[v] = ((lane & O) ? hi : lo) + aos_shfl_f((lane & O) ? lo : hi, lane ^ O);
+      }
+    } else {
+      acc[0] = acc[0] + aos_shfl_f(acc[0], lane ^ O);
+    }
+    fold_sums<(W > 1 ? W / 2 : 1), O / 2>(acc, lane);
+  }
+}
+
+/* Routing from router features, TT tokens per workgroup (the plain router): with one token per
+ * workgroup every token reads all n weight rows from L2 (2039 tokens, 64 adapters of 5120 features:
+ * 2.6 GB, 180 us). Here wave w holds adapters a0 + w + 16 j (j < AW) of a pass of 16 AW adapters
+ * against all TT tokens: a weight chunk, loaded a chunk ahead, meets TT tokens' features from LDS and a
+ * feature chunk AW adapters, which leaves the float32 multiply-adds as the bound (17 of its 33 us). Each dot product keeps dot_finish's order: lane l sums elements 256 k + 4 l + e in
+ * ascending k and e, then the xor butterfly. The butterflies of a wave's dot products fold into each
+ * other: at step o lanes with bit o clear keep one value and lanes with it set another, so that each
+ * shuffle adds for two; addition commutes, so the sums are the same bits.
+ * LDS: two stages of [TT][KC 256] features (KC chunks of 256: one 16-byte word per thread), then the
+ * priors [TT][n]. Waves 0 .. TT - 1 route one token each. */
+template <int TT, int AW>
+__global__ void __launch_bounds__(1024) aos_route_tokens_kernel(aos_route_params p) {
+  extern __shared__ float lds[];
+  constexpr int KC = 16 / TT; /* 1024 threads x 4 floats / (TT x 256) */
+  constexpr int NV = TT * (AW == 3 ? 4 : AW);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int t0 = blockIdx.x * TT, d = p.d, n = p.n;
+  float *priors = lds + 2 * TT * KC * 256;
+  RouteMeta meta = {1, 1, 0ull};
+  if (wave < TT) meta = route_meta<false>(p, lane);
+  /* this thread's word of a stage: token st, features 4 sw .. of the stage */
+  const int st = tid / (KC * 64), sw = tid % (KC * 64);
+  const float *frow = p.features + (size_t)(t0 + st < p.T ? t0 + st : p.T - 1) * d;
+  const int nk = d >> 8, tail = d & 255, ns = (nk + (tail ? 1 : 0) + KC - 1) / KC;
+  auto fetch = [&](int s) {
+    const int e = s * KC * 256 + 4 * sw;
+    return e < d ? *(const float4 *)(frow + e) : float4{0.0f, 0.0f, 0.0f, 0.0f};
+  };
+  for (int a0 = 0; a0 < n; a0 += 16 * AW) {
+    const float *wr[AW];
+#pragma unroll
+    for (int j = 0; j < AW; ++j) {
+      const int a = a0 + wave + 16 * j;
+      wr[j] = p.router_w + (size_t)(a < n ? a : n - 1) * d;
+    }
+    const bool live = a0 + wave < n; /* uniform per wave */
+    float acc[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) acc[v] = 0.0f;
+    /* chunk k of the wave's rows (lanes past a row's end read its last word and are not summed) */
+    auto weights = [&](int k, float4 (&w)[AW]) {
+      int e = k * 256 + 4 * lane;
+      e = e < d ? e : d - 4;
+#pragma unroll
+      for (int j = 0; j < AW; ++j) w[j] = *(const float4 *)(wr[j] + e);
+    };
+    auto use = [&](const float *f, const float4 (&w)[AW]) {
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        const float4 fv = ((const float4 *)(f + t * KC * 256))[lane];
+#pragma unroll
+        for (int j = 0; j < AW; ++j) {
+          float x = acc[t * (NV / TT) + j];
+          x = fmaf(w[j].x, fv.x, x);
+          x = fmaf(w[j].y, fv.y, x);
+          x = fmaf(w[j].z, fv.z, x);
+          x = fmaf(w[j].w, fv.w, x);
+          acc[t * (NV / TT) + j] = x;
+        }
+      }
+    };
+    float4 wv[2][AW];
+    if (live) weights(0, wv[0]);
+    float4 fv = fetch(0);
+    for (int s = 0; s < ns; ++s) {
+      float *buf = lds + (s & 1) * TT * KC * 256;
+      ((float4 *)(buf + st * KC * 256))[sw] = fv;
+      __syncthreads(); /* stage s is in; stage s - 2 was read before the previous barrier */
+      if (s + 1 < ns) fv = fetch(s + 1);
+      if (!live) continue;
+#pragma unroll
+      for (int c = 0; c < KC; ++c) {
+        const int k = s * KC + c;
+        /* chunk k sits in wv[k & 1]: KC is even, so the parity is c's */
+        if (k < nk) {
+          weights(k + 1, wv[(c + 1) & 1]);
+          use(buf + c * 256, wv[c & 1]);
+        } else if (k == nk && 4 * lane < tail) {
+          use(buf + c * 256, wv[c & 1]);
+        }
+      }
+    }
+    __syncthreads(); /* the last stage is read: the next pass may refill it */
+    if (live) {
+      fold_sums<NV, 32>(acc, lane);
+      constexpr int LV = 64 / NV; /* lanes per value */
+      const int v = lane / LV, t = v / (NV / TT), j = v % (NV / TT), a = a0 + wave + 16 * j;
+      if (lane % LV == 0 && j < AW && a < n) {
+        priors[t * n + a] = acc[0];
+        if (p.priors_out && t0 + t < p.T) p.priors_out[(size_t)(t0 + t) * n + a] = acc[0];
+      }
+    }
+  }
+  __syncthreads();
+  if (wave < TT && t0 + wave < p.T) route_one<true, false, TT>(p, priors + wave * n, t0 + wave, lane, &meta, wave);
+}
+
 /* The router's workgroups (one per token, the plain router), then the x shrink and the gate/up
  * GEMV of the layer those rings feed: the shrink does not depend on the rings, so it and the
  * weight stream run while the tokens are routed; only the adapter plan, and through it the
@@ -224,10 +339,39 @@ extern "C" int aos_launch_route_gate_up(const aos_route_gu_params *q, const aos_
   return launch_rgu<16>(q, ctx);
 }
 
+template <int TT>
+static int launch_route_tokens(const aos_route_params *p, const aos_launch_ctx *ctx) {
+  const dim3 grid((p->T + TT - 1) / TT), block(1024);
+  const size_t lds = (size_t)(2 * 4096 + TT * p->n) * sizeof(float);
+  if (p->n <= 16) AOS_LAUNCH(ctx, (aos_route_tokens_kernel<TT, 1>), grid, block, lds, *p);
+  else if (p->n <= 32) AOS_LAUNCH(ctx, (aos_route_tokens_kernel<TT, 2>), grid, block, lds, *p);
+  else if (p->n <= 48) AOS_LAUNCH(ctx, (aos_route_tokens_kernel<TT, 3>), grid, block, lds, *p);
+  else AOS_LAUNCH(ctx, (aos_route_tokens_kernel<TT, 4>), grid, block, lds, *p);
+  return (int)hipGetLastError();
+}
+
+/* Tokens per workgroup of a plain router call from features: the fewest that give each CU at most
+ * one workgroup, up to 8; one token each (aos_route_features_kernel) while the tokens do not outnumber
+ * the CUs. A second round costs as much as the first, more than wider workgroups do (64 adapters of
+ * 5120 features: one round of 2 / 4 / 8 tokens 21 / 23 / 31 us, two rounds of 4 tokens 40 us). Before,
+ * with one token a workgroup: 384 tokens 46 us, 768 68 us, 2039 178 us; now 21, 23 and 33 us. The
+ * priors of the tokens must fit beside 32 KB of stages. */
+#define AOS_ROUTE_CUS 256
+static int route_tokens(const aos_route_params *p) {
+  int tt = 1;
+  while (tt < 8 && p->T > tt * AOS_ROUTE_CUS) tt <<= 1;
+  while (tt > 1 && (size_t)tt * p->n * sizeof(float) > 16 * 1024) tt >>= 1;
+  return tt;
+}
+
 extern "C" int aos_launch_route(const aos_route_params *p, const aos_launch_ctx *ctx) {
   const bool x =
       p->scope || p->tie_key || p->post_allowed || p->active_ids || p->strengths || p->hashes || p->decisions;
   if (p->features) {
+    const int tt = x ? 1 : route_tokens(p);
+    if (tt == 8) return launch_route_tokens<8>(p, ctx);
+    if (tt == 4) return launch_route_tokens<4>(p, ctx);
+    if (tt == 2) return launch_route_tokens<2>(p, ctx);
     const int waves = p->n < 16 ? p->n : 16;
     const size_t lds = (size_t)(p->d + p->n) * sizeof(float);
     if (x) AOS_LAUNCH(ctx, aos_route_features_kernel<true>, dim3(p->T), dim3(64 * waves), lds, *p);
