@@ -1291,12 +1291,48 @@ static void gemv_geometry_rows(int RB, int G, int T, bool swiglu, int W, aos_gem
   g.ks = ks;
 }
 
+/* Decode GEMVs whose waves read x themselves (3-32 tokens): one row block per workgroup, its K groups over
+ * the workgroup's four waves and ks workgroups, about AOS_GEMV_DX_WAVES waves in all. LDS holds the wave
+ * reduction only, so the whole grid is resident at once and its wait for S is paid once; with x staged, 27
+ * tokens of the 7B gate/up launch were 1280 workgroups of 48 KB, two and a half rounds, and 34 MB of split
+ * partials. 7B MLP at 8 / 16 / 27 / 32 tokens: 56 / 91 / 127 / 126 us staged, 55 / 65 / 82 / 92 us here; the
+ * 0.5B-shaped MLP 46 -> 36 us at 8. 1024 and 1536 waves measure the same, 512 and 3072 lose up to a fifth;
+ * the projections, whose splits' reduction is a larger part, are best at 512 (7B q/k/v and o at 8 tokens 30 us,
+ * at 2048 waves 33 us, staged 35 us).
+ * A gate/up launch of at most 8 tokens over a wide adapter table stays staged: a row block then has twice the
+ * waves to share its expand steps (64 adapters of rank 64, hidden 5120: 350 us staged, 415 us here at 8
+ * tokens; 671 and 597 us at 16, where staging x costs more). */
+#define AOS_GEMV_DX_MIN_T 3
+#define AOS_GEMV_DX_MIN_G 8
+#define AOS_GEMV_DX_WAVES 1024
+#define AOS_GEMV_DX_WAVES_PROJ 512
+#define AOS_GEMV_DX_GU_COLS 1024 /* a module's columns over the whole table, up to which 3-8 tokens read x directly */
+static bool gemv_direct(int G, int T, int wr_force, int ks_force) {
+  return T >= AOS_GEMV_DX_MIN_T && G >= AOS_GEMV_DX_MIN_G && wr_force <= 0 && ks_force <= 0;
+}
+
+static void gemv_geometry_direct(int RB, int G, int T, bool swiglu, bool lora, aos_gemv_params &g, int waves) {
+  int ks = ceil_div(waves, 4 * RB);
+  if (ks > G / 8) ks = G / 8;
+  g.dx = 1;
+  g.wr = 1;
+  g.waves = 4;
+  g.ks = ks;
+  g.nrbg = g.w0.RB;
+  g.has_expand = lora ? 1 : 0;
+  g.lds_bytes = 4 * (swiglu ? 2 : 1) * nv_for(T) * 64 * 4;
+}
+
 /* Every wave of a K split must get at least one group (G / ks >= W): the 8-wave single-matrix
  * kernel falls back to 4 waves when the LDS budget forces more splits (many tokens, long K).
  * From 3 tokens on, the row-split geometry above. */
 static void gemv_geometry(int RB, int G, int T, bool swiglu, bool lora, aos_gemv_params &g,
                           int waves_target = AOS_GEMV_WAVES, bool four_waves = false, int wr_force = 0,
-                          int ks_force = 0) {
+                          int ks_force = 0, int direct_waves = 0) {
+  if (direct_waves > 0) {
+    gemv_geometry_direct(RB, G, T, swiglu, lora, g, direct_waves);
+    return;
+  }
   int W = (swiglu || four_waves) ? 4 : (G >= AOS_GEMV_W8_MIN_G ? 8 : 4);
   int ks = 1;
   g.wr = 1;
@@ -1341,7 +1377,9 @@ static void gemv_geometry(int RB, int G, int T, bool swiglu, bool lora, aos_gemv
  * keep the launch within one round of resident workgroups (the 32-stream projections: 336 shrink
  * workgroups at 32 KB, 192 at 64 KB). */
 #define AOS_XSHRINK_LDS_MAX_T32 (64 * 1024)
-static size_t x_shrink_lds_max(int T) { return T > 16 ? AOS_XSHRINK_LDS_MAX_T32 : AOS_GEMV_LDS_MAX; }
+static size_t x_shrink_lds_max(int T, bool direct) {
+  return T > 16 && !direct ? AOS_XSHRINK_LDS_MAX_T32 : AOS_GEMV_LDS_MAX;
+}
 
 static void shrink_geometry(int rb_total, int G, int T, aos_shrink_params &sp, int waves = 4,
                             size_t lds_max = AOS_GEMV_LDS_MAX) {
@@ -1358,7 +1396,8 @@ static void shrink_geometry(int rb_total, int G, int T, aos_shrink_params &sp, i
   sp.lds_bytes = (int)(lds_x > lds_r ? lds_x : lds_r);
 }
 
-/* Diagnostic (no counterpart in the reference): the decode geometry the forwards use, for a
+/* Diagnostic (no counterpart in the reference): the decode geometry of the launches that stage x in LDS
+ * (1-2 tokens, pinned shapes, few K groups, wide unions; the others: gemv_geometry_direct), for a
  * CPU-side check that every wave of every launch gets at least one K group. kind 0: the gate/up
  * GEMV (out = intermediate, in = hidden); 1: the down GEMV (out = hidden, in = intermediate);
  * 2: a projection GEMV (out = the row count of the matrices sharing x); 3: a shrink over `out`
@@ -1397,7 +1436,7 @@ extern "C" int aoship_internal_decode_geometry_pinned(int kind, int out, int in,
     aos_shrink_params sp;
     memset(&sp, 0, sizeof(sp));
     W = kind == 4 ? 8 : (G >= AOS_GEMV_W8_MIN_G ? 8 : 4);
-    shrink_geometry(RB, G, T, sp, W, kind == 3 ? x_shrink_lds_max(T) : AOS_GEMV_LDS_MAX);
+    shrink_geometry(RB, G, T, sp, W, kind == 3 ? x_shrink_lds_max(T, false) : AOS_GEMV_LDS_MAX);
     k = sp.ks;
   } else {
     return set_err("aoship_internal_decode_geometry: unknown kind");
@@ -1510,7 +1549,7 @@ static size_t fused_flag_words(const aos_gemv_params *gp, int n) {
 
 static void plan_x_shrink(aoship_layer *l, Carve &cv, const uint16_t *x, int T, int in,
                           const aos_lora_tab *tabs, int nm, aos_plan *plan,
-                          const aoship_ring_t *rings, XShrink &xs) {
+                          const aoship_ring_t *rings, bool direct, XShrink &xs) {
   const int n = (int)l->table.size();
   int umax = n < 8 * T ? n : 8 * T;
   if (umax < 1) umax = 1;
@@ -1535,7 +1574,7 @@ static void plan_x_shrink(aoship_layer *l, Carve &cv, const uint16_t *x, int T, 
     rb_total += sp.n_rb[i];
   }
   /* sized for the waves of the GEMV it may be fused with (valid for the 4-wave launch too) */
-  shrink_geometry(rb_total, in / 64, T, sp, in / 64 >= AOS_GEMV_W8_MIN_G ? 8 : 4, x_shrink_lds_max(T));
+  shrink_geometry(rb_total, in / 64, T, sp, in / 64 >= AOS_GEMV_W8_MIN_G ? 8 : 4, x_shrink_lds_max(T, direct));
   sp.part = cv.b.take<float>((size_t)rb_total * sp.ks * nv_for(T) * 64);
   sp.counters = cv.counters((size_t)rb_total + 1);
   xs.separate_plan = !all;
@@ -1593,7 +1632,11 @@ static void plan_mlp(aoship_layer *l, int T, const uint16_t *x, const aoship_rin
   Carve cv(ws, ctr, flg);
   aos_plan *plan = cv.b.take<aos_plan>(1);
   uint16_t *h = cv.b.take<uint16_t>((size_t)T * I);
-  plan_x_shrink(l, cv, x, T, H, tabs_gu, 2, plan, rings, P.sx);
+  const int cols_gu = n * (tabs_gu[0].rpad > tabs_gu[1].rpad ? tabs_gu[0].rpad : tabs_gu[1].rpad);
+  const bool direct_gu =
+      gemv_direct(Wg.G, T, l->geo_wr[0], l->geo_ks[0]) && (T > 8 || cols_gu <= AOS_GEMV_DX_GU_COLS);
+  const bool direct_dn = gemv_direct(Wd.G, T, l->geo_wr[1], l->geo_ks[1]);
+  plan_x_shrink(l, cv, x, T, H, tabs_gu, 2, plan, rings, direct_gu, P.sx);
 
   aos_gemv_params &g1 = P.gv1;
   memset(&g1, 0, sizeof(g1));
@@ -1602,7 +1645,7 @@ static void plan_mlp(aoship_layer *l, int T, const uint16_t *x, const aoship_rin
   g1.x = x;
   g1.T = T;
   gemv_geometry(Wg.RB, Wg.G, T, true, tabs_gu[0].rpad > 0 || tabs_gu[1].rpad > 0, g1, AOS_GEMV_WAVES, false,
-                l->geo_wr[0], l->geo_ks[0]);
+                l->geo_wr[0], l->geo_ks[0], direct_gu ? AOS_GEMV_DX_WAVES : 0);
   g1.tab0 = tabs_gu[0];
   g1.tab1 = tabs_gu[1];
   g1.S0 = P.sx.sp.S[0];
@@ -1645,7 +1688,7 @@ static void plan_mlp(aoship_layer *l, int T, const uint16_t *x, const aoship_rin
    * 7B shape) keep its tail short; at 1-2 tokens it runs in the gate/up launch's grid, in
    * 4-wave workgroups like the rest of that grid */
   gemv_geometry(Wd.RB, Wd.G, T, false, td.rpad > 0, g2, T <= 2 ? AOS_GEMV_WAVES_DOWN12 : 2 * AOS_GEMV_WAVES, T <= 2,
-                l->geo_wr[1], l->geo_ks[1]);
+                l->geo_wr[1], l->geo_ks[1], direct_dn ? AOS_GEMV_DX_WAVES : 0);
   g2.tab0 = td;
   g2.S0 = s2.S[0];
   g2.s_stride0 = s2.s_stride[0];
@@ -2712,7 +2755,8 @@ static void plan_proj_decode(aoship_layer *l, Carve &cv, const int *mods, int nm
   aos_lora_tab tabs[3];
   for (int i = 0; i < nm; ++i) tabs[i] = lora_tab(l, mods[i], in, l->mats[mods[i]].out);
   aos_plan *plan = cv.b.take<aos_plan>(1);
-  plan_x_shrink(l, cv, xc, Tc, in, tabs, nm, plan, rc, Q.xs);
+  const bool direct = gemv_direct(in / 64, Tc, l->geo_wr[2], l->geo_ks[2]);
+  plan_x_shrink(l, cv, xc, Tc, in, tabs, nm, plan, rc, direct, Q.xs);
   memset(&Q.g3, 0, sizeof(Q.g3));
   aos_gemv_params *gp = Q.g3.p;
   int rb_all = 0;
@@ -2723,7 +2767,7 @@ static void plan_proj_decode(aoship_layer *l, Carve &cv, const int *mods, int nm
     gp[i].x = xc;
     gp[i].T = Tc;
     gemv_geometry(rb_all, W.G, Tc, false, tabs[i].rpad > 0, gp[i], Tc <= 2 ? AOS_GEMV_WAVES_PROJ12 : AOS_GEMV_WAVES,
-                  false, l->geo_wr[2], l->geo_ks[2]);
+                  false, l->geo_wr[2], l->geo_ks[2], direct ? AOS_GEMV_DX_WAVES_PROJ : 0);
     gp[i].tab0 = tabs[i];
     gp[i].S0 = Q.xs.sp.S[i];
     gp[i].s_stride0 = Q.xs.sp.s_stride[i];

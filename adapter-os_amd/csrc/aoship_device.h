@@ -77,11 +77,12 @@ __device__ __forceinline__ float aos_f16_to_f32(uint32_t h16) {
 /* Four packed bfloat16 pairs (128 + q) from one nibble-shuffled weight word: register p holds
  * (q[2p], q[2p+1]) of the original MLX word as bf16 values 128 + q (exact). One shift and one
  * v_and_or_b32 per register; the mask lives in an SGPR and the exponent pattern in a VGPR
- * (gfx950's VOP3 encoding takes no literal operands). */
+ * (gfx950's VOP3 encoding takes no literal operands). Written as plain operations: the compiler places
+ * the wait states that an MFMA needs after a VALU write of its operands, and before a VALU write of the
+ * result registers of an MFMA in flight, only for instructions it knows, not for an asm statement's
+ * (as one, the 32-token kernels that read x themselves returned NaN). */
 __device__ __forceinline__ uint32_t aos_and_or(uint32_t a, uint32_t smask, uint32_t vmagic) {
-  uint32_t r;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(smask), "v"(vmagic));
-  return r;
+  return (a & smask) | vmagic;
 }
 
 __device__ __forceinline__ u32x4 aos_q4_magic(uint32_t w, uint32_t smask, uint32_t vmagic) {
@@ -95,7 +96,11 @@ __device__ __forceinline__ u32x4 aos_q4_magic(uint32_t w, uint32_t smask, uint32
 
 /* Uniform (SGPR) copies of the extraction constants. */
 __device__ __forceinline__ uint32_t aos_q4_mask() { return __builtin_amdgcn_readfirstlane(0x000F000Fu); }
-__device__ __forceinline__ uint32_t aos_q4_exp() { return 0x43004300u; }
+__device__ __forceinline__ uint32_t aos_q4_exp() { /* (a value the compiler cannot fold into a literal) */
+  uint32_t v = 0x43004300u;
+  asm("" : "+v"(v));
+  return v;
+}
 
 /* 16-byte load through the global address space. Pointers read from tables (adapter rows, the
  * union's B pointers) are otherwise generic, and a generic (flat) load counts against the LDS

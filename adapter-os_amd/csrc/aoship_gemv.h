@@ -59,6 +59,17 @@ __device__ __forceinline__ float load_f(const float *a, bool coherent) {
   return coherent ? __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *a;
 }
 
+/* Four values of S at element `at` (a multiple of 4; S is 16-byte aligned). coherent: one 16-byte load with the
+ * device scope of load_f. Such loads bypass L2, so their cost is their requests: as eight 4-byte loads per
+ * expand step, S took most of a 32-token launch. */
+__device__ __forceinline__ float4 load_s4(const float *S, int at, bool coherent) {
+  if (coherent) {
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)S, (short)0, -1, 0x00020000);
+    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, at * 4, 0, 16));
+  }
+  return *(const float4 *)(S + at);
+}
+
 /* Row pointer of union slot u in a table the plan lists (pk = 1 + its pointer table). */
 __device__ __forceinline__ const uint16_t *plan_ptr(const aos_gemv_params &p, int pk, int u, bool coherent) {
   const uint64_t *a = &p.plan->ptr[pk - 1][u];
@@ -83,7 +94,7 @@ __device__ __forceinline__ void expand_load_b(const aos_gemv_params &p, const ao
   const int a = coherent ? (int)__hip_atomic_load(&p.plan->list[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
                          : (int)p.plan->list[u];
   e.a = a;
-  e.cf = i < p.T ? load_f(&p.plan->coef[ti][u], coherent) : 0.0f;
+  e.cf = i < p.T ? load_f(&p.plan->coef[u][ti], coherent) : 0.0f;
   const uint16_t *B = slot_ptr(p, tab.B, pk, u, a, coherent);
   const uint16_t *bp = B ? B + (size_t)row * rpad + j0 + 8 * c : p.zero_row;
   e.b = aos_gld16(bp);
@@ -97,14 +108,9 @@ __device__ __forceinline__ void expand_load_s(const aos_gemv_params &p, const ao
   const int rpad = tab.rpad;
   const int colq = 16 * q, u = colq / rpad, j0 = colq - u * rpad;
   const int scol = (p.s_all ? e.a : u) * rpad + j0 + 8 * c;
-  const float *sp = S + (size_t)ti * stride + scol;
-  if (coherent) {
-    e.s0 = make_float4(load_f(sp, true), load_f(sp + 1, true), load_f(sp + 2, true), load_f(sp + 3, true));
-    e.s1 = make_float4(load_f(sp + 4, true), load_f(sp + 5, true), load_f(sp + 6, true), load_f(sp + 7, true));
-  } else {
-    e.s0 = *(const float4 *)sp;
-    e.s1 = *(const float4 *)(sp + 4);
-  }
+  const int sp = ti * stride + scol;
+  e.s0 = load_s4(S, sp, coherent);
+  e.s1 = load_s4(S, sp + 4, coherent);
 }
 
 __device__ __forceinline__ void expand_load(const aos_gemv_params &p, const aos_lora_tab &tab, int pk, const float *S,
@@ -134,7 +140,7 @@ __device__ __forceinline__ PlanPart expand_plan_part(const aos_gemv_params &p, i
   r.j0 = colq - u0 * rpad;
   r.u = u0 < AOS_PLAN_MAXU ? u0 : AOS_PLAN_MAXU - 1;
   e.a = (int)__hip_atomic_load(&p.plan->list[r.u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const float cf = load_f(&p.plan->coef[ti][r.u], true);
+  const float cf = load_f(&p.plan->coef[r.u][ti], true);
   e.cf = i < p.T ? cf : 0.0f;
   r.B = plan_ptr(p, pk, r.u, true);
   return r;
@@ -150,9 +156,9 @@ __device__ __forceinline__ void expand_s_of(const aos_gemv_params &p, int rpad, 
                                             const float *S, int stride, int lane, ExpandStep &e) {
   const int i = lane & 31, c = lane >> 5;
   const int ti = i < p.T ? i : 0;
-  const float *sp = S + (in ? (size_t)ti * stride + (p.s_all ? e.a : pp.u) * rpad + pp.j0 + 8 * c : 0);
-  e.s0 = make_float4(load_f(sp, true), load_f(sp + 1, true), load_f(sp + 2, true), load_f(sp + 3, true));
-  e.s1 = make_float4(load_f(sp + 4, true), load_f(sp + 5, true), load_f(sp + 6, true), load_f(sp + 7, true));
+  const int sp = in ? ti * stride + (p.s_all ? e.a : pp.u) * rpad + pp.j0 + 8 * c : 0;
+  e.s0 = load_s4(S, sp, true);
+  e.s1 = load_s4(S, sp + 4, true);
 }
 
 __device__ __forceinline__ void expand_apply(const ExpandStep &e, f32x16 &f) {
@@ -198,16 +204,11 @@ __device__ __forceinline__ void expand_rest(const aos_gemv_params &p, const aos_
     for (int k = 0; k < EB; ++k) {
       if (qb + k * qs >= nq) continue;
       e[k].a = a[k];
-      e[k].cf = i < p.T ? load_f(&p.plan->coef[ti][u[k]], coherent) : 0.0f;
+      e[k].cf = i < p.T ? load_f(&p.plan->coef[u[k]][ti], coherent) : 0.0f;
       e[k].b = aos_gld16(bptr[k] ? bptr[k] + (size_t)row * rpad + j0[k] + 8 * c : p.zero_row);
-      const float *sp = S + (size_t)ti * stride + (p.s_all ? a[k] : u[k]) * rpad + j0[k] + 8 * c;
-      if (coherent) {
-        e[k].s0 = make_float4(load_f(sp, true), load_f(sp + 1, true), load_f(sp + 2, true), load_f(sp + 3, true));
-        e[k].s1 = make_float4(load_f(sp + 4, true), load_f(sp + 5, true), load_f(sp + 6, true), load_f(sp + 7, true));
-      } else {
-        e[k].s0 = *(const float4 *)sp;
-        e[k].s1 = *(const float4 *)(sp + 4);
-      }
+      const int sp = ti * stride + (p.s_all ? a[k] : u[k]) * rpad + j0[k] + 8 * c;
+      e[k].s0 = load_s4(S, sp, coherent);
+      e[k].s1 = load_s4(S, sp + 4, coherent);
     }
 #pragma unroll
     for (int k = 0; k < EB; ++k)
@@ -265,16 +266,11 @@ __device__ __forceinline__ void expand_rest2(const aos_gemv_params &p, int qa, i
       for (int k = 0; k < EB; ++k) {
         if (!on[m][k]) continue;
         e[m][k].a = a[m][k];
-        e[m][k].cf = i < p.T ? load_f(&p.plan->coef[ti][u[m][k]], coherent) : 0.0f;
+        e[m][k].cf = i < p.T ? load_f(&p.plan->coef[u[m][k]][ti], coherent) : 0.0f;
         e[m][k].b = aos_gld16(bptr[m][k] ? bptr[m][k] + (size_t)row * rpad + j0[m][k] + 8 * c : p.zero_row);
-        const float *sp = S + (size_t)ti * stride + (p.s_all ? a[m][k] : u[m][k]) * rpad + j0[m][k] + 8 * c;
-        if (coherent) {
-          e[m][k].s0 = make_float4(load_f(sp, true), load_f(sp + 1, true), load_f(sp + 2, true), load_f(sp + 3, true));
-          e[m][k].s1 = make_float4(load_f(sp + 4, true), load_f(sp + 5, true), load_f(sp + 6, true), load_f(sp + 7, true));
-        } else {
-          e[m][k].s0 = *(const float4 *)sp;
-          e[m][k].s1 = *(const float4 *)(sp + 4);
-        }
+        const int sp = ti * stride + (p.s_all ? a[m][k] : u[m][k]) * rpad + j0[m][k] + 8 * c;
+        e[m][k].s0 = load_s4(S, sp, coherent);
+        e[m][k].s1 = load_s4(S, sp + 4, coherent);
       }
     }
 #pragma unroll
@@ -444,6 +440,85 @@ __device__ __forceinline__ bool poll_lines_once(const uint32_t *lines, int n, ui
   return all;
 }
 
+/* K groups ga .. ga + ng - 1 of row block rb (and of the up matrix's with SW) for 3-32 tokens, with x
+ * read by the wave itself: a wave's K piece is its own, so a slice of x staged in LDS would serve no
+ * other wave of the workgroup, and its size bounded the workgroups per CU and forced K splits whose
+ * partials cost more than x does (x comes out of L2: 4 KB a group beside 2 KB of each matrix). The
+ * group's sum of x, which the bias term needs per token, is formed by the matrix cores as well (x
+ * times a column of ones, in the accumulators' layout). Lanes without a token read the last token's
+ * row; their accumulators are never stored. Requires ng >= 1. */
+template <int NV, bool SW, int D>
+__device__ __forceinline__ void stream_direct(const aos_gemv_params &p, int rb, int ga, int ng, int lane,
+                                              float (&acc0)[NV], float (&acc1)[NV]) {
+  constexpr int XD = 2; /* groups of x in flight */
+  static_assert(D % XD == 0, "the x ring's slot must be static in the unrolled loop");
+  const int G = p.w0.G, in = p.w0.in, T = p.T;
+  const int i = lane & 31, c = lane >> 5;
+  const uint32_t qmask = aos_q4_mask(), qexp = aos_q4_exp();
+  const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+  const u32x4 *q0 = (const u32x4 *)p.w0.qt + ((size_t)rb * G + ga) * 64 + lane;
+  const uint32_t *s0 = p.w0.sb + ((size_t)rb * G + ga) * 32 + i;
+  const u32x4 *q1 = SW ? (const u32x4 *)p.w1.qt + ((size_t)rb * G + ga) * 64 + lane : nullptr;
+  const uint32_t *s1 = SW ? p.w1.sb + ((size_t)rb * G + ga) * 32 + i : nullptr;
+  const u32x4 *xp = (const u32x4 *)(p.x + (size_t)(i < T ? i : T - 1) * in + (size_t)ga * 64 + 32 * c);
+  u32x4 wa[D], wb[D], xr[XD][4];
+  uint32_t sa[D], sb[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const int jj = d < ng ? d : ng - 1;
+    wa[d] = q0[(size_t)jj * 64];
+    sa[d] = s0[(size_t)jj * 32];
+    if (SW) {
+      wb[d] = q1[(size_t)jj * 64];
+      sb[d] = s1[(size_t)jj * 32];
+    }
+    if (d < XD) {
+#pragma unroll
+      for (int st = 0; st < 4; ++st) xr[d][st] = xp[(size_t)jj * 8 + st];
+    }
+  }
+  for (int base = 0; base < ng; base += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int j = base + d;
+      if (j < ng) {
+        f32x16 t0 = {}, t1 = {}, tx = {};
+#pragma unroll
+        for (int st = 0; st < 4; ++st) {
+          const u32x4 a = xr[d % XD][st];
+          t0 = aos_mfma32(a, aos_q4_magic(wa[d][st], qmask, qexp), t0);
+          if (SW) t1 = aos_mfma32(a, aos_q4_magic(wb[d][st], qmask, qexp), t1);
+          tx = aos_mfma32(a, ones, tx);
+        }
+        const float c0 = aos_f16_to_f32(sa[d] & 0xffffu), b0 = fmaf(-128.0f, c0, aos_f16_to_f32(sa[d] >> 16));
+        const float c1 = SW ? aos_f16_to_f32(sb[d] & 0xffffu) : 0.0f;
+        const float b1 = SW ? fmaf(-128.0f, c1, aos_f16_to_f32(sb[d] >> 16)) : 0.0f;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+          acc0[v] = fmaf(c0, t0[v], fmaf(b0, tx[v], acc0[v]));
+          if (SW) acc1[v] = fmaf(c1, t1[v], fmaf(b1, tx[v], acc1[v]));
+        }
+        if (NV < 16) {
+          aos_mfma_hold(t0);
+          if (SW) aos_mfma_hold(t1);
+          aos_mfma_hold(tx);
+        }
+      }
+      int jn = j + D, jx = j + XD; /* refills past the end reload the last group and are never used */
+      jn = jn < ng ? jn : ng - 1;
+      jx = jx < ng ? jx : ng - 1;
+      wa[d] = q0[(size_t)jn * 64];
+      sa[d] = s0[(size_t)jn * 32];
+      if (SW) {
+        wb[d] = q1[(size_t)jn * 64];
+        sb[d] = s1[(size_t)jn * 32];
+      }
+#pragma unroll
+      for (int st = 0; st < 4; ++st) xr[d % XD][st] = xp[(size_t)jx * 8 + st];
+    }
+  }
+}
+
 /* Row-block group rbg, K split ksi of one matrix (or of the gate/up pair): the workgroup's waves
  * cover p.wr row blocks (wave w: row block p.wr * rbg + w % p.wr, K piece w / p.wr of the split),
  * all reading the one x slice staged for the split. Waves of a row block past the matrix (the
@@ -454,8 +529,9 @@ __device__ __forceinline__ bool poll_lines_once(const uint32_t *lines, int n, ui
  * MLP turns them off, since in its kernel they cost the compiler's promotion of the kernel
  * arguments to registers (the arguments would be copied to private memory). PP: when the plan
  * arrives after the K loop, poll the other producers with the plan's parts (the launch with the
- * router, whose plan comes last; elsewhere the extra loads measured slower). */
-template <int NV, bool SW, int W, int D, bool XL = false, bool DP = true, bool PP = false>
+ * router, whose plan comes last; elsewhere the extra loads measured slower). DX: the waves read x
+ * themselves (stream_direct); one row block per workgroup. */
+template <int NV, bool SW, int W, int D, bool XL = false, bool DP = true, bool PP = false, bool DX = false>
 __device__ __forceinline__ void gemv_body(const aos_gemv_params &p, int rbg, int ksi, const uint32_t *xflag = nullptr) {
   constexpr int NA = SW ? 2 : 1;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -463,8 +539,8 @@ __device__ __forceinline__ void gemv_body(const aos_gemv_params &p, int rbg, int
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6); /* uniform: keeps the loop scalar */
   const int G = p.w0.G, in = p.w0.in, T = p.T;
   const int i = lane & 31, c = lane >> 5;
-  const int WR = p.wr, WK = W / WR;
-  const int wr = wave % WR, wk = wave / WR;
+  const int WR = DX ? 1 : p.wr, WK = W / WR;
+  const int wr = DX ? 0 : wave % WR, wk = DX ? wave : wave / WR;
   const bool live = rbg * WR + wr < p.w0.RB;
   const int rb = live ? rbg * WR + wr : p.w0.RB - 1;
   const int row = rb * 32 + i;
@@ -492,13 +568,14 @@ __device__ __forceinline__ void gemv_body(const aos_gemv_params &p, int rbg, int
     const int U = __builtin_amdgcn_readfirstlane(p.plan->U);
     nq0 = p.tab0.rpad ? U * p.tab0.rpad / 16 : 0;
     nq1 = (SW && p.tab1.rpad) ? U * p.tab1.rpad / 16 : 0;
-    if (SW && q_first < nq0) expand_load(p, p.tab0, p.pk0, p.S0, p.s_stride0, q_first, row, lane, e0);
-    if (SW && q_first < nq1) expand_load(p, p.tab1, p.pk1, p.S1, p.s_stride1, q_first, row, lane, e1);
+    if (SW && !DX && q_first < nq0) expand_load(p, p.tab0, p.pk0, p.S0, p.s_stride0, q_first, row, lane, e0);
+    if (SW && !DX && q_first < nq1) expand_load(p, p.tab1, p.pk1, p.S1, p.s_stride1, q_first, row, lane, e1);
   }
   /* a fused launch whose plan comes from an earlier launch (only S is produced here): the plan and
    * the first step's B fragments load before the K loop, so that after it only S is waited for.
-   * Not with XL: the one-launch MLP's down GEMV reads a plan built earlier in its own launch. */
-  const bool plan_early = !XL && expands && fused && p.pre_lines != nullptr && p.plan_line < 0;
+   * Not in the SwiGLU kernels that read x themselves (registers), and not with XL: the one-launch
+   * MLP's down GEMV reads a plan built earlier in its own launch. */
+  const bool plan_early = !XL && !(DX && SW) && expands && fused && p.pre_lines != nullptr && p.plan_line < 0;
   /* direct: the plan lists the row pointers of every table read through it, so wave 0 waits for
    * every producer's line at once, and the first expand step then costs two round trips (the
    * plan's part with U, then the B fragments and S) rather than five. (Measured and not kept:
@@ -508,7 +585,7 @@ __device__ __forceinline__ void gemv_body(const aos_gemv_params &p, int rbg, int
                       (!SW || p.tab1.rpad == 0 || p.pk1 != 0) && (!SW || p.hpart == nullptr || p.pkh != 0);
   /* single-matrix kernels with the direct loads: the wave's next NB steps (q_first + k q_step,
    * k = 1 .. NB) load with its first, so that its first NB + 1 steps cost the round trips of one */
-  constexpr int NB = (SW || NV == 1) ? 0 : 3;
+  constexpr int NB = (SW || NV == 1) ? 0 : (DX && NV == 16) ? 1 : 3;
   ExpandStep er[NB > 0 ? NB : 1];
   PlanPart pr[NB > 0 ? NB : 1];
   if (plan_early) {
@@ -520,7 +597,11 @@ __device__ __forceinline__ void gemv_body(const aos_gemv_params &p, int rbg, int
     if (q_first < nq0) expand_load_b(p, p.tab0, p.pk0, q_first, row, lane, e0, false);
     if (SW && q_first < nq1) expand_load_b(p, p.tab1, p.pk1, q_first, row, lane, e1, false);
   }
-  {
+  if constexpr (DX) {
+    const int wt = ksi * W + wave, wn = p.ks * W; /* the row block's waves share its groups evenly */
+    const int ga = (int)((long)wt * G / wn), gb = (int)((long)(wt + 1) * G / wn);
+    stream_direct<NV, SW, D>(p, rb, ga, gb - ga, lane, acc0, acc1);
+  } else {
     const int gw0 = (int)((long)ksi * G / p.ks), gw1 = (int)((long)(ksi + 1) * G / p.ks);
     const int GR = gw1 - gw0;
     const int ga = gw0 + wk * GR / WK, gb = gw0 + (wk + 1) * GR / WK, ng = gb - ga;
@@ -661,7 +742,7 @@ __device__ __forceinline__ void gemv_body(const aos_gemv_params &p, int rbg, int
      * then overlap the shrink's tail). Plan from an earlier launch: wait, then S. */
     if (!plan_early) {
       const bool all_up = poll_lines_once(p.pre_lines, p.n_pre_lines, p.gen, lane);
-      bool ready = all_up || aos_wait_lines(p.pre_lines + (size_t)p.plan_line * 32, 1, p.gen, lane);
+      bool ready = all_up || (DX && p.plan_line < 0) || aos_wait_lines(p.pre_lines + (size_t)p.plan_line * 32, 1, p.gen, lane);
       PlanPart pe0 = {}, pe1 = {};
       int Ue = 0;
       if (ready) {
@@ -758,6 +839,7 @@ __device__ __forceinline__ void gemv_body(const aos_gemv_params &p, int rbg, int
       }
     }
     lds_barrier();
+    aos_compiler_barrier();
     if (ok && expands && !plan_early) {
       int U = __builtin_amdgcn_readfirstlane(
           __hip_atomic_load(&p.plan->U, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
@@ -785,6 +867,7 @@ __device__ __forceinline__ void gemv_body(const aos_gemv_params &p, int rbg, int
         }
       }
       lds_barrier();
+      aos_compiler_barrier();
       if (!ok2) {
         nq0 = 0;
         nq1 = 0;
@@ -801,8 +884,9 @@ __device__ __forceinline__ void gemv_body(const aos_gemv_params &p, int rbg, int
     } else if (fused) {
       if (q_first < nq0) expand_load_s(p, p.tab0, p.S0, p.s_stride0, q_first, lane, e0, true);
       if (SW && q_first < nq1) expand_load_s(p, p.tab1, p.S1, p.s_stride1, q_first, lane, e1, true);
-    } else if (!SW && q_first < nq0) {
-      expand_load(p, p.tab0, p.pk0, p.S0, p.s_stride0, q_first, row, lane, e0);
+    } else if (!SW || DX) {
+      if (q_first < nq0) expand_load(p, p.tab0, p.pk0, p.S0, p.s_stride0, q_first, row, lane, e0);
+      if (SW && q_first < nq1) expand_load(p, p.tab1, p.pk1, p.S1, p.s_stride1, q_first, row, lane, e1);
     }
     if (q_first < nq0) expand_apply(e0, f0);
     if (SW && q_first < nq1) expand_apply(e1, f1);
@@ -843,6 +927,25 @@ __device__ __forceinline__ void gemv_body(const aos_gemv_params &p, int rbg, int
     }
   }
   lds_barrier();
+  if (DX && p.ks == 1) { /* the whole row block is here: each wave sums and stores its share of the tokens */
+    constexpr int VW = NV / W > 0 ? NV / W : 1;
+#pragma unroll
+    for (int k = 0; k < VW; ++k) {
+      const int v = wave * VW + k;
+      const int m = aos_acc_m(v, lane);
+      if (v >= NV || m >= T) continue;
+      float a0 = red[v * 64 + lane], a1 = SW ? red[(NV + v) * 64 + lane] : 0.0f;
+#pragma unroll
+      for (int w = 1; w < W; ++w) {
+        a0 += red[(w * NA * NV + v) * 64 + lane];
+        if (SW) a1 += red[(w * NA * NV + NV + v) * 64 + lane];
+      }
+      if (SW) a0 = (a0 * (1.0f / (1.0f + expf(-a0)))) * a1;
+      if (!SW && p.yf) p.yf[(size_t)m * p.w0.out + row] = a0;
+      else p.y[(size_t)m * p.w0.out + row] = aos_f32_to_bf16(a0);
+    }
+    return;
+  }
   if (wk != 0) return;
   if (WK > 1) {
 #pragma unroll
@@ -878,11 +981,12 @@ __device__ __forceinline__ void gemv_body(const aos_gemv_params &p, int rbg, int
       acc0[v] = 0.0f;
       acc1[v] = 0.0f;
     }
-    /* partials are read 4 at a time (all loads in flight together) and summed in order */
-    for (int k0 = 0; k0 < nsplit; k0 += 4) {
-      float v0[4][NV], v1[4][NV];
+    /* partials are read PB at a time (all loads in flight together) and summed in order */
+    constexpr int PB = DX && SW && NV == 16 ? 2 : 4; /* (registers) */
+    for (int k0 = 0; k0 < nsplit; k0 += PB) {
+      float v0[PB][NV], v1[PB][NV];
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
+      for (int kk = 0; kk < PB; ++kk) {
         const int k = k0 + kk < nsplit ? k0 + kk : nsplit - 1;
         const float *pp = p.part + ((size_t)rb * nsplit + k) * (NA * NV * 64);
 #pragma unroll
@@ -892,7 +996,7 @@ __device__ __forceinline__ void gemv_body(const aos_gemv_params &p, int rbg, int
         }
       }
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk)
+      for (int kk = 0; kk < PB; ++kk)
         if (k0 + kk < nsplit) {
 #pragma unroll
           for (int v = 0; v < NV; ++v) {

@@ -31,32 +31,36 @@ namespace {
 
 using namespace aos_gemv;
 
-template <int NV, bool SW, int W, int D>
-__global__ void __launch_bounds__(64 * W) aos_gemv_kernel(aos_gemv_params p) {
-  gemv_body<NV, SW, W, D>(p, blockIdx.x, blockIdx.y);
+/* Waves per SIMD that the kernels reading x themselves are held to: their whole grid is resident then
+ * (the 7B gate/up launch is 592 workgroups and its producers), so that its wait for S is paid once. */
+constexpr int dx_waves(bool sw) { return sw ? 3 : 4; }
+
+template <int NV, bool SW, int W, int D, bool DX = false>
+__global__ void __launch_bounds__(64 * W, DX ? dx_waves(SW) : 1) aos_gemv_kernel(aos_gemv_params p) {
+  gemv_body<NV, SW, W, D, false, true, false, DX>(p, blockIdx.x, blockIdx.y);
 }
 
 /* Up to three matrices sharing x (q, k and v) in one launch: workgroup b of the 1-D grid is row
  * block b % RB, K split b / RB of the matrix whose range of workgroups holds it. */
-template <int NV, int W, int D>
-__global__ void __launch_bounds__(64 * W) aos_gemv3_kernel(aos_gemv3_params mp) {
+template <int NV, int W, int D, bool DX = false>
+__global__ void __launch_bounds__(64 * W, DX ? dx_waves(false) : 1) aos_gemv3_kernel(aos_gemv3_params mp) {
   const int b = blockIdx.x;
   if (b < mp.wg_end[0]) {
-    gemv_body<NV, false, W, D>(mp.p[0], b % mp.p[0].nrbg, b / mp.p[0].nrbg);
+    gemv_body<NV, false, W, D, false, true, false, DX>(mp.p[0], b % mp.p[0].nrbg, b / mp.p[0].nrbg);
   } else if (b < mp.wg_end[1]) {
     const int r = b - mp.wg_end[0];
-    gemv_body<NV, false, W, D>(mp.p[1], r % mp.p[1].nrbg, r / mp.p[1].nrbg);
+    gemv_body<NV, false, W, D, false, true, false, DX>(mp.p[1], r % mp.p[1].nrbg, r / mp.p[1].nrbg);
   } else {
     const int r = b - mp.wg_end[1];
-    gemv_body<NV, false, W, D>(mp.p[2], r % mp.p[2].nrbg, r / mp.p[2].nrbg);
+    gemv_body<NV, false, W, D, false, true, false, DX>(mp.p[2], r % mp.p[2].nrbg, r / mp.p[2].nrbg);
   }
 }
 
 /* A shrink (workgroups [0, n_pre)) and the GEMVs consuming its S (the rest) in one launch. Each
  * shrink workgroup, once its stores are complete, counts itself into sync; the last one raises
  * every GEMV workgroup's ready flag. */
-template <int NV, bool SW, int W, int D>
-__global__ void __launch_bounds__(64 * W) aos_gemv_fused_kernel(aos_gemv_fused_params fp) {
+template <int NV, bool SW, int W, int D, bool DX = false>
+__global__ void __launch_bounds__(64 * W, DX ? dx_waves(SW) : 1) aos_gemv_fused_kernel(aos_gemv_fused_params fp) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int b = blockIdx.x;
   if (b < fp.n_pre) {
@@ -73,7 +77,7 @@ __global__ void __launch_bounds__(64 * W) aos_gemv_fused_kernel(aos_gemv_fused_p
   const aos_gemv_params &g = *(const aos_gemv_params *)((const char *)__builtin_amdgcn_kernarg_segment_ptr() +
                                                         offsetof(aos_gemv_fused_params, gp) +
                                                         (size_t)m * sizeof(aos_gemv_params));
-  gemv_body<NV, SW, W, D>(g, r % g.nrbg, r / g.nrbg);
+  gemv_body<NV, SW, W, D, false, true, false, DX>(g, r % g.nrbg, r / g.nrbg);
 }
 
 /* The decode MLP of 1-2 tokens in one launch (4-wave workgroups throughout):
@@ -137,7 +141,12 @@ int launchf_nv(const aos_gemv_fused_params *fp, int swiglu, const aos_launch_ctx
   const int nwg = fp->n_pre + (int)fp->n_cons;
   size_t lds = fp->hsum ? (size_t)HSUM_V * 64 * (fp->gp[0].waves) * 4 : (size_t)fp->sp.lds_bytes;
   for (int i = 0; i < fp->n; ++i) lds = lds > (size_t)fp->gp[i].lds_bytes ? lds : (size_t)fp->gp[i].lds_bytes;
-  if (swiglu) {
+  if (fp->gp[0].dx) {
+    if constexpr (NV >= 4) {
+      if (swiglu) AOS_LAUNCH(ctx, (aos_gemv_fused_kernel<NV, true, 4, 2, true>), dim3(nwg), dim3(256), lds, *fp);
+      else AOS_LAUNCH(ctx, (aos_gemv_fused_kernel<NV, false, 4, 4, true>), dim3(nwg), dim3(256), lds, *fp);
+    }
+  } else if (swiglu) {
     AOS_LAUNCH(ctx, (aos_gemv_fused_kernel<NV, true, 4, AOS_GU_RING>), dim3(nwg), dim3(256), lds, *fp);
   } else if (fp->gp[0].waves == 4) {
     AOS_LAUNCH(ctx, (aos_gemv_fused_kernel<NV, false, 4, AOS_ONE_RING>), dim3(nwg), dim3(256), lds, *fp);
@@ -152,7 +161,10 @@ int launch3_nv(const aos_gemv3_params *mp, const aos_launch_ctx *ctx) {
   const int nwg = mp->wg_end[mp->n - 1];
   size_t lds = 0;
   for (int i = 0; i < mp->n; ++i) lds = lds > (size_t)mp->p[i].lds_bytes ? lds : (size_t)mp->p[i].lds_bytes;
-  if (mp->p[0].waves == 4) {
+  if (mp->p[0].dx) {
+    if constexpr (NV >= 4)
+      AOS_LAUNCH(ctx, (aos_gemv3_kernel<NV, 4, 4, true>), dim3(nwg), dim3(256), lds, *mp);
+  } else if (mp->p[0].waves == 4) {
     AOS_LAUNCH(ctx, (aos_gemv3_kernel<NV, 4, 12>), dim3(nwg), dim3(256), lds, *mp);
   } else {
     AOS_LAUNCH(ctx, (aos_gemv3_kernel<NV, 8, 12>), dim3(nwg), dim3(512), lds, *mp);
@@ -164,7 +176,12 @@ template <int NV>
 int launch_nv(const aos_gemv_params *p, int swiglu, const aos_launch_ctx *ctx) {
   dim3 grid(p->nrbg, p->ks);
   const size_t lds = p->lds_bytes;
-  if (swiglu) {
+  if (p->dx) {
+    if constexpr (NV >= 4) {
+      if (swiglu) AOS_LAUNCH(ctx, (aos_gemv_kernel<NV, true, 4, 2, true>), grid, dim3(256), lds, *p);
+      else AOS_LAUNCH(ctx, (aos_gemv_kernel<NV, false, 4, 4, true>), grid, dim3(256), lds, *p);
+    }
+  } else if (swiglu) {
     AOS_LAUNCH(ctx, (aos_gemv_kernel<NV, true, 4, 4>), grid, dim3(256), lds, *p);
   } else if (p->waves == 4) {
     AOS_LAUNCH(ctx, (aos_gemv_kernel<NV, false, 4, 12>), grid, dim3(256), lds, *p);
@@ -180,6 +197,8 @@ int launch_nv(const aos_gemv_params *p, int swiglu, const aos_launch_ctx *ctx) {
  * the one-launch hand-off (which use the workgroup's LDS per row block) only with wr == 1. */
 static bool rbg_ok(const aos_gemv_params &p) {
   if (p.wr < 1 || p.waves % p.wr || p.w0.RB < 1 || p.nrbg != (p.w0.RB + p.wr - 1) / p.wr) return false;
+  if (p.dx) /* x read by the waves: 4 waves on one row block, a K group for each wave */
+    return p.wr == 1 && p.waves == 4 && p.T > 2 && !p.hpart && !p.hdone && p.ks >= 1 && 4 * p.ks <= p.w0.G;
   return p.wr == 1 || (!p.hpart && !p.hdone);
 }
 
@@ -207,7 +226,7 @@ extern "C" int aos_launch_gemv3(const aos_gemv3_params *mp, const aos_launch_ctx
   for (int i = 0; i < 3; ++i) {
     if (i < n) {
       const aos_gemv_params &p = mp->p[i];
-      if (p.waves != waves || p.T != T || !rbg_ok(p) || p.ks < 1) return (int)hipErrorInvalidValue;
+      if (p.waves != waves || p.T != T || p.dx != mp->p[0].dx || !rbg_ok(p) || p.ks < 1) return (int)hipErrorInvalidValue;
       end += p.nrbg * p.ks;
     }
     if (mp->wg_end[i] != end) return (int)hipErrorInvalidValue;
@@ -259,7 +278,7 @@ extern "C" int aos_fused_params_ok(const aos_gemv_fused_params *fp, int swiglu) 
   for (int i = 0; i < 3; ++i) {
     if (i < n) {
       const aos_gemv_params &p = fp->gp[i];
-      if (p.waves != waves || p.T != T || !rbg_ok(p) || p.ks < 1 || p.gen != fp->gen) return false;
+      if (p.waves != waves || p.T != T || p.dx != fp->gp[0].dx || !rbg_ok(p) || p.ks < 1 || p.gen != fp->gen) return false;
       if (lines ? (p.pre_lines != fp->lines || p.n_pre_lines != fp->n_lines || p.plan_line != plan_line ||
                    p.sync != nullptr)
                 : (p.sync != fp->sync || p.flags != fp->flags + (size_t)end * 32 ||

@@ -78,7 +78,7 @@ typedef struct {
   int U;
   int pad[3];
   uint16_t list[AOS_PLAN_MAXU];
-  float coef[AOS_DECODE_MAX_T][AOS_PLAN_MAXU];
+  float coef[AOS_PLAN_MAXU][AOS_DECODE_MAX_T]; /* a slot's tokens side by side: one line for a wave's lanes */
   uint64_t ptr[AOS_PLAN_NPTR][AOS_PLAN_MAXU];
 } aos_plan;
 
@@ -158,6 +158,8 @@ typedef struct {
                          w / wr of the workgroup's K split; all of them share the staged x */
   int nrbg;           /* row-block groups: ceil(RB / wr); workgroup (rbg, ksi) of the grid */
   int lds_bytes;      /* dynamic LDS: x staging + group sums, or the wave reduction */
+  int dx;             /* 1: 3-32 tokens with x read by the waves (stream_direct): wr == 1, 4 waves; lds_bytes holds
+                       * the wave reduction only */
   int has_expand;     /* 1: the K-split workgroups of each row block add the LoRA expand */
   /* LoRA expand: coef(t, u) * S[t][col(u) + j] . B_list[u][row][j] over the plan's union */
   aos_lora_tab tab0, tab1;

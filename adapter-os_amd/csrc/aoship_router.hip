@@ -243,8 +243,8 @@ __device__ __forceinline__ bool route_part_block(const aos_route_gu_params &q, i
  * the arrival word */
 __host__ __device__ constexpr size_t rgu_tabs_off(int d, int n) { return ((size_t)(d + n + 4) * 4 + 15) & ~(size_t)15; }
 
-template <int NV>
-__global__ void __launch_bounds__(256) aos_route_gu_kernel(aos_route_gu_params q) {
+template <int NV, bool DX = false>
+__global__ void __launch_bounds__(256, DX ? 3 : 1) aos_route_gu_kernel(aos_route_gu_params q) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int T = q.rp.T, R = q.rparts;
   const int b = blockIdx.x;
@@ -301,7 +301,7 @@ __global__ void __launch_bounds__(256) aos_route_gu_kernel(aos_route_gu_params q
     return;
   }
   const int r = b2 - q.fp.n_pre;
-  aos_gemv::gemv_body<NV, true, 4, 4, false, true, true>(q.fp.gp[0], r % q.fp.gp[0].nrbg, r / q.fp.gp[0].nrbg);
+  aos_gemv::gemv_body<NV, true, 4, DX ? 2 : 4, false, true, true, DX>(q.fp.gp[0], r % q.fp.gp[0].nrbg, r / q.fp.gp[0].nrbg);
 }
 
 template <int NV>
@@ -310,7 +310,11 @@ int launch_rgu(const aos_route_gu_params *q, const aos_launch_ctx *ctx) {
   size_t lds = rgu_tabs_off(q->rp.d, q->rp.n) + sizeof(aos_shrink::PlanTabs);
   if ((size_t)q->fp.sp.lds_bytes > lds) lds = (size_t)q->fp.sp.lds_bytes;
   if ((size_t)q->fp.gp[0].lds_bytes > lds) lds = (size_t)q->fp.gp[0].lds_bytes;
-  AOS_LAUNCH(ctx, aos_route_gu_kernel<NV>, dim3(nwg), dim3(256), lds, *q);
+  if (q->fp.gp[0].dx) {
+    if constexpr (NV >= 4) AOS_LAUNCH(ctx, (aos_route_gu_kernel<NV, true>), dim3(nwg), dim3(256), lds, *q);
+  } else {
+    AOS_LAUNCH(ctx, (aos_route_gu_kernel<NV>), dim3(nwg), dim3(256), lds, *q);
+  }
   return (int)hipGetLastError();
 }
 

@@ -76,7 +76,7 @@ __device__ __forceinline__ void plan_tabs_store(const aos_plan_params &pp, const
 
 /* Plan of one call, built by a whole workgroup: ring slot s of token t contributes adapter
  * a = adapter_indices[s] when s < top_k, its gate q > 0 and the adapter is bound
- * (backend.rs:409-425 skips q <= 0 and unknown handles). coef[t][u] = sum over such slots of
+ * (backend.rs:409-425 skips q <= 0 and unknown handles). coef[u][t] = sum over such slots of
  * scale[a] * (float(q) / 32767.0f), the product mod.scale * blend_weights[i] of the MLX
  * forward. */
 /* lt: the per-adapter inputs staged in LDS (NULL: read from memory). own_rings: the rings were written
@@ -133,7 +133,7 @@ __device__ __forceinline__ void build_plan(const aos_plan_params &pp, const Plan
     if (tid < U && pp.ptab[k]) pv[k] = lt ? lt->ptr[k][list[tid]] : (uint64_t)aos_gld_ptr(pp.ptab[k] + list[tid]);
   }
   for (int idx = tid; idx < pp.T * U; idx += nt) {
-    const int t = idx / U, u = idx - t * U;
+    const int u = idx / pp.T, t = idx - u * pp.T;
     const int a = list[u];
     const aoship_ring_t &r = rs[t];
     float c = 0.0f;
@@ -143,7 +143,7 @@ __device__ __forceinline__ void build_plan(const aos_plan_params &pp, const Plan
         c += (lt ? lt->scale[a] : pp.scale[a]) * blend;
       }
     }
-    aos_publish(&pp.plan->coef[t][u], c);
+    aos_publish(&pp.plan->coef[u][t], c);
   }
 #pragma unroll
   for (int k = 0; k < AOS_PLAN_NPTR; ++k) {
@@ -296,18 +296,20 @@ __device__ __forceinline__ bool shrink_block(const aos_shrink_params &p, int lrb
     if (lane == 0) aos_reset(&p.counters[rb_global]);
 #pragma unroll
     for (int v = 0; v < NV; ++v) tot[v] = 0.0f;
-    /* partials are read 8 at a time (all loads in flight together) and summed in order */
-    for (int k0 = 0; k0 < p.ks; k0 += 8) {
-      float vals[8][NV];
+    /* partials are read PB at a time (all loads in flight together) and summed in order; fewer at
+     * 32 tokens, where 8 would take 128 registers */
+    constexpr int PB = NV < 16 ? 8 : 4;
+    for (int k0 = 0; k0 < p.ks; k0 += PB) {
+      float vals[PB][NV];
 #pragma unroll
-      for (int kk = 0; kk < 8; ++kk) {
+      for (int kk = 0; kk < PB; ++kk) {
         const int k = k0 + kk < p.ks ? k0 + kk : p.ks - 1;
         const float *pp = p.part + ((size_t)rb_global * p.ks + k) * (NV * 64);
 #pragma unroll
         for (int v = 0; v < NV; ++v) vals[kk][v] = aos_collect(pp + v * 64 + lane);
       }
 #pragma unroll
-      for (int kk = 0; kk < 8; ++kk)
+      for (int kk = 0; kk < PB; ++kk)
         if (k0 + kk < p.ks) {
 #pragma unroll
           for (int v = 0; v < NV; ++v) tot[v] += vals[kk][v];
