@@ -197,7 +197,8 @@ __device__ __forceinline__ uint32_t set_hash(const uint16_t (&ids)[8], uint32_t 
 constexpr int GP_NT = 1024;
 constexpr int GP_HT = 2 * AOS_PREFILL_MAX_T; /* hash table slots (load factor <= 1/2) */
 constexpr int GP_BLK = AOS_PREFILL_MAX_T / 64; /* 64-token blocks: (pass, wave) in token order */
-constexpr int GP_SMALL = 64;                   /* groups ranked with ballots; more fall back to a sort */
+constexpr int GP_BINS = 64;                    /* a digit of the group index: 6 bits */
+static_assert(GP_BLK == 64 && AOS_PREFILL_MAX_T <= GP_BINS * GP_BINS, "a lane per block, two digits");
 constexpr uint32_t GP_EMPTY = 0xffffffffu;
 
 /* Dynamic LDS of the plan kernel. */
@@ -205,49 +206,61 @@ constexpr int GP_OFF_TABH = 0;
 constexpr int GP_OFF_TABF = GP_OFF_TABH + GP_HT * 4;
 constexpr int GP_OFF_BOUND = GP_OFF_TABF + GP_HT * 4;
 constexpr int GP_OFF_BLK = GP_OFF_BOUND + AOS_MAX_ADAPTERS;
-constexpr int GP_OFF_MISC = GP_OFF_BLK + GP_SMALL * GP_BLK * 4;
+constexpr int GP_OFF_MISC = GP_OFF_BLK + GP_BINS * GP_BLK * 4;
 constexpr int GP_LDS = GP_OFF_MISC + (AOS_MAX_ADAPTERS / 32) * 4 + (AOS_MAX_ADAPTERS / 32 + 1) * 4 +
-                       (GP_BLK + GP_SMALL + 2) * 4;
+                       (GP_BLK + GP_BINS + 2) * 4;
 
-/* Compare-exchange of a bitonic network between this lane's key and the key of lane ^ d: the
- * lower lane keeps the smaller key of an ascending pair. */
-__device__ __forceinline__ uint64_t bitonic_lane(uint64_t a, int lane, int d, bool up) {
-  const uint64_t b = aos_shfl64(a, lane ^ d);
-  const bool lower = (lane & d) == 0;
-  const bool take_min = lower == up;
-  return take_min ? (a < b ? a : b) : (a > b ? a : b);
+/* Sum over lanes 0 .. lane. */
+__device__ __forceinline__ uint32_t lane_scan(uint32_t v, int lane) {
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t u = aos_shfl(v, (lane - d) & 63);
+    v += lane >= d ? u : 0u;
+  }
+  return v;
 }
 
-/* Bitonic sort of key[0, NP) in LDS by the workgroup (element i: thread i % GP_NT); stages whose
- * partner lies in the same wave exchange through lane shuffles. */
-__device__ void gp_sort(uint64_t *key, int NP) {
-  const int tid = threadIdx.x, lane = tid & 63;
-  for (int k = 2; k <= NP; k <<= 1) {
-    int j = k >> 1;
-    for (; j >= 64; j >>= 1) {
-      for (int i = tid; i < NP; i += GP_NT) {
-        const int ixj = i ^ j;
-        if (ixj > i) {
-          const uint64_t a = key[i], b = key[ixj];
-          if (((i & k) == 0) ? (a > b) : (a < b)) {
-            key[i] = b;
-            key[ixj] = a;
-          }
-        }
-      }
-      __syncthreads();
+/* Positions of a stable counting sort by a 6-bit digit. Element tid + q GP_NT (block q GP_NT / 64 + wave of
+ * 64 consecutive elements) counts if on[q]; a lane finds the lanes of its block with its digit by one ballot
+ * per bit, the counts per (digit, block) in blk are summed along the blocks by a wave per digit (a lane per
+ * block), the digits' sizes in start by one wave. */
+template <int RPT>
+__device__ __forceinline__ void gp_positions(const bool (&on)[RPT], const uint32_t (&dig)[RPT], uint32_t *blk,
+                                             uint32_t *start, uint32_t (&pos)[RPT]) {
+  constexpr int NB = RPT * (GP_NT / 64); /* blocks */
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint64_t lt = (1ull << lane) - 1ull;
+  for (int e = tid; e < GP_BINS * NB; e += GP_NT) blk[e] = 0u;
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < RPT; ++q) {
+    uint64_t m = __ballot(on[q]);
+#pragma unroll
+    for (int b = 0; b < 6; ++b) {
+      const bool bit = (dig[q] >> b) & 1u;
+      const uint64_t v = __ballot(bit);
+      m &= bit ? v : ~v;
     }
-    for (int i0 = 0; i0 < NP; i0 += GP_NT) {
-      const int i = i0 + tid;
-      if (i < NP) { /* uniform per wave: NP and GP_NT are multiples of 64 */
-        uint64_t v = key[i];
-        const bool up = (i & k) == 0;
-        for (int d = j; d > 0; d >>= 1) v = bitonic_lane(v, lane, d, up);
-        key[i] = v;
-      }
-    }
-    __syncthreads();
+    pos[q] = (uint32_t)__popcll(m & lt);
+    if (on[q] && pos[q] == 0) blk[dig[q] * NB + q * (GP_NT / 64) + wave] = (uint32_t)__popcll(m);
   }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < GP_BINS / (GP_NT / 64); ++k) {
+    const int d = wave + k * (GP_NT / 64);
+    const uint32_t v = lane < NB ? blk[d * NB + lane] : 0u, incl = lane_scan(v, lane);
+    if (lane < NB) blk[d * NB + lane] = incl - v;
+    if (lane == 63) start[d] = incl;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const uint32_t v = start[lane], incl = lane_scan(v, lane);
+    start[lane] = incl - v;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < RPT; ++q)
+    if (on[q]) pos[q] += start[dig[q]] + blk[dig[q] * NB + q * (GP_NT / 64) + wave];
 }
 
 /* One workgroup per tile; every workgroup derives the same order of all the tokens, then writes
@@ -257,28 +270,32 @@ __device__ void gp_sort(uint64_t *key, int NP) {
  * The order: tokens with equal adapter sets (equal set hashes) form a group; groups come in the
  * order of their first token, tokens within a group in index order. Each token finds its group's
  * first token through an LDS hash table (atomicMin per slot); the group index is the count of
- * first tokens before it. With at most GP_SMALL groups a token's position is its group's start
- * plus its rank among the group's tokens before it, counted with one ballot per (group, 64-token
- * block); otherwise the (first token, token) keys are sorted. */
+ * first tokens before it. The order is then a stable counting sort of the tokens by group index: one
+ * pass of 6 bits with at most 64 groups, two above. Latency-bound (one workgroup derives everything), so
+ * every sum over blocks, digits or groups is a scan by a wave: as loops of one thread over LDS, and a
+ * bitonic sort above 64 groups, they took more than half of it (4096 tokens of 32 adapter sets and 1000 of
+ * their own: 78 us, 36 us with the scans). RPT: tokens per thread (straight-line code that runs once: a
+ * prompt of up to 1024 tokens fetches a third of the instructions). */
+template <int RPT>
 __global__ void __launch_bounds__(GP_NT) aos_gplan_kernel(aos_gplan_params p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char gsm[];
   uint32_t *tab_h = (uint32_t *)(gsm + GP_OFF_TABH);
   uint32_t *tab_f = (uint32_t *)(gsm + GP_OFF_TABF);
   uint8_t *bound_s = (uint8_t *)(gsm + GP_OFF_BOUND);
-  uint32_t *blk = (uint32_t *)(gsm + GP_OFF_BLK);               /* [GP_SMALL][GP_BLK] */
+  uint32_t *blk = (uint32_t *)(gsm + GP_OFF_BLK);               /* [GP_BINS][GP_BLK] */
   uint32_t *bits = (uint32_t *)(gsm + GP_OFF_MISC);            /* [AOS_MAX_ADAPTERS / 32] */
   int *base = (int *)(bits + AOS_MAX_ADAPTERS / 32);           /* [.. + 1] */
   uint32_t *wsum = (uint32_t *)(base + AOS_MAX_ADAPTERS / 32 + 1); /* [GP_BLK] */
-  uint32_t *gstart = wsum + GP_BLK;                            /* [GP_SMALL + 1] */
-  uint32_t *ngroups = gstart + GP_SMALL + 1;
+  uint32_t *gstart = wsum + GP_BLK;                            /* [GP_BINS] */
+  uint32_t *ngroups = gstart + GP_BINS + 1;
+  constexpr int HT = 2 * RPT * GP_NT; /* hash table slots used (of GP_HT; load factor <= 1/2) */
+  static_assert(RPT == 1 || RPT == 2 || (RPT == 4 && HT == GP_HT), "hash bits");
   uint16_t *tperm = (uint16_t *)tab_h; /* sorted position -> token, once the table is done */
-  uint64_t *key = (uint64_t *)tab_h;   /* sort keys of the fallback, likewise */
-  constexpr int RPT = AOS_PREFILL_MAX_T / GP_NT;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, T = p.T, n = p.n;
   const uint64_t lt = (1ull << lane) - 1ull;
 
   for (int a = tid; a < n; a += GP_NT) bound_s[a] = p.bound[a];
-  for (int e = tid; e < GP_HT; e += GP_NT) {
+  for (int e = tid; e < HT; e += GP_NT) {
     tab_h[e] = GP_EMPTY;
     tab_f[e] = GP_EMPTY;
   }
@@ -301,13 +318,16 @@ __global__ void __launch_bounds__(GP_NT) aos_gplan_kernel(aos_gplan_params p) {
       uint16_t ids[8];
       uint32_t h = set_hash(ids, ring_set(rw[q], n, bound_s, ids));
       h = h == GP_EMPTY ? GP_EMPTY - 1u : h;
-      uint32_t sl = (h * 0x9E3779B1u) >> 19; /* 13 bits: GP_HT slots */
+      uint32_t sl = (h * 0x9E3779B1u) >> (RPT == 1 ? 21 : RPT == 2 ? 20 : 19); /* HT slots */
       for (;;) {
-        const uint32_t old = atomicCAS(&tab_h[sl], GP_EMPTY, h);
+        /* a token whose set is there already only reads: the lanes of one set would queue on its slot */
+        uint32_t old = __hip_atomic_load(&tab_h[sl], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (old == GP_EMPTY) old = atomicCAS(&tab_h[sl], GP_EMPTY, h);
         if (old == GP_EMPTY || old == h) break;
-        sl = (sl + 1) & (GP_HT - 1);
+        sl = (sl + 1) & (HT - 1);
       }
-      atomicMin(&tab_f[sl], (uint32_t)t);
+      if (__hip_atomic_load(&tab_f[sl], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) > (uint32_t)t)
+        atomicMin(&tab_f[sl], (uint32_t)t);
       slot[q] = sl;
     }
   }
@@ -324,14 +344,10 @@ __global__ void __launch_bounds__(GP_NT) aos_gplan_kernel(aos_gplan_params p) {
     if (lane == 0) wsum[q * (GP_NT / 64) + wave] = (uint32_t)__popcll(fb[q]);
   }
   __syncthreads();
-  if (tid == 0) {
-    uint32_t acc = 0;
-    for (int b = 0; b < GP_BLK; ++b) {
-      const uint32_t v = wsum[b];
-      wsum[b] = acc;
-      acc += v;
-    }
-    *ngroups = acc;
+  if (wave == 0) {
+    const uint32_t v = lane < RPT * (GP_NT / 64) ? wsum[lane] : 0u, incl = lane_scan(v, lane);
+    wsum[lane] = incl - v;
+    if (lane == 63) *ngroups = incl;
   }
   __syncthreads();
   const uint32_t D = *ngroups;
@@ -346,57 +362,34 @@ __global__ void __launch_bounds__(GP_NT) aos_gplan_kernel(aos_gplan_params p) {
   for (int q = 0; q < RPT; ++q) gid[q] = tid + q * GP_NT < T ? tab_f[slot[q]] : GP_EMPTY;
   __syncthreads(); /* the table is no longer read: its memory takes the order */
 
-  if (D <= (uint32_t)GP_SMALL) {
-    uint32_t rank[RPT];
+  {
+    bool on[RPT];
+    uint32_t dig[RPT], pos[RPT];
 #pragma unroll
-    for (int q = 0; q < RPT; ++q) rank[q] = 0;
-    for (uint32_t g = 0; g < D; ++g) {
+    for (int q = 0; q < RPT; ++q) {
+      on[q] = tid + q * GP_NT < T;
+      dig[q] = gid[q] & (GP_BINS - 1);
+    }
+    gp_positions(on, dig, blk, gstart, pos);
+    if (D <= (uint32_t)GP_BINS) {
+#pragma unroll
+      for (int q = 0; q < RPT; ++q)
+        if (on[q]) tperm[pos[q]] = (uint16_t)(tid + q * GP_NT);
+    } else { /* by the low digit into tab_f, then by the high digit */
+#pragma unroll
+      for (int q = 0; q < RPT; ++q)
+        if (on[q]) tab_f[pos[q]] = (gid[q] << 16) | (uint32_t)(tid + q * GP_NT);
+      __syncthreads();
+      uint32_t e[RPT];
 #pragma unroll
       for (int q = 0; q < RPT; ++q) {
-        const uint64_t b = __ballot(gid[q] == g);
-        if (lane == 0) blk[g * GP_BLK + q * (GP_NT / 64) + wave] = (uint32_t)__popcll(b);
-        if (gid[q] == g) rank[q] = (uint32_t)__popcll(b & lt);
+        e[q] = on[q] ? tab_f[tid + q * GP_NT] : 0u;
+        dig[q] = e[q] >> 22;
       }
-    }
-    __syncthreads();
-    if (tid < (int)D) { /* block prefix within group tid, and its size */
-      uint32_t acc = 0;
-      for (int b = 0; b < GP_BLK; ++b) {
-        const uint32_t v = blk[tid * GP_BLK + b];
-        blk[tid * GP_BLK + b] = acc;
-        acc += v;
-      }
-      gstart[tid + 1] = acc;
-    }
-    __syncthreads();
-    if (tid == 0) {
-      gstart[0] = 0;
-      for (uint32_t g = 1; g <= D; ++g) gstart[g] += gstart[g - 1];
-    }
-    __syncthreads();
+      gp_positions(on, dig, blk, gstart, pos);
 #pragma unroll
-    for (int q = 0; q < RPT; ++q) {
-      const int t = tid + q * GP_NT;
-      if (t < T) tperm[gstart[gid[q]] + blk[gid[q] * GP_BLK + q * (GP_NT / 64) + wave] + rank[q]] = (uint16_t)t;
-    }
-  } else {
-    int NP = 64;
-    while (NP < T) NP <<= 1;
-#pragma unroll
-    for (int q = 0; q < RPT; ++q) {
-      const int t = tid + q * GP_NT;
-      if (t < NP) key[t] = t < T ? ((uint64_t)first[q] << 32) | (uint32_t)t : ~0ull;
-    }
-    __syncthreads();
-    gp_sort(key, NP);
-    /* keys -> tokens in place, a pass of GP_NT at a time: pass j writes bytes 2 i of tperm, which
-     * hold keys below (j + 1) * GP_NT / 4, all read by passes up to j */
-    for (int j = 0; j * GP_NT < T; ++j) {
-      const int i = j * GP_NT + tid;
-      const uint16_t t = i < T ? (uint16_t)(uint32_t)key[i] : 0;
-      __syncthreads();
-      if (i < T) tperm[i] = t;
-      __syncthreads();
+      for (int q = 0; q < RPT; ++q)
+        if (on[q]) tperm[pos[q]] = (uint16_t)e[q];
     }
   }
   __syncthreads();
@@ -437,12 +430,19 @@ __global__ void __launch_bounds__(GP_NT) aos_gplan_kernel(aos_gplan_params p) {
     if ((m >> (a & 31)) & 1u) {
       const int u = base[a >> 5] + __builtin_popcount(m & ((1u << (a & 31)) - 1u));
       p.list[trow + u] = (uint16_t)a;
-      for (int k = 0; k < p.nmod; ++k) {
-        const aos_lora_tab &tb = p.tab[k];
-        const bool has = tb.rpad && a < tb.n;
-        p.ap[(size_t)k * mtiles * p.tu_cap + trow + u] = has ? tb.A[a] : nullptr;
-        p.bp[(size_t)k * mtiles * p.tu_cap + trow + u] = has ? tb.Bf[a] : nullptr;
+      const uint16_t *pa[3], *pb[3]; /* loaded together, then stored */
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const bool has = k < p.nmod && p.tab[k].rpad && a < p.tab[k].n;
+        pa[k] = has ? aos_gld_ptr(&p.tab[k].A[a]) : nullptr;
+        pb[k] = has ? aos_gld_ptr(&p.tab[k].Bf[a]) : nullptr;
       }
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        if (k < p.nmod) {
+          p.ap[(size_t)k * mtiles * p.tu_cap + trow + u] = pa[k];
+          p.bp[(size_t)k * mtiles * p.tu_cap + trow + u] = pb[k];
+        }
     }
   }
   /* coefficient rows of the tile: each token's (slot, coefficient) pairs by one thread, summed in
@@ -2265,7 +2265,9 @@ extern "C" int aos_launch_gplan(const aos_gplan_params *p, const aos_launch_ctx 
     return (int)hipErrorInvalidValue;
   const int ucap = p->n < AOS_TILE_U_MAX ? p->n : AOS_TILE_U_MAX;
   if (p->tu_cap < ucap || p->tu_cap < 1) return (int)hipErrorInvalidValue;
-  AOS_LAUNCH(ctx, aos_gplan_kernel, dim3(mtiles), dim3(GP_NT), GP_LDS, *p);
+  if (p->T <= GP_NT) AOS_LAUNCH(ctx, aos_gplan_kernel<1>, dim3(mtiles), dim3(GP_NT), GP_LDS, *p);
+  else if (p->T <= 2 * GP_NT) AOS_LAUNCH(ctx, aos_gplan_kernel<2>, dim3(mtiles), dim3(GP_NT), GP_LDS, *p);
+  else AOS_LAUNCH(ctx, aos_gplan_kernel<AOS_PREFILL_MAX_T / GP_NT>, dim3(mtiles), dim3(GP_NT), GP_LDS, *p);
   return (int)hipGetLastError();
 }
 

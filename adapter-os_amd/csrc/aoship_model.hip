@@ -129,48 +129,57 @@ __global__ void __launch_bounds__(1024) aos_norm_kernel(aos_norm_params p) {
 /* A bfloat16 infinity or NaN. */
 __device__ __forceinline__ bool bf16_nonfinite(uint32_t b) { return (b & 0x7f80u) == 0x7f80u; }
 
-/* One thread per rotated pair of q or k, or per element of v. */
+/* Workgroup (part, token): items w = 256 part + thread, then every gridDim.x * 256 further; an item is a
+ * rotated pair of q or k, or an element of v. The token's cosines and sines are formed once per workgroup
+ * in LDS: one per item, the same angle's for every head, they took three quarters of the launch (1900
+ * tokens of 28 + 4 heads of 128: 32 us). */
 __global__ void __launch_bounds__(256) aos_rope_kernel(aos_rope_params p) {
+  __shared__ float cs[AOS_ATTN_MAX_HD / 2], sn[AOS_ATTN_MAX_HD / 2];
   const int t = blockIdx.y, half = p.hd / 2;
   const int pos = p.offset + t;
   const float fpos = (float)pos;
   const int nq = p.nh * half, nk = p.nkv * half, nv = p.nkv * p.hd;
-  const int w = blockIdx.x * 256 + threadIdx.x;
-  if (w >= nq + nk + nv) return;
-  if (w < nq + nk) {
-    const bool isq = w < nq;
-    const int idx = isq ? w : w - nq;
-    const int h = idx / half, i = idx - h * half;
-    const int width = (isq ? p.nh : p.nkv) * p.hd;
-    const uint16_t *src = (isq ? p.q : p.k) + (size_t)t * width + (size_t)h * p.hd;
-    const float *bias = isq ? p.bq : p.bk;
-    float x1 = aos_bf16_to_f32(src[i]), x2 = aos_bf16_to_f32(src[i + half]);
-    if (bias) {
-      x1 = x1 + bias[h * p.hd + i];
-      x2 = x2 + bias[h * p.hd + i + half];
-    }
+  for (int i = threadIdx.x; i < half; i += 256) {
     const float ang = fpos * p.inv_freq[i];
-    const float c = cosf(ang), s = sinf(ang);
-    const float r1 = x1 * c - x2 * s, r2 = x1 * s + x2 * c;
-    if (isq) {
-      float *dst = p.qr + ((size_t)t * p.nh + h) * p.hd;
-      dst[i] = r1;
-      dst[i + half] = r2;
+    cs[i] = cosf(ang);
+    sn[i] = sinf(ang);
+  }
+  __syncthreads();
+  for (int w = blockIdx.x * 256 + threadIdx.x; w < nq + nk + nv; w += gridDim.x * 256) {
+    if (w < nq + nk) {
+      const bool isq = w < nq;
+      const int idx = isq ? w : w - nq;
+      const int h = idx / half, i = idx - h * half;
+      const int width = (isq ? p.nh : p.nkv) * p.hd;
+      const uint16_t *src = (isq ? p.q : p.k) + (size_t)t * width + (size_t)h * p.hd;
+      const float *bias = isq ? p.bq : p.bk;
+      float x1 = aos_bf16_to_f32(src[i]), x2 = aos_bf16_to_f32(src[i + half]);
+      if (bias) {
+        x1 = x1 + bias[h * p.hd + i];
+        x2 = x2 + bias[h * p.hd + i + half];
+      }
+      const float c = cs[i], s = sn[i];
+      const float r1 = x1 * c - x2 * s, r2 = x1 * s + x2 * c;
+      if (isq) {
+        float *dst = p.qr + ((size_t)t * p.nh + h) * p.hd;
+        dst[i] = r1;
+        dst[i + half] = r2;
+      } else {
+        uint16_t *dst = p.kc + ((size_t)h * p.max_seq + pos) * p.hd;
+        const uint16_t b1 = aos_f32_to_bf16(r1), b2 = aos_f32_to_bf16(r2);
+        dst[i] = b1;
+        dst[i + half] = b2;
+        if (bf16_nonfinite(b1) || bf16_nonfinite(b2)) *p.nonfinite = 1u;
+      }
     } else {
-      uint16_t *dst = p.kc + ((size_t)h * p.max_seq + pos) * p.hd;
-      const uint16_t b1 = aos_f32_to_bf16(r1), b2 = aos_f32_to_bf16(r2);
-      dst[i] = b1;
-      dst[i + half] = b2;
-      if (bf16_nonfinite(b1) || bf16_nonfinite(b2)) *p.nonfinite = 1u;
+      const int idx = w - nq - nk;
+      const int h = idx / p.hd, d = idx - h * p.hd;
+      float v = aos_bf16_to_f32(p.v[(size_t)t * nv + idx]);
+      if (p.bv) v = v + p.bv[idx];
+      const uint16_t b = aos_f32_to_bf16(v);
+      p.vc[((size_t)h * p.max_seq + pos) * p.hd + d] = b;
+      if (bf16_nonfinite(b)) *p.nonfinite = 1u;
     }
-  } else {
-    const int idx = w - nq - nk;
-    const int h = idx / p.hd, d = idx - h * p.hd;
-    float v = aos_bf16_to_f32(p.v[(size_t)t * nv + idx]);
-    if (p.bv) v = v + p.bv[idx];
-    const uint16_t b = aos_f32_to_bf16(v);
-    p.vc[((size_t)h * p.max_seq + pos) * p.hd + d] = b;
-    if (bf16_nonfinite(b)) *p.nonfinite = 1u;
   }
 }
 
@@ -810,9 +819,12 @@ extern "C" int aos_launch_norm(const aos_norm_params *p, const aos_launch_ctx *c
 }
 
 extern "C" int aos_launch_rope(const aos_rope_params *p, const aos_launch_ctx *ctx) {
-  if (!p->nonfinite) return (int)hipErrorInvalidValue;
+  if (!p->nonfinite || p->hd > AOS_ATTN_MAX_HD) return (int)hipErrorInvalidValue;
   const int items = p->nh * (p->hd / 2) + p->nkv * (p->hd / 2) + p->nkv * p->hd;
-  AOS_LAUNCH(ctx, aos_rope_kernel, dim3((items + 255) / 256, p->T), dim3(256), 0, *p);
+  /* parts of a token: as many as about 1024 workgroups allow (few tokens), so that none loops long */
+  int parts = p->T < 1024 ? 1024 / p->T : 1;
+  if (parts > (items + 255) / 256) parts = (items + 255) / 256;
+  AOS_LAUNCH(ctx, aos_rope_kernel, dim3(parts, p->T), dim3(256), 0, *p);
   return (int)hipGetLastError();
 }
 

@@ -28,14 +28,14 @@ def _q4(rng, out, inp):
     return packed, scale, bias, dense
 
 
-def _build(hip, rng, shapes, n, rank):
+def _build(hip, rng, shapes, n, rank, bscale=0.05):
     layer, base, lora = hip.Layer(0), {}, {}
     ads = [hip.LoraAdapter(i, 1, 1.0) for i in range(n)]
     for m, (out, inp) in shapes.items():
         packed, scale, bias, base[m] = _q4(rng, out, inp)
         layer.set_base(m, packed, scale, bias)
         a = _bf16(rng.standard_normal((n, rank, inp)) * inp**-0.5).float().numpy()
-        b = _bf16(rng.standard_normal((n, out, rank)) * 0.05).float().numpy()
+        b = _bf16(rng.standard_normal((n, out, rank)) * bscale).float().numpy()
         lora[m] = (a.astype(np.float64), b.astype(np.float64))
         for i, ad in enumerate(ads):
             ad.set_module(0, m, a[i], b[i])
