@@ -131,8 +131,8 @@ __device__ __forceinline__ bool bf16_nonfinite(uint32_t b) { return (b & 0x7f80u
 
 /* Workgroup (part, token): items w = 256 part + thread, then every gridDim.x * 256 further; an item is a
  * rotated pair of q or k, or an element of v. The token's cosines and sines are formed once per workgroup
- * in LDS: one per item, the same angle's for every head, they took three quarters of the launch (1900
- * tokens of 28 + 4 heads of 128: 32 us). */
+ * in LDS: formed per item, the same angle's for every head, they made the launch arithmetic-bound (1900
+ * tokens of 28 + 4 heads of 128: 32 us, now 17). */
 __global__ void __launch_bounds__(256) aos_rope_kernel(aos_rope_params p) {
   __shared__ float cs[AOS_ATTN_MAX_HD / 2], sn[AOS_ATTN_MAX_HD / 2];
   const int t = blockIdx.y, half = p.hd / 2;
