@@ -144,6 +144,9 @@ def lib():
         L.aoship_internal_layer_last_adapter_major.argtypes = [_P]
         L.aoship_internal_layer_last_perm.restype = C.c_int
         L.aoship_internal_layer_last_perm.argtypes = [_P, _P, C.c_int]
+        L.aoship_internal_model_workspace.restype = C.c_int
+        L.aoship_internal_model_workspace.argtypes = [C.POINTER(ModelConfig), C.c_int, C.POINTER(C.c_size_t),
+                                                      C.POINTER(C.c_size_t)]
         L.aoship_internal_decode_geometry.restype = C.c_int
         L.aoship_internal_decode_geometry.argtypes = [C.c_int, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int),
                                                       C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int)]
@@ -168,6 +171,15 @@ def decode_geometry(kind: int, out: int, inp: int, T: int, wr_pin: int = 0, ks_p
                                                         C.byref(r), C.byref(g)),
            "aoship_internal_decode_geometry")
     return w.value, k.value, r.value, g.value
+
+
+def model_workspace(cfg: ModelConfig, T: int) -> tuple[int, int]:
+    """(bytes of a model's per-call buffers for calls of up to T tokens, floats of them for the attention
+    splits' partials): see aoship_internal_model_workspace."""
+    b, p = C.c_size_t(), C.c_size_t()
+    _check(lib().aoship_internal_model_workspace(C.byref(cfg), T, C.byref(b), C.byref(p)),
+           "aoship_internal_model_workspace")
+    return b.value, p.value
 
 
 SPIN_LIMIT_DEFAULT = 1 << 24

@@ -3089,11 +3089,19 @@ extern "C" int aoship_model_cache_len(const aoship_model_t *m) { return m ? m->c
 
 /* per-call buffers: hidden f32, normed / q / k / v / attention / y bf16, rotated q f32, the
  * attention splits' partials */
-static int attn_splits(const aoship_model *m, int T, int visible_max) {
+static int attn_splits(const aoship_model_config_t &c, int T, int visible_max) {
   const int chunks = ceil_div(visible_max, 64);
-  int s = ceil_div(1024, m->cfg.num_heads * T);
+  int s = ceil_div(1024, c.num_heads * T);
   if (s > chunks) s = chunks;
   return s < 1 ? 1 : s;
+}
+
+/* Rows of split partials that a call of T tokens can need: T * heads * attn_splits is at most 1023 above
+ * T * heads, and at most T * heads * the cache's chunks. Both bounds grow with T where the product itself does
+ * not (28 heads: 1 split at 37 tokens, 2 at 36), so a buffer sized for T tokens serves every smaller call. */
+static size_t attn_part_rows(const aoship_model_config_t &c, int T) {
+  const size_t rows = (size_t)T * c.num_heads;
+  return std::min(rows + 1023, rows * (size_t)ceil_div(c.max_seq, 64));
 }
 
 /* Prompts take the matrix-core attention from AOS_ATTN_PREFILL_ROWS (token, head) rows on: below, its
@@ -3111,14 +3119,13 @@ struct ModelWs {
   size_t bytes;
 };
 
-static ModelWs model_ws(const aoship_model *m, int T, void *base) {
-  const aoship_model_config_t &c = m->cfg;
-  const int splits = attn_splits(m, T, c.max_seq);
+/* (every part, so the whole too, grows with T: see attn_part_rows) */
+static ModelWs model_ws(const aoship_model_config_t &c, int T, void *base) {
   Bump b(base, 0);
   ModelWs w;
   w.hidden = b.take<float>((size_t)T * c.hidden);
   w.qr = b.take<float>((size_t)T * c.num_heads * c.head_dim);
-  w.part = b.take<float>((size_t)T * c.num_heads * splits * (c.head_dim + 2));
+  w.part = b.take<float>(attn_part_rows(c, T) * (size_t)(c.head_dim + 2));
   w.normed = b.take<uint16_t>((size_t)T * c.hidden);
   w.q = b.take<uint16_t>((size_t)T * c.num_heads * c.head_dim);
   w.k = b.take<uint16_t>((size_t)T * c.num_kv_heads * c.head_dim);
@@ -3129,13 +3136,25 @@ static ModelWs model_ws(const aoship_model *m, int T, void *base) {
   return w;
 }
 
+/* Diagnostic (no counterpart in the reference): the bytes of the per-call buffers that a model of this
+ * shape holds for calls of up to T tokens, and the floats of them for the attention splits' partials. */
+extern "C" int aoship_internal_model_workspace(const aoship_model_config_t *c, int T, size_t *bytes,
+                                               size_t *part_floats) {
+  if (!c || T < 1 || T > c->max_seq || c->num_heads < 1 || c->max_seq < 1 || !bytes || !part_floats)
+    return set_err("aoship_internal_model_workspace: bad arguments");
+  *bytes = model_ws(*c, T, nullptr).bytes;
+  *part_floats = attn_part_rows(*c, T) * (size_t)(c->head_dim + 2);
+  return 0;
+}
+
 extern "C" int aoship_model_reserve(aoship_model_t *m, int max_tokens) {
   if (!m || max_tokens < 1) return set_err("aoship_model_reserve: bad arguments");
   if (ensure_device()) return -1;
   for (auto *l : m->layers)
     if (aoship_layer_reserve(l, max_tokens)) return -1;
   if (max_tokens > m->ws_T) {
-    if (m->ws.alloc(model_ws(m, max_tokens, nullptr).bytes, false) ||
+    m->ws_T = 0; /* nothing fits should an allocation fail */
+    if (m->ws.alloc(model_ws(m->cfg, max_tokens, nullptr).bytes, false) ||
         m->attn_ctr.alloc((size_t)max_tokens * m->cfg.num_heads * 4, true))
       return -1;
     m->ws_T = max_tokens;
@@ -3158,11 +3177,12 @@ extern "C" int aoship_model_forward(aoship_model_t *m, const int32_t *ids, int T
     if (check_no_timeout(l)) return -1;
   if (ensure_device()) return -1;
   if (T > m->ws_T) {
-    const size_t bytes = model_ws(m, T, nullptr).bytes;
+    const size_t bytes = model_ws(c, T, nullptr).bytes;
+    m->ws_T = 0;
     if (m->ws.alloc(bytes, false) || m->attn_ctr.alloc((size_t)T * c.num_heads * 4, true)) return -1;
     m->ws_T = T;
   }
-  const ModelWs w = model_ws(m, T, m->ws.p);
+  const ModelWs w = model_ws(c, T, m->ws.p);
   aos_launch_ctx ctx = {m->stream, nullptr, nullptr};
   const int hd = c.head_dim, nh = c.num_heads, nkv = c.num_kv_heads;
 
@@ -3228,7 +3248,7 @@ extern "C" int aoship_model_forward(aoship_model_t *m, const int32_t *ids, int T
     ap.hd = hd;
     ap.offset = position_offset;
     ap.max_seq = c.max_seq;
-    ap.splits = attn_splits(m, T, position_offset + T);
+    ap.splits = attn_splits(c, T, position_offset + T);
     ap.chunk = ceil_div(ceil_div(position_offset + T, ap.splits), 64) * 64;
     ap.scale = 1.0f / std::sqrt((float)hd);
     ap.part = w.part;
