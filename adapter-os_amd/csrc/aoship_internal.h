@@ -622,7 +622,8 @@ typedef struct {
   const uint16_t *qb, *kb, *vb;
   const float *bq, *bk, *bv;
   const float *inv_freq;
-  /* set to 1 (rope_fused) when an infinity or NaN enters the cache; the prompt kernel reads it */
+  /* set to 1 (rope_fused) when an infinity or NaN enters the cache; set, the prompt kernel runs
+   * as the wave per (token, head) */
   uint32_t *nonfinite;
   int prefill; /* 1: the prompt kernel (head_dim 64 or 128, rotated queries, no splits) */
 } aos_attn_params;
