@@ -144,6 +144,8 @@ def lib():
         L.aoship_internal_layer_last_adapter_major.argtypes = [_P]
         L.aoship_internal_layer_last_perm.restype = C.c_int
         L.aoship_internal_layer_last_perm.argtypes = [_P, _P, C.c_int]
+        L.aoship_internal_route_tokens.restype = C.c_int
+        L.aoship_internal_route_tokens.argtypes = [C.c_int, C.c_int, C.c_int]
         L.aoship_internal_model_workspace.restype = C.c_int
         L.aoship_internal_model_workspace.argtypes = [C.POINTER(ModelConfig), C.c_int, C.POINTER(C.c_size_t),
                                                       C.POINTER(C.c_size_t)]
@@ -171,6 +173,11 @@ def decode_geometry(kind: int, out: int, inp: int, T: int, wr_pin: int = 0, ks_p
                                                         C.byref(r), C.byref(g)),
            "aoship_internal_decode_geometry")
     return w.value, k.value, r.value, g.value
+
+
+def route_tokens(T: int, n: int, d: int) -> int:
+    """Tokens per workgroup of a plain Router.route_features call (see aoship_internal_route_tokens)."""
+    return lib().aoship_internal_route_tokens(T, n, d)
 
 
 def model_workspace(cfg: ModelConfig, T: int) -> tuple[int, int]:

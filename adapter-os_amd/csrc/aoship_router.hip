@@ -354,25 +354,42 @@ static int launch_route_tokens(const aos_route_params *p, const aos_launch_ctx *
   return (int)hipGetLastError();
 }
 
-/* Tokens per workgroup of a plain router call from features: the fewest that give each CU at most
- * one workgroup, up to 8; one token each (aos_route_features_kernel) while the tokens do not outnumber
+/* Tokens per workgroup of a plain router call from features: the fewest that give each CU (MI355X's 256) at
+ * most one workgroup, up to 8; one token each (aos_route_features_kernel) while the tokens do not outnumber
  * the CUs. A second round costs as much as the first, more than wider workgroups do (64 adapters of
  * 5120 features: one round of 2 / 4 / 8 tokens 21 / 23 / 31 us, two rounds of 4 tokens 40 us). Before,
  * with one token a workgroup: 384 tokens 46 us, 768 68 us, 2039 178 us; now 21, 23 and 33 us. The
- * priors of the tokens must fit beside 32 KB of stages. */
+ * priors of the tokens must fit beside 32 KB of stages.
+ * A few adapters stay with one token each: most of a wide workgroup's 16 waves then hold no adapter, and its
+ * chain of stages is as long as with 16 (5120 features, 2 adapters: 1100 tokens 12.3 us wide, 10.1 us with one
+ * token each; 3584 features, 4 adapters: 600 tokens 8.8 and 8.2 us), as long as the waves (one per adapter and
+ * token) are few per CU (4 adapters of 3584 features: 800 tokens, 12 waves a CU, level; 3 adapters: 1100 tokens,
+ * where the wide workgroups hold 8 tokens, 13 waves a CU, 10.6 and 9.4 us, 1500 tokens 10.8 and 11.0 us), each
+ * adapter has a long row (2 adapters: at 2048 features level, at 896 7.6 and 8.0 us), and the workgroups are
+ * resident at once with a token's features in LDS (1 adapter of 5120 features: 7 a CU, 2039 tokens 15.8 and
+ * 24.4 us). */
 #define AOS_ROUTE_CUS 256
-static int route_tokens(const aos_route_params *p) {
+#define AOS_ROUTE_ONE_WAVES 10  /* per CU, at most, for a few adapters with one token each */
+#define AOS_ROUTE_ONE_WAVES8 13 /* ... against workgroups of 8 tokens */
+#define AOS_ROUTE_ONE_D 800     /* ... and their features per adapter, at least */
+static int route_tokens(int T, int n, int d) {
+  const long one_wgs = (long)AOS_ROUTE_CUS * ((160 * 1024) / ((size_t)(d + n) * sizeof(float)));
+  const long waves = (T > 4 * AOS_ROUTE_CUS ? AOS_ROUTE_ONE_WAVES8 : AOS_ROUTE_ONE_WAVES) * AOS_ROUTE_CUS;
+  if ((long)T * n <= waves && d >= AOS_ROUTE_ONE_D * n && T <= one_wgs) return 1;
   int tt = 1;
-  while (tt < 8 && p->T > tt * AOS_ROUTE_CUS) tt <<= 1;
-  while (tt > 1 && (size_t)tt * p->n * sizeof(float) > 16 * 1024) tt >>= 1;
+  while (tt < 8 && T > tt * AOS_ROUTE_CUS) tt <<= 1;
+  while (tt > 1 && (size_t)tt * n * sizeof(float) > 16 * 1024) tt >>= 1;
   return tt;
 }
+
+/* Diagnostic (no counterpart in the reference): tokens per workgroup of a plain router call. */
+extern "C" int aoship_internal_route_tokens(int T, int n, int d) { return route_tokens(T, n, d); }
 
 extern "C" int aos_launch_route(const aos_route_params *p, const aos_launch_ctx *ctx) {
   const bool x =
       p->scope || p->tie_key || p->post_allowed || p->active_ids || p->strengths || p->hashes || p->decisions;
   if (p->features) {
-    const int tt = x ? 1 : route_tokens(p);
+    const int tt = x ? 1 : route_tokens(p->T, p->n, p->d);
     if (tt == 8) return launch_route_tokens<8>(p, ctx);
     if (tt == 4) return launch_route_tokens<4>(p, ctx);
     if (tt == 2) return launch_route_tokens<2>(p, ctx);
