@@ -150,10 +150,7 @@ def lib():
         L.aoship_internal_model_workspace.argtypes = [C.POINTER(ModelConfig), C.c_int, C.POINTER(C.c_size_t),
                                                       C.POINTER(C.c_size_t)]
         L.aoship_internal_decode_geometry.restype = C.c_int
-        L.aoship_internal_decode_geometry.argtypes = [C.c_int, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int),
-                                                      C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int)]
-        L.aoship_internal_decode_geometry_pinned.restype = C.c_int
-        L.aoship_internal_decode_geometry_pinned.argtypes = [C.c_int] * 6 + [C.POINTER(C.c_int)] * 4
+        L.aoship_internal_decode_geometry.argtypes = [C.c_int] * 8 + [C.POINTER(C.c_int)] * 5
         L.aoship_internal_layer_set_gemv_geometry.restype = C.c_int
         L.aoship_internal_layer_set_gemv_geometry.argtypes = [_P, C.c_int, C.c_int, C.c_int]
         L.aoship_internal_layer_set_mlp1.restype = C.c_int
@@ -164,15 +161,22 @@ def lib():
     return _lib
 
 
-def decode_geometry(kind: int, out: int, inp: int, T: int, wr_pin: int = 0, ks_pin: int = 0) -> tuple[int, int, int, int]:
-    """(waves, K splits, row blocks per workgroup, fewest K groups of any wave) of a decode launch
-    shape (see aoship_internal_decode_geometry), optionally with a GEMV shape pinned as
-    Layer.set_gemv_geometry pins it."""
-    w, k, r, g = C.c_int(), C.c_int(), C.c_int(), C.c_int()
-    _check(lib().aoship_internal_decode_geometry_pinned(kind, out, inp, T, wr_pin, ks_pin, C.byref(w), C.byref(k),
-                                                        C.byref(r), C.byref(g)),
+def decode_launch(kind: int, out: int, inp: int, T: int, wr_pin: int = 0, ks_pin: int = 0, n: int = 0,
+                  rpad: int = 0) -> tuple[bool, int, int, int, int]:
+    """(whether the waves read x themselves, then decode_geometry's values) of a decode launch over a table of
+    n adapters of padded rank rpad (see aoship_internal_decode_geometry)."""
+    d, w, k, r, g = (C.c_int() for _ in range(5))
+    _check(lib().aoship_internal_decode_geometry(kind, out, inp, T, n, rpad, wr_pin, ks_pin, C.byref(d), C.byref(w),
+                                                 C.byref(k), C.byref(r), C.byref(g)),
            "aoship_internal_decode_geometry")
-    return w.value, k.value, r.value, g.value
+    return bool(d.value), w.value, k.value, r.value, g.value
+
+
+def decode_geometry(kind: int, out: int, inp: int, T: int, wr_pin: int = 0, ks_pin: int = 0, n: int = 0,
+                    rpad: int = 0) -> tuple[int, int, int, int]:
+    """(waves, K splits, row blocks per workgroup, fewest K groups of any wave) of a decode launch
+    shape, optionally with a GEMV shape pinned as Layer.set_gemv_geometry pins it."""
+    return decode_launch(kind, out, inp, T, wr_pin, ks_pin, n, rpad)[1:]
 
 
 def route_tokens(T: int, n: int, d: int) -> int:

@@ -1240,7 +1240,9 @@ static int gemv_splits(int RB, int G, int T, int W, int waves_target) {
  * reduction's LDS. */
 static size_t gemv_lds_x(int T, int G, int ks) { return 128 + (size_t)T * ceil_div(G, ks) * 136; }
 
-/* Row-split geometry (3 or more tokens): the waves of a workgroup take different row blocks over
+/* Row-split geometry (3 or more tokens with x staged: a gate/up launch of at most 8 tokens over a wide adapter
+ * table, fewer than AOS_GEMV_DX_MIN_G K groups, and pinned shapes; the 8-wave rule serves pinned shapes
+ * alone): the waves of a workgroup take different row blocks over
  * one K split, so the x slice staged in LDS serves WR row blocks instead of one (x staged over a
  * whole launch scales with RB / WR). The rules below are the best of sweeps over (WR, ks) on
  * MI355X (the 7B MLP at 4, 8 and 32 tokens, the 3B projections at 32): the fewest K splits that
@@ -1307,8 +1309,17 @@ static void gemv_geometry_rows(int RB, int G, int T, bool swiglu, int W, aos_gem
 #define AOS_GEMV_DX_WAVES 1024
 #define AOS_GEMV_DX_WAVES_PROJ 512
 #define AOS_GEMV_DX_GU_COLS 1024 /* a module's columns over the whole table, up to which 3-8 tokens read x directly */
-static bool gemv_direct(int G, int T, int wr_force, int ks_force) {
-  return T >= AOS_GEMV_DX_MIN_T && G >= AOS_GEMV_DX_MIN_G && wr_force <= 0 && ks_force <= 0;
+
+/* The decode GEMV launches, as the diagnostics number them. */
+enum { GV_GATE_UP = 0, GV_DOWN = 1, GV_PROJ = 2 };
+
+/* Waves of a decode GEMV launch that reads x itself, 0 for one that stages x in LDS. n, rpad: the adapter
+ * table's size and the widest padded rank of the launch's modules; wr_force, ks_force: a pinned (staged)
+ * shape. */
+static int gemv_direct_waves(int kind, int G, int T, int n, int rpad, int wr_force, int ks_force) {
+  if (T < AOS_GEMV_DX_MIN_T || G < AOS_GEMV_DX_MIN_G || wr_force > 0 || ks_force > 0) return 0;
+  if (kind == GV_GATE_UP && T <= 8 && n * rpad > AOS_GEMV_DX_GU_COLS) return 0;
+  return kind == GV_PROJ ? AOS_GEMV_DX_WAVES_PROJ : AOS_GEMV_DX_WAVES;
 }
 
 static void gemv_geometry_direct(int RB, int G, int T, bool swiglu, bool lora, aos_gemv_params &g, int waves) {
@@ -1328,11 +1339,7 @@ static void gemv_geometry_direct(int RB, int G, int T, bool swiglu, bool lora, a
  * From 3 tokens on, the row-split geometry above. */
 static void gemv_geometry(int RB, int G, int T, bool swiglu, bool lora, aos_gemv_params &g,
                           int waves_target = AOS_GEMV_WAVES, bool four_waves = false, int wr_force = 0,
-                          int ks_force = 0, int direct_waves = 0) {
-  if (direct_waves > 0) {
-    gemv_geometry_direct(RB, G, T, swiglu, lora, g, direct_waves);
-    return;
-  }
+                          int ks_force = 0) {
   int W = (swiglu || four_waves) ? 4 : (G >= AOS_GEMV_W8_MIN_G ? 8 : 4);
   int ks = 1;
   g.wr = 1;
@@ -1365,6 +1372,23 @@ static void gemv_geometry(int RB, int G, int T, bool swiglu, bool lora, aos_gemv
   g.lds_bytes = (int)(lds_x > lds_r ? lds_x : lds_r);
 }
 
+/* Geometry of a layer's decode GEMV launch over RB row blocks (of all its matrices): the forwards' choice
+ * between reading x directly and staging it. The down GEMV streams beside the h shrink of its launch: more K
+ * splits (measured: 3 at the 7B shape) keep its tail short; at 1-2 tokens it runs in the gate/up launch's
+ * grid, in 4-wave workgroups like the rest of that grid. */
+static void gemv_launch_geometry(int kind, int RB, int G, int T, int n, int rpad, int wr_force, int ks_force,
+                                 aos_gemv_params &g) {
+  const int dx = gemv_direct_waves(kind, G, T, n, rpad, wr_force, ks_force);
+  if (dx > 0) {
+    gemv_geometry_direct(RB, G, T, kind == GV_GATE_UP, rpad > 0, g, dx);
+    return;
+  }
+  const int target = kind == GV_DOWN   ? (T <= 2 ? AOS_GEMV_WAVES_DOWN12 : 2 * AOS_GEMV_WAVES)
+                     : kind == GV_PROJ ? (T <= 2 ? AOS_GEMV_WAVES_PROJ12 : AOS_GEMV_WAVES)
+                                       : AOS_GEMV_WAVES;
+  gemv_geometry(RB, G, T, kind == GV_GATE_UP, rpad > 0, g, target, kind == GV_DOWN && T <= 2, wr_force, ks_force);
+}
+
 /* Shrink geometry: a target number of workgroups over the row blocks (512 waves for 4-wave
  * workgroups, 2048 for 8-wave ones; measured best at decode with the shrink running beside its
  * GEMV), at least one group per wave, x slice within the LDS budget, at most 16 K splits (their
@@ -1372,71 +1396,53 @@ static void gemv_geometry(int RB, int G, int T, bool swiglu, bool lora, aos_gemv
 #ifndef AOS_SHRINK_WGS
 #define AOS_SHRINK_WGS 256
 #endif
-/* The x shrink's budget for staged x above 16 tokens: those fused launches run two waves per SIMD
- * (their registers), so 64 KB of LDS per workgroup costs them no residency, and fewer K splits
- * keep the launch within one round of resident workgroups (the 32-stream projections: 336 shrink
- * workgroups at 32 KB, 192 at 64 KB). */
-#define AOS_XSHRINK_LDS_MAX_T32 (64 * 1024)
-static size_t x_shrink_lds_max(int T, bool direct) {
-  return T > 16 && !direct ? AOS_XSHRINK_LDS_MAX_T32 : AOS_GEMV_LDS_MAX;
-}
-
-static void shrink_geometry(int rb_total, int G, int T, aos_shrink_params &sp, int waves = 4,
-                            size_t lds_max = AOS_GEMV_LDS_MAX) {
+static void shrink_geometry(int rb_total, int G, int T, aos_shrink_params &sp, int waves = 4) {
   const int target = waves == 8 ? AOS_SHRINK_WGS : AOS_SHRINK_WGS / 2;
   int ks = ceil_div(target, rb_total > 0 ? rb_total : 1);
   int cap = G / waves; /* every wave of a workgroup gets at least one group */
   if (cap < 1) cap = 1;
   if (cap > 16) cap = 16;
   if (ks > cap) ks = cap;
-  while (ks < G && 128 + (size_t)T * ceil_div(G, ks) * 128 > lds_max) ++ks;
+  while (ks < G && 128 + (size_t)T * ceil_div(G, ks) * 128 > AOS_GEMV_LDS_MAX) ++ks;
   size_t lds_x = 128 + (size_t)T * ceil_div(G, ks) * 128;
   size_t lds_r = (size_t)waves * nv_for(T) * 64 * 4;
   sp.ks = ks;
   sp.lds_bytes = (int)(lds_x > lds_r ? lds_x : lds_r);
 }
 
-/* Diagnostic (no counterpart in the reference): the decode geometry of the launches that stage x in LDS
- * (1-2 tokens, pinned shapes, few K groups, wide unions; the others: gemv_geometry_direct), for a
+/* Diagnostic (no counterpart in the reference): the decode geometry that the forwards choose, for a
  * CPU-side check that every wave of every launch gets at least one K group. kind 0: the gate/up
  * GEMV (out = intermediate, in = hidden); 1: the down GEMV (out = hidden, in = intermediate);
  * 2: a projection GEMV (out = the row count of the matrices sharing x); 3: a shrink over `out`
  * rank rows launched with 8 waves when in / 64 >= AOS_GEMV_W8_MIN_G, else 4 (the x shrink);
- * 4: the same with 8 waves (the h shrink). Writes the waves, the K splits, the row blocks per
- * workgroup (GEMVs; 1 for a shrink) and the fewest groups any wave gets. */
-extern "C" int aoship_internal_decode_geometry_pinned(int kind, int out, int in, int T, int wr_pin, int ks_pin,
-                                                      int *waves, int *ks, int *wr, int *min_groups);
-
-extern "C" int aoship_internal_decode_geometry(int kind, int out, int in, int T, int *waves, int *ks, int *wr,
+ * 4: the same with 8 waves (the h shrink). n, rpad: the adapter table's size and padded rank (GEMVs).
+ * wr_pin, ks_pin: a GEMV shape pinned as aoship_internal_layer_set_gemv_geometry pins it (wr_pin row
+ * blocks per workgroup, ks_pin K splits; 0: the geometry's own choice; GEMV kinds only). Writes whether
+ * the launch's waves read x themselves, the waves, the K splits, the row blocks per workgroup (GEMVs; 1
+ * for a shrink) and the fewest groups any wave gets. */
+extern "C" int aoship_internal_decode_geometry(int kind, int out, int in, int T, int n, int rpad, int wr_pin,
+                                               int ks_pin, int *direct, int *waves, int *ks, int *wr,
                                                int *min_groups) {
-  return aoship_internal_decode_geometry_pinned(kind, out, in, T, 0, 0, waves, ks, wr, min_groups);
-}
-
-/* The same with a GEMV shape pinned as aoship_internal_layer_set_gemv_geometry pins it (wr_pin row
- * blocks per workgroup, ks_pin K splits; 0: the geometry's own choice; GEMV kinds only). */
-extern "C" int aoship_internal_decode_geometry_pinned(int kind, int out, int in, int T, int wr_pin, int ks_pin,
-                                                      int *waves, int *ks, int *wr, int *min_groups) {
-  if (out < 32 || in < 64 || in % 64 || T < 1 || T > AOS_DECODE_MAX_T || !waves || !ks || !wr || !min_groups ||
-      wr_pin < 0 || wr_pin > 8 || (wr_pin & (wr_pin - 1)) || ks_pin < 0 || ks_pin > 64 ||
-      (kind > 2 && (wr_pin || ks_pin)))
+  if (out < 32 || in < 64 || in % 64 || T < 1 || T > AOS_DECODE_MAX_T || n < 0 || n > AOS_MAX_ADAPTERS || rpad < 0 ||
+      rpad > 1024 || rpad % 16 || !direct || !waves || !ks || !wr || !min_groups || wr_pin < 0 || wr_pin > 8 ||
+      (wr_pin & (wr_pin - 1)) || ks_pin < 0 || ks_pin > 64 || (kind > 2 && (wr_pin || ks_pin)))
     return set_err("aoship_internal_decode_geometry: bad arguments");
   const int G = in / 64, RB = out / 32;
   int W = 4, k = 1, r = 1;
-  if (kind <= 2) {
+  *direct = 0;
+  if (kind >= 0 && kind <= 2) {
     aos_gemv_params g;
     memset(&g, 0, sizeof(g));
-    const int target = kind == 1   ? (T <= 2 ? AOS_GEMV_WAVES_DOWN12 : 2 * AOS_GEMV_WAVES)
-                       : kind == 2 ? (T <= 2 ? AOS_GEMV_WAVES_PROJ12 : AOS_GEMV_WAVES)
-                                   : AOS_GEMV_WAVES;
-    gemv_geometry(RB, G, T, kind == 0, true, g, target, kind == 1 && T <= 2, wr_pin, ks_pin);
+    gemv_launch_geometry(kind, RB, G, T, n, rpad, wr_pin, ks_pin, g);
+    *direct = g.dx;
     W = g.waves;
     k = g.ks;
     r = g.wr;
-  } else if (kind <= 4) {
+  } else if (kind == 3 || kind == 4) {
     aos_shrink_params sp;
     memset(&sp, 0, sizeof(sp));
     W = kind == 4 ? 8 : (G >= AOS_GEMV_W8_MIN_G ? 8 : 4);
-    shrink_geometry(RB, G, T, sp, W, kind == 3 ? x_shrink_lds_max(T, false) : AOS_GEMV_LDS_MAX);
+    shrink_geometry(RB, G, T, sp, W);
     k = sp.ks;
   } else {
     return set_err("aoship_internal_decode_geometry: unknown kind");
@@ -1444,7 +1450,7 @@ extern "C" int aoship_internal_decode_geometry_pinned(int kind, int out, int in,
   *waves = W;
   *ks = k;
   *wr = r;
-  *min_groups = (G / k) / (W / r);
+  *min_groups = *direct ? G / (k * W) : (G / k) / (W / r);
   return 0;
 }
 
@@ -1549,7 +1555,7 @@ static size_t fused_flag_words(const aos_gemv_params *gp, int n) {
 
 static void plan_x_shrink(aoship_layer *l, Carve &cv, const uint16_t *x, int T, int in,
                           const aos_lora_tab *tabs, int nm, aos_plan *plan,
-                          const aoship_ring_t *rings, bool direct, XShrink &xs) {
+                          const aoship_ring_t *rings, XShrink &xs) {
   const int n = (int)l->table.size();
   int umax = n < 8 * T ? n : 8 * T;
   if (umax < 1) umax = 1;
@@ -1574,7 +1580,7 @@ static void plan_x_shrink(aoship_layer *l, Carve &cv, const uint16_t *x, int T, 
     rb_total += sp.n_rb[i];
   }
   /* sized for the waves of the GEMV it may be fused with (valid for the 4-wave launch too) */
-  shrink_geometry(rb_total, in / 64, T, sp, in / 64 >= AOS_GEMV_W8_MIN_G ? 8 : 4, x_shrink_lds_max(T, direct));
+  shrink_geometry(rb_total, in / 64, T, sp, in / 64 >= AOS_GEMV_W8_MIN_G ? 8 : 4);
   sp.part = cv.b.take<float>((size_t)rb_total * sp.ks * nv_for(T) * 64);
   sp.counters = cv.counters((size_t)rb_total + 1);
   xs.separate_plan = !all;
@@ -1632,11 +1638,7 @@ static void plan_mlp(aoship_layer *l, int T, const uint16_t *x, const aoship_rin
   Carve cv(ws, ctr, flg);
   aos_plan *plan = cv.b.take<aos_plan>(1);
   uint16_t *h = cv.b.take<uint16_t>((size_t)T * I);
-  const int cols_gu = n * (tabs_gu[0].rpad > tabs_gu[1].rpad ? tabs_gu[0].rpad : tabs_gu[1].rpad);
-  const bool direct_gu =
-      gemv_direct(Wg.G, T, l->geo_wr[0], l->geo_ks[0]) && (T > 8 || cols_gu <= AOS_GEMV_DX_GU_COLS);
-  const bool direct_dn = gemv_direct(Wd.G, T, l->geo_wr[1], l->geo_ks[1]);
-  plan_x_shrink(l, cv, x, T, H, tabs_gu, 2, plan, rings, direct_gu, P.sx);
+  plan_x_shrink(l, cv, x, T, H, tabs_gu, 2, plan, rings, P.sx);
 
   aos_gemv_params &g1 = P.gv1;
   memset(&g1, 0, sizeof(g1));
@@ -1644,8 +1646,8 @@ static void plan_mlp(aoship_layer *l, int T, const uint16_t *x, const aoship_rin
   g1.w1 = Wu.dev();
   g1.x = x;
   g1.T = T;
-  gemv_geometry(Wg.RB, Wg.G, T, true, tabs_gu[0].rpad > 0 || tabs_gu[1].rpad > 0, g1, AOS_GEMV_WAVES, false,
-                l->geo_wr[0], l->geo_ks[0], direct_gu ? AOS_GEMV_DX_WAVES : 0);
+  gemv_launch_geometry(GV_GATE_UP, Wg.RB, Wg.G, T, n, std::max(tabs_gu[0].rpad, tabs_gu[1].rpad),
+                       l->geo_wr[GV_GATE_UP], l->geo_ks[GV_GATE_UP], g1);
   g1.tab0 = tabs_gu[0];
   g1.tab1 = tabs_gu[1];
   g1.S0 = P.sx.sp.S[0];
@@ -1684,11 +1686,7 @@ static void plan_mlp(aoship_layer *l, int T, const uint16_t *x, const aoship_rin
   g2.w0 = Wd.dev();
   g2.x = h;
   g2.T = T;
-  /* the down GEMV streams beside the h shrink of its launch: more K splits (measured: 3 at the
-   * 7B shape) keep its tail short; at 1-2 tokens it runs in the gate/up launch's grid, in
-   * 4-wave workgroups like the rest of that grid */
-  gemv_geometry(Wd.RB, Wd.G, T, false, td.rpad > 0, g2, T <= 2 ? AOS_GEMV_WAVES_DOWN12 : 2 * AOS_GEMV_WAVES, T <= 2,
-                l->geo_wr[1], l->geo_ks[1], direct_dn ? AOS_GEMV_DX_WAVES : 0);
+  gemv_launch_geometry(GV_DOWN, Wd.RB, Wd.G, T, n, td.rpad, l->geo_wr[GV_DOWN], l->geo_ks[GV_DOWN], g2);
   g2.tab0 = td;
   g2.S0 = s2.S[0];
   g2.s_stride0 = s2.s_stride[0];
@@ -2755,19 +2753,22 @@ static void plan_proj_decode(aoship_layer *l, Carve &cv, const int *mods, int nm
   aos_lora_tab tabs[3];
   for (int i = 0; i < nm; ++i) tabs[i] = lora_tab(l, mods[i], in, l->mats[mods[i]].out);
   aos_plan *plan = cv.b.take<aos_plan>(1);
-  const bool direct = gemv_direct(in / 64, Tc, l->geo_wr[2], l->geo_ks[2]);
-  plan_x_shrink(l, cv, xc, Tc, in, tabs, nm, plan, rc, direct, Q.xs);
+  plan_x_shrink(l, cv, xc, Tc, in, tabs, nm, plan, rc, Q.xs);
   memset(&Q.g3, 0, sizeof(Q.g3));
   aos_gemv_params *gp = Q.g3.p;
-  int rb_all = 0;
-  for (int i = 0; i < nm; ++i) rb_all += l->mats[mods[i]].RB;
+  int rb_all = 0, rmax = 0;
+  for (int i = 0; i < nm; ++i) {
+    rb_all += l->mats[mods[i]].RB;
+    rmax = std::max(rmax, tabs[i].rpad);
+  }
   for (int i = 0; i < nm; ++i) {
     const Q4Mat &W = l->mats[mods[i]];
     gp[i].w0 = W.dev();
     gp[i].x = xc;
     gp[i].T = Tc;
-    gemv_geometry(rb_all, W.G, Tc, false, tabs[i].rpad > 0, gp[i], Tc <= 2 ? AOS_GEMV_WAVES_PROJ12 : AOS_GEMV_WAVES,
-                  false, l->geo_wr[2], l->geo_ks[2], direct ? AOS_GEMV_DX_WAVES_PROJ : 0);
+    gemv_launch_geometry(GV_PROJ, rb_all, W.G, Tc, (int)l->table.size(), rmax, l->geo_wr[GV_PROJ],
+                         l->geo_ks[GV_PROJ], gp[i]);
+    gp[i].has_expand = tabs[i].rpad > 0 ? 1 : 0;
     gp[i].tab0 = tabs[i];
     gp[i].S0 = Q.xs.sp.S[i];
     gp[i].s_stride0 = Q.xs.sp.s_stride[i];

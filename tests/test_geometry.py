@@ -1,10 +1,11 @@
 """Decode launch geometry (CPU): every wave of every GEMV launch gets at least one K group.
 
-The decode GEMVs split K over the waves of a workgroup and over ks workgroups per row block, and
-the LDS budget for the staged activations can force more splits than the waves per workgroup
-allow. The geometry then falls back to 4-wave workgroups; a wave with no group would otherwise
-prime its weight ring from before the matrix. This replays the library's own geometry (the same
-function the forwards call) for every workload shape at every decode token count.
+The decode GEMVs split K over the waves of a workgroup and over ks workgroups per row block. Where
+the waves read the activations themselves (3 or more tokens, in general) a wave with no group would
+read before the row block; where the activations are staged, the LDS budget can force more splits
+than the waves per workgroup allow, and the geometry then falls back to 4-wave workgroups. This
+replays the library's own choice (the same function the forwards call) for every workload shape at
+every decode token count, over narrow and wide adapter tables.
 """
 import pytest
 
@@ -19,29 +20,44 @@ PROJ_SHAPES = [(3072 + 1024 + 1024, 3072), (3072, 3072), (3584 + 512 + 512, 3584
 SHRINK_ROWS = [(8 * 16 * 2, 896), (16 * 16 * 2, 3584), (32 * 16 * 3, 3072), (64 * 64 * 2, 5120),
                (16 * 48 * 2, 3584)]
 H_SHRINK_ROWS = [(8 * 16, 4864), (16 * 16, 18944), (64 * 64, 27648), (16 * 48, 18944)]
+# adapter tables: none, 16 of rank 16, 64 of rank 64
+TABLES = [(0, 0), (16, 16), (64, 64)]
+LAUNCHES = [(k, o, i) for H, I in MLP_SHAPES for k, o, i in ((0, I, H), (1, H, I))] + [(2, o, i) for o, i in PROJ_SHAPES]
+# few K groups: the fewest that a launch reading x itself takes (8), and fewer; few and many row blocks
+LAUNCHES += [(k, o, 64 * G) for k in (0, 1, 2) for o in (32, 96, 4096) for G in (4, 5, 7, 8, 9, 15, 16, 17, 33)]
 
 
 @pytest.mark.parametrize("T", range(1, 33))
-def test_every_gemv_wave_gets_a_group(T):
-    for H, I in MLP_SHAPES:
-        for kind, out, inp in ((0, I, H), (1, H, I)):
-            w, ks, wr, g = aoship.decode_geometry(kind, out, inp, T)
-            assert w in (4, 8) and 1 <= ks <= inp // 64 and wr in (1, 2, 4, 8) and w % wr == 0
-            assert wr == 1 or T > 2, "1-2 tokens keep one row block per workgroup (the h shrink needs it)"
-            assert g >= 1, f"kind {kind} {out}x{inp} T={T}: waves {w}, splits {ks}, rows {wr}"
-            budget = 64 * 1024 if (kind == 1 and w == 8 and T > 2) else 32 * 1024
-            assert 128 + T * -(-(inp // 64) // ks) * 136 <= budget, "staged x exceeds the LDS budget"
-    for out, inp in PROJ_SHAPES:
-        w, ks, wr, g = aoship.decode_geometry(2, out, inp, T)
-        assert g >= 1, f"projection {out}x{inp} T={T}: waves {w}, splits {ks}, rows {wr}"
-        budget = 64 * 1024 if (w == 8 and T > 2) else 32 * 1024
-        assert 128 + T * -(-(inp // 64) // ks) * 136 <= budget, "staged x exceeds the LDS budget"
+@pytest.mark.parametrize("n,rpad", TABLES)
+def test_every_gemv_wave_gets_a_group(T, n, rpad):
+    for kind, out, inp in LAUNCHES:
+        G = inp // 64
+        direct, w, ks, wr, g = aoship.decode_launch(kind, out, inp, T, n=n, rpad=rpad)
+        case = f"kind {kind} {out}x{inp} T={T} n={n}: direct {direct}, waves {w}, splits {ks}, rows {wr}"
+        assert w in (4, 8) and 1 <= ks <= G and wr in (1, 2, 4, 8) and w % wr == 0, case
+        assert wr == 1 or T > 2, "1-2 tokens keep one row block per workgroup (the h shrink needs it)"
+        assert g >= 1, case
+        assert direct == (T > 2 and G >= 8 and not (kind == 0 and T <= 8 and n * rpad > 1024)), case
+        if direct:  # 4 waves on one row block, a K group for each wave of its splits
+            assert w == 4 and wr == 1 and 4 * ks <= G, case
+        else:
+            assert 128 + T * -(-G // ks) * 136 <= 32 * 1024, f"staged x exceeds the LDS budget: {case}"
+
+
+@pytest.mark.parametrize("T", range(3, 33))
+def test_every_wave_of_a_pinned_staged_launch_gets_a_group(T):
+    """Pinned to any one row split, the launches stage x: 8 waves over a long K with up to 64 KB of it."""
+    for kind, out, inp in LAUNCHES[: 2 * len(MLP_SHAPES) + len(PROJ_SHAPES)]:
+        for wr_pin in (1, 2, 4, 8):
+            direct, w, ks, wr, g = aoship.decode_launch(kind, out, inp, T, wr_pin=wr_pin)
+            case = f"kind {kind} {out}x{inp} T={T} pin {wr_pin}: waves {w}, splits {ks}, rows {wr}"
+            assert not direct and w in (4, 8) and 1 <= ks <= inp // 64 and w % wr == 0 and g >= 1, case
+            assert 128 + T * -(-(inp // 64) // ks) * 136 <= (64 if w == 8 else 32) * 1024, case
 
 
 @pytest.mark.parametrize("T", range(1, 33))
 def test_shrink_geometry_within_limits(T):
-    """Shrinks: the K splits stay within the groups and the LDS budget (64 KB for the x shrink above
-    16 tokens, else 32 KB). A shrink wave may get no
+    """Shrinks: the K splits stay within the groups and the LDS budget (32 KB). A shrink wave may get no
     group when its launch runs more waves per workgroup than its splits leave groups; it then
     reads the zero row and adds nothing."""
     for kind, shapes in ((3, SHRINK_ROWS), (4, H_SHRINK_ROWS)):
@@ -49,10 +65,7 @@ def test_shrink_geometry_within_limits(T):
             w, ks, _, g = aoship.decode_geometry(kind, rows, inp, T)
             G = inp // 64
             assert 1 <= ks <= G
-            # the x shrink above 16 tokens runs in launches held to two waves per SIMD by their
-            # registers: 64 KB of staged x costs them no residency
-            budget = 64 * 1024 if (kind == 3 and T > 16) else 32 * 1024
-            assert 128 + T * -(-G // ks) * 128 <= budget
+            assert 128 + T * -(-G // ks) * 128 <= 32 * 1024
 
 
 @pytest.mark.parametrize("T", [1, 2])
@@ -75,3 +88,5 @@ def test_geometry_rejects_bad_shapes():
         aoship.decode_geometry(0, 3584, 100, 1)
     with pytest.raises(aoship.AosError):
         aoship.decode_geometry(0, 3584, 3584, 33)
+    with pytest.raises(aoship.AosError):
+        aoship.decode_geometry(0, 3584, 3584, 3, n=4, rpad=20)
