@@ -1301,14 +1301,24 @@ static void gemv_geometry_rows(int RB, int G, int T, bool swiglu, int W, aos_gem
  * 0.5B-shaped MLP 46 -> 36 us at 8. 1024 and 1536 waves measure the same, 512 and 3072 lose up to a fifth;
  * the projections, whose splits' reduction is a larger part, are best at 512 (7B q/k/v and o at 8 tokens 30 us,
  * at 2048 waves 33 us, staged 35 us).
- * A gate/up launch of at most 8 tokens over a wide adapter table stays staged: a row block then has twice the
- * waves to share its expand steps (64 adapters of rank 64, hidden 5120: 350 us staged, 415 us here at 8
- * tokens; 671 and 597 us at 16, where staging x costs more). */
+ * With a wide union (a module's columns over the adapters that the tokens can use above AOS_GEMV_DX_COLS) the
+ * expand, whose steps a row block's waves share, is the longer part: a launch then takes more waves (several
+ * splits of a row block). 64 adapters of rank 64, staged before / these waves / the waves above:
+ *   q/k/v, 7B shape (144 row blocks) at 4, 8 and 16 tokens: 43, 57, 83 / 40, 50, 63 / 50, 63, 81 us;
+ *   o, hidden 5120 (160 row blocks): 39, 44, 79 / 35, 38, 52 / 43, 52, 69 us;
+ *   down, 32B shape at 3, 8 and 16 tokens: 61, 115, 205 / 58, 100, 140 / 66, 109, 145 us (20 adapters, 7B shape
+ *   at 12 tokens: 61 / 46 / 43 us, hence its wider line);
+ *   gate/up, hidden 4096, intermediate 11008, at 12 and 16 tokens: 202, 242 / 140, 157 / 218, 251 us.
+ * A gate/up launch of at most 8 tokens over a wide table stays staged: the 7B and 32B shapes at 8 tokens take
+ * 167 and 246 us staged, 185 and 308 us here. */
 #define AOS_GEMV_DX_MIN_T 3
 #define AOS_GEMV_DX_MIN_G 8
 #define AOS_GEMV_DX_WAVES 1024
 #define AOS_GEMV_DX_WAVES_PROJ 512
-#define AOS_GEMV_DX_GU_COLS 1024 /* a module's columns over the whole table, up to which 3-8 tokens read x directly */
+#define AOS_GEMV_DX_COLS 1024
+#define AOS_GEMV_DX_COLS_DOWN 1280
+#define AOS_GEMV_DX_WAVES_WIDE 2048
+#define AOS_GEMV_DX_WAVES_WIDE_DOWN 1536
 
 /* The decode GEMV launches, as the diagnostics number them. */
 enum { GV_GATE_UP = 0, GV_DOWN = 1, GV_PROJ = 2 };
@@ -1318,7 +1328,10 @@ enum { GV_GATE_UP = 0, GV_DOWN = 1, GV_PROJ = 2 };
  * shape. */
 static int gemv_direct_waves(int kind, int G, int T, int n, int rpad, int wr_force, int ks_force) {
   if (T < AOS_GEMV_DX_MIN_T || G < AOS_GEMV_DX_MIN_G || wr_force > 0 || ks_force > 0) return 0;
-  if (kind == GV_GATE_UP && T <= 8 && n * rpad > AOS_GEMV_DX_GU_COLS) return 0;
+  if (kind == GV_GATE_UP && T <= 8 && n * rpad > AOS_GEMV_DX_COLS) return 0;
+  const int cols = std::min(n, 8 * T) * rpad;
+  if (kind == GV_DOWN) return cols > AOS_GEMV_DX_COLS_DOWN ? AOS_GEMV_DX_WAVES_WIDE_DOWN : AOS_GEMV_DX_WAVES;
+  if (cols > AOS_GEMV_DX_COLS) return AOS_GEMV_DX_WAVES_WIDE;
   return kind == GV_PROJ ? AOS_GEMV_DX_WAVES_PROJ : AOS_GEMV_DX_WAVES;
 }
 

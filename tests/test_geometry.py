@@ -44,6 +44,20 @@ def test_every_gemv_wave_gets_a_group(T, n, rpad):
             assert 128 + T * -(-G // ks) * 136 <= 32 * 1024, f"staged x exceeds the LDS budget: {case}"
 
 
+# (kind, row blocks, K groups): 7B q/k/v, 32B o and down, gate/up of hidden 4096
+@pytest.mark.parametrize("kind,rb,G", [(2, 144, 56), (2, 160, 80), (1, 160, 432), (0, 344, 64)])
+@pytest.mark.parametrize("T", [3, 8, 9, 32])
+def test_wide_unions_get_more_waves(kind, rb, G, T):
+    """Over 64 adapters of rank 64 (up to 256 expand steps of each row block) a launch that reads x itself has
+    at least half as many splits again; over the columns of the line and below, the narrow table's."""
+    if kind == 0 and T <= 8:
+        return  # staged
+    narrow = aoship.decode_geometry(kind, 32 * rb, 64 * G, T, n=16, rpad=16)[1]
+    line = aoship.decode_geometry(kind, 32 * rb, 64 * G, T, n=64, rpad=16)[1]
+    wide = aoship.decode_geometry(kind, 32 * rb, 64 * G, T, n=64, rpad=64)[1]
+    assert narrow == line and 2 * wide >= 3 * narrow, (narrow, line, wide)
+
+
 @pytest.mark.parametrize("T", range(3, 33))
 def test_every_wave_of_a_pinned_staged_launch_gets_a_group(T):
     """Pinned to any one row split, the launches stage x: 8 waves over a long K with up to 64 KB of it."""
