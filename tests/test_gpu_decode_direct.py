@@ -2,7 +2,9 @@
 
 Token counts on both sides of each accumulator size (8, 16, 32), the fewest K groups the path takes (8)
 and the most that do not (7), group and row-block counts that nothing divides, one rank step and several,
-each hand-off setting, routed in the call or not, against 64-bit arithmetic over the same weights. Three
+each hand-off setting, against 64-bit arithmetic over the same weights; wide adapter tables, which get more
+waves or keep a staged gate/up launch beside a direct down launch, and a plan built by a launch of its own; and
+the routed call, bit for bit the separate calls. Three
 roundings to bfloat16 separate them (h, the scaled shrink, the result), each at most 2^-9 of what it
 rounds: 3 * 2^-9 in the 2-norm.
 """
@@ -67,8 +69,17 @@ def _err(got, ref):
     return np.linalg.norm(got.float().cpu().numpy().astype(np.float64) - ref) / np.linalg.norm(ref)
 
 
-@pytest.mark.parametrize("hidden,inter,n,rank", [(448, 512, 4, 4), (512, 576, 5, 16), (1088, 2112, 20, 40)])
-@pytest.mark.parametrize("T", [3, 8, 9, 16, 17, 32])
+NARROW = [(h, i, n, r, T) for h, i, n, r in [(448, 512, 4, 4), (512, 576, 5, 16), (1088, 2112, 20, 40)]
+          for T in (3, 8, 9, 16, 17, 32)]
+# at 3 tokens 64 adapters are more than twice a union: the plan comes from a launch of its own, before a direct
+# gate/up launch (1024 columns) and before a staged one (65 adapters, 1040 columns; 26 of rank 40, 1248); the
+# wide unions at 9 and more tokens, one of them past the down launch's line (27 of padded rank 48, 1296)
+WIDE = [(1088, 2112, 64, 16, 3), (1088, 2112, 64, 16, 8), (1088, 2112, 65, 16, 3), (1088, 2112, 65, 16, 8),
+        (1088, 2112, 65, 16, 9), (1088, 2112, 26, 40, 32), (1088, 2112, 27, 40, 3), (1088, 2112, 27, 40, 17),
+        (512, 576, 70, 40, 32)]
+
+
+@pytest.mark.parametrize("hidden,inter,n,rank,T", NARROW + WIDE)
 def test_direct_decode_mlp_and_projections(hip, hidden, inter, n, rank, T):
     import torch
 
@@ -101,3 +112,25 @@ def test_direct_decode_mlp_and_projections(hip, hidden, inter, n, rank, T):
         assert _err(y[0], ref) <= TOL, s
         for m, out in (("q_proj", q), ("k_proj", k), ("v_proj", v), ("o_proj", o)):
             assert _err(out, _linear(base, lora, m, xf, coef)) <= TOL, (s, m)
+
+
+@pytest.mark.parametrize("hidden,inter,n,rank", [(512, 576, 5, 16), (1088, 2112, 20, 40), (1088, 2112, 65, 16)])
+@pytest.mark.parametrize("T", [3, 8, 17, 27, 32])
+def test_routed_call_equals_the_separate_calls(hip, hidden, inter, n, rank, T):
+    """The router in the gate/up launch (at 3 tokens over 65 adapters: ahead of it)."""
+    import torch
+
+    from test_gpu_route_mlp import _combined, _separate
+
+    rng = np.random.default_rng(7000 + T + n)
+    layer, ads, _, _ = _build(hip, rng, dict(gate_proj=(inter, hidden), up_proj=(inter, hidden),
+                                             down_proj=(hidden, inter)), n, rank)
+    router = hip.Router(n, min(4, n), 1.0, 0.02, 1.0, rng.permutation(n).astype(np.uint64))
+    f = torch.from_numpy(rng.standard_normal((T, hidden), dtype=np.float32)).cuda()
+    w = torch.from_numpy(rng.standard_normal((n, hidden), dtype=np.float32) * np.float32(0.05)).cuda()
+    x = _bf16(rng.standard_normal((T, hidden))).view(torch.int16).cuda()
+    ref = _separate(router, layer, f, w, x)
+    for got in (_combined(router, layer, f, w, x), _combined(router, layer, f, w, x)):
+        for a, b, name in zip(ref, got, ("rings", "status", "y")):
+            assert np.array_equal(a, b), name
+    assert layer.wait_timeouts() == 0
