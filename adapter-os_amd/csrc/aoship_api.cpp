@@ -53,7 +53,7 @@ static int g_device = -1;
  * ends): arrival counters (zero at rest), generation-stamped ready flags (zero at first use),
  * then the workspace. Host code never uses the array's name as an address: at set-up, with the
  * device current, hipGetSymbolAddress gives this device's copy, kept per device. */
-#define AOS_SCRATCH_BYTES ((size_t)32 << 20)
+#define AOS_SCRATCH_BYTES ((size_t)33 << 20)
 #define AOS_SCRATCH_CTR_BYTES ((size_t)256 << 10)
 #define AOS_SCRATCH_FLAG_BYTES ((size_t)4 << 20)
 #define AOS_SCRATCH_WS_BYTES (AOS_SCRATCH_BYTES - AOS_SCRATCH_CTR_BYTES - AOS_SCRATCH_FLAG_BYTES)
@@ -1631,7 +1631,7 @@ struct MlpPlan {
                               (1-2 tokens only, else NULL) */
   uint32_t *hdone;         /* one-launch MLP (1-2 tokens): gate/up row blocks done */
   uint32_t *hflags;        /* ... and the lines raised when h is complete */
-  int hsum_wgs = 0;        /* workgroups summing the h shrink's partials */
+  int hsum_wgs = 0;        /* workgroups summing the h shrink's partials (0 without them) */
   uint32_t *route_done;    /* the combined route + gate/up launch's router arrivals */
   uint32_t *route_flag;    /* ... and its routing flag */
   uint32_t *rpart_ctr;     /* ... its per-token counts of prior workgroups */
@@ -1711,8 +1711,9 @@ static void plan_mlp(aoship_layer *l, int T, const uint16_t *x, const aoship_rin
   g2.part = cv.b.take<float>((size_t)Wd.RB * g2.ks * nv_for(T) * 64);
   g2.counters = cv.counters((size_t)Wd.RB);
 
-  P.hpart = T <= 2 ? cv.b.take<float>((size_t)Wg.RB * T * s2.s_stride[0]) : nullptr;
-  P.hsum_wgs = ceil_div(T * s2.s_stride[0], AOS_HSUM_V);
+  const bool h_parts = T <= 2;
+  P.hpart = h_parts ? cv.b.take<float>((size_t)Wg.RB * T * s2.s_stride[0]) : nullptr;
+  P.hsum_wgs = h_parts ? ceil_div(T * s2.s_stride[0], AOS_HSUM_V) : 0;
   P.hdone = cv.counter_lines(AOS_ARRIVE_WORDS(Wg.RB));
   P.hflags = cv.flag_lines(((size_t)P.hsum_wgs + (size_t)g2.nrbg * g2.ks) * 32);
   P.route_done = cv.counter_lines(32);

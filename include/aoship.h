@@ -270,7 +270,7 @@ int aoship_mlp_forward(aoship_layer_t *layer, const aoship_bf16_t *x, int T,
 /* No counterpart in the reference: the decode MLP forward (aoship_mlp_forward's launches, T <= 32)
  * for callers that cannot allocate device memory (code under HIP graph capture, serving loops and
  * harnesses that forbid hipMalloc). Its workspace, counters and flags live in a static device array
- * of 32 MiB (about 29.75 MiB of workspace) that each GPU holds until the process ends; a layer and
+ * of 33 MiB (28.75 MiB of workspace) that each GPU holds until the process ends; a layer and
  * token count whose workspace does not fit is rejected with an error (-1), as is T > 32. Makes no
  * hipMalloc, hipFree or other allocating call. The array keeps the last call's contents; calls that
  * overlap on one GPU (on different streams) share it and race: serialise them. Output equals

@@ -72,3 +72,21 @@ def test_noalloc_rejections(hip):
         fits = False
     if fits:  # when it fits, it must equal the regular forward
         assert np.array_equal(y.cpu().numpy().view(np.uint16), _fwd(big, x, r, False))
+
+
+def test_noalloc_takes_a_wide_table_near_the_scratch_limit(hip):
+    """31 tokens over 32 adapters of rank 64, hidden 2048, intermediate 5632: the down launch's hand-off lines
+    alone would pass the scratch if the 1-2 token launch's partial sums (a line for every 4 values, which no
+    other launch has) were counted in."""
+    import torch
+
+    from test_gpu_decode_direct import _bf16, _build, _rings
+
+    rng = np.random.default_rng(3)
+    hidden, inter, n, T = 2048, 5632, 32, 31
+    layer, ads, _, _ = _build(hip, rng, dict(gate_proj=(inter, hidden), up_proj=(inter, hidden),
+                                             down_proj=(hidden, inter)), n, 64)
+    rings, _ = _rings(hip, rng, T, n, 4)
+    r = torch.from_numpy(rings.view(np.uint8).copy()).cuda()
+    x = _bf16(rng.standard_normal((T, hidden))).view(torch.int16).cuda()
+    assert np.array_equal(_fwd(layer, x, r, True), _fwd(layer, x, r, False))
