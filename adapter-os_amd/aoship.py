@@ -142,6 +142,8 @@ def lib():
         L.aoship_internal_layer_set_prefill_expand_adapter_major.argtypes = [_P, C.c_int]
         L.aoship_internal_layer_last_adapter_major.restype = C.c_int
         L.aoship_internal_layer_last_adapter_major.argtypes = [_P]
+        L.aoship_internal_layer_workspace.restype = C.c_size_t
+        L.aoship_internal_layer_workspace.argtypes = [_P]
         L.aoship_internal_layer_last_perm.restype = C.c_int
         L.aoship_internal_layer_last_perm.argtypes = [_P, _P, C.c_int]
         L.aoship_internal_route_tokens.restype = C.c_int
@@ -443,6 +445,10 @@ class Layer:
         or the readers look them up through the plan's list; outputs are identical."""
         _check(lib().aoship_internal_layer_set_plan_pointers(self.h, 1 if on else 0),
                "aoship_internal_layer_set_plan_pointers")
+
+    def workspace(self) -> int:
+        """Diagnostic: the bytes of the layer's workspace as it is now."""
+        return lib().aoship_internal_layer_workspace(self.h)
 
     def set_gemv_geometry(self, kind: int, wr: int = 0, ks: int = 0) -> None:
         """Diagnostic: pin the decode GEMV geometry of launch kind 0 (gate/up), 1 (down) or 2

@@ -2198,34 +2198,33 @@ static void size_proj(aoship_layer *l, const int *mods, int nm, int max_tokens, 
 
 static size_t mlp1_flag_words(aoship_layer *l);
 
-extern "C" int aoship_layer_reserve(aoship_layer_t *l, int max_tokens) {
-  if (!l) return set_err("aoship_layer_reserve: null layer");
-  if (max_tokens < 1) return set_err("aoship_layer_reserve: max_tokens must be >= 1");
-  if (ensure_device()) return -1;
-  size_t bytes = 0, ctr = 0, flg = 0;
-  const bool mlp = l->mats[MOD_GATE].valid && l->mats[MOD_UP].valid && l->mats[MOD_DOWN].valid;
-  for (int T = 1; T <= AOS_DECODE_MAX_T && T <= max_tokens; ++T) {
-    if (mlp) {
+/* Workspace bytes, counter words and flag words of every forward of up to max_tokens tokens. */
+static void size_layer(aoship_layer *l, int max_tokens, size_t &bytes, size_t &ctr, size_t &flg) {
+  auto take = [&](size_t b, size_t c, size_t f) {
+    bytes = std::max(bytes, b);
+    ctr = std::max(ctr, c);
+    flg = std::max(flg, f);
+  };
+  if (l->mats[MOD_GATE].valid && l->mats[MOD_UP].valid && l->mats[MOD_DOWN].valid) {
+    for (int T = 1; T <= AOS_DECODE_MAX_T && T <= max_tokens; ++T) {
       MlpPlan P;
       plan_mlp(l, T, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, P);
-      if (P.bytes > bytes) bytes = P.bytes;
-      if (P.ctr > ctr) ctr = P.ctr;
-      if (P.flg > flg) flg = P.flg;
+      take(P.bytes, P.ctr, P.flg);
     }
-  }
-  if (mlp) { /* the one-token launch's tagged words */
-    const size_t fw = mlp1_flag_words(l);
-    if (fw > flg) flg = fw;
-  }
-  /* every number of token tiles up to the largest chunk's: fewer tiles are cut into more pieces */
-  for (int t0 = 0; mlp && t0 < chunk_prefill_t(max_tokens); t0 += AOS_GEMM_BM) {
-    const int T = std::min(t0 + AOS_GEMM_BM, chunk_prefill_t(max_tokens));
-    if (T <= AOS_DECODE_MAX_T) break;
-    MlpPrefill M;
-    plan_mlp_prefill(l, T, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, M);
-    if (M.bytes > bytes) bytes = M.bytes;
-    if (M.ctr > ctr) ctr = M.ctr;
-    if (M.flg > flg) flg = M.flg;
+    take(0, 0, mlp1_flag_words(l)); /* the one-token launch's tagged words */
+    /* every number of token tiles up to the largest chunk's (fewer tiles are cut into more pieces), and with
+     * adapter-major shrinks every number of blocks of AOS_GEMM_BM of a token's 8 users (fewer are cut into
+     * more K slices): within a step every part grows with the tokens */
+    const int most = chunk_prefill_t(max_tokens);
+    const bool am = l->prefill_am_tu > 0 && (int)l->table.size() >= l->prefill_am_tu;
+    const int step = am ? AOS_GEMM_BM / 8 : AOS_GEMM_BM;
+    for (int t0 = 0; t0 < most; t0 += step) {
+      const int T = std::min(t0 + step, most);
+      if (T <= AOS_DECODE_MAX_T) continue;
+      MlpPrefill M;
+      plan_mlp_prefill(l, T, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, M);
+      take(M.bytes, M.ctr, M.flg);
+    }
   }
   /* the projections: q, k and v together (aoship_qkv_forward) and each one alone */
   const int qkv[3] = {MOD_Q, MOD_K, MOD_V};
@@ -2234,8 +2233,19 @@ extern "C" int aoship_layer_reserve(aoship_layer_t *l, int max_tokens) {
     size_proj(l, qkv, 3, max_tokens, bytes, ctr, flg);
   for (int m = MOD_Q; m <= MOD_O; ++m)
     if (l->mats[m].valid) size_proj(l, &m, 1, max_tokens, bytes, ctr, flg);
+}
+
+extern "C" int aoship_layer_reserve(aoship_layer_t *l, int max_tokens) {
+  if (!l) return set_err("aoship_layer_reserve: null layer");
+  if (max_tokens < 1) return set_err("aoship_layer_reserve: max_tokens must be >= 1");
+  if (ensure_device()) return -1;
+  size_t bytes = 0, ctr = 0, flg = 0;
+  size_layer(l, max_tokens, bytes, ctr, flg);
   return ws_reserve(l, bytes, ctr, flg);
 }
+
+/* Diagnostic (no counterpart in the reference): the bytes of the layer's workspace as it is now. */
+extern "C" size_t aoship_internal_layer_workspace(const aoship_layer_t *l) { return l ? l->ws_cap : 0; }
 
 static int check_common(aoship_layer *l, const void *x, int T, const aoship_ring_t *rings,
                         const void *y) {
@@ -2798,7 +2808,7 @@ static void plan_proj_decode(aoship_layer *l, Carve &cv, const int *mods, int nm
 }
 
 /* Workspace of projections sharing x for calls of up to max_tokens tokens (decode chunks at every
- * power of two up to 32 tokens, and prefill chunks of every number of token tiles). */
+ * number of tokens, and prefill chunks of every number of token tiles). */
 static void size_proj(aoship_layer *l, const int *mods, int nm, int max_tokens, size_t &bytes, size_t &ctr,
                       size_t &flg) {
   auto take = [&](const Carve &cv) {
