@@ -1934,17 +1934,24 @@ static long gemm_tasks(int T, int RB, bool swiglu) {
   return (long)ceil_div(T, AOS_GEMM_BM) * ceil_div(RB, wv);
 }
 
+/* Floats of the partial sums of GEMM g in S pieces. */
+static size_t piece_floats(const aos_gemm_params &g, int S, bool swiglu) {
+  if (S < 2) return 0;
+  return (size_t)S * gemm_tasks(g.T, g.w0.RB, swiglu) * aos_gemm_sk_slot_floats(swiglu ? 1 : 0);
+}
+
 /* The GEMMs gp[0, n) (planned, without shrink workgroups or stream-K) as one launch in S pieces; the
- * pieces' partial sums from the workspace. */
-static void plan_multi(Carve &cv, const aos_gemm_params *gp, int n, int S, bool swiglu, aos_gemm_multi_params &q) {
+ * pieces' partial sums in part (piece_floats each, one after the other). */
+static void plan_multi(const aos_gemm_params *gp, int n, int S, bool swiglu, float *part, aos_gemm_multi_params &q) {
   memset(&q, 0, sizeof(q));
   q.n = n;
   q.S = S;
+  size_t off = 0;
   for (int i = 0; i < n; ++i) {
     q.g[i] = gp[i];
-    if (S > 1)
-      q.g[i].sk_part = cv.b.take<float>((size_t)S * gemm_tasks(gp[i].T, gp[i].w0.RB, swiglu) *
-                                        aos_gemm_sk_slot_floats(swiglu ? 1 : 0));
+    if (S < 2) continue;
+    q.g[i].sk_part = part ? part + off : nullptr;
+    off += piece_floats(gp[i], S, swiglu);
   }
 }
 
@@ -2144,8 +2151,10 @@ static void plan_mlp_prefill(aoship_layer *l, int T, const uint16_t *x, const ao
     M.xe.xam_tu = xt;
     M.use_xam = true;
   }
-  plan_multi(cv, &M.g1, 1, s1, true, M.m1);
-  plan_multi(cv, &M.g2, 1, s2, false, M.m2);
+  /* gate/up's pieces are summed before the down GEMM starts: the two share their memory */
+  float *part = cv.b.take<float>(std::max(piece_floats(M.g1, s1, true), piece_floats(M.g2, s2, false)));
+  plan_multi(&M.g1, 1, s1, true, part, M.m1);
+  plan_multi(&M.g2, 1, s2, false, part, M.m2);
   M.bytes = cv.b.off + 256;
   M.ctr = cv.coff + 64;
   M.flg = cv.foff + 64;
@@ -2760,7 +2769,9 @@ static void plan_proj_prefill(aoship_layer *l, Carve &cv, const int *mods, int n
   for (int i = 0; i < nm; ++i)
     plan_gemm(l, Q.P, Q.sp, l->mats[mods[i]], nullptr, xc, perm, perm, Tc, i, i, yc ? yc[i] : nullptr, Q.gp[i]);
   if (S == 1 && nm == 1) plan_sk(l, cv, Q.gp[0], false);
-  plan_multi(cv, Q.gp, nm, S, false, Q.mu);
+  size_t floats = 0;
+  for (int i = 0; i < nm; ++i) floats += piece_floats(Q.gp[i], S, false);
+  plan_multi(Q.gp, nm, S, false, cv.b.take<float>(floats), Q.mu);
 }
 
 /* Decode chunk (T <= 32) of projections sharing x: the x shrink (and plan) and the GEMVs, whose

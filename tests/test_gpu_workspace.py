@@ -1,4 +1,5 @@
-"""GPU: after reserve(N) a layer's forwards of up to N tokens allocate nothing (the workspace keeps its size)."""
+"""GPU: after reserve(N) a layer's forwards of up to N tokens allocate nothing (the workspace keeps its size), and
+memory that is not live together is shared."""
 import numpy as np
 import pytest
 
@@ -45,3 +46,17 @@ def test_reserve_covers_every_shorter_call(hip, hidden, inter, n, rank, most, ca
         layer.proj_forward("o_proj", x[:T], r[: 40 * T], y[:T])
         torch.cuda.synchronize()
         assert layer.workspace() == held, f"{T} tokens grew the workspace reserved for {most}"
+
+
+def test_short_prompt_pieces_share_their_memory(hip):
+    """A 7B-shaped layer at 128 tokens, no adapters: 3 pieces of 148 gate/up tasks and 18 of 14 down tasks, 128 KB
+    of partial sums a piece, of which one GEMM's are live at a time; and h."""
+    hidden, inter, T = 3584, 18944, 128
+    layer = hip.Layer(0)
+    for m, (out, inp) in dict(gate_proj=(inter, hidden), up_proj=(inter, hidden), down_proj=(hidden, inter)).items():
+        layer.set_base(m, np.zeros((out, inp // 8), np.uint32), np.zeros((out, inp // 64), np.float16),
+                       np.zeros((out, inp // 64), np.float16))
+    layer.set_adapters([])
+    layer.reserve(T)
+    pieces = 131072 * max(3 * 148, 18 * 14)
+    assert pieces < layer.workspace() <= pieces + 2 * T * inter + (1 << 20)
