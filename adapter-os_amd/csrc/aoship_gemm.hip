@@ -2033,7 +2033,8 @@ __global__ void __launch_bounds__(64 * WV, OCC) aos_gemm_sk_kernel(aos_gemm_para
   }
 }
 
-/* Up to three GEMMs in one launch, each task's K groups in q.S pieces (aos_gemm_multi_params).
+/* Up to three GEMMs in one launch, each task's K groups in q.S pieces (aos_gemm_multi_params; a SwiGLU
+ * GEMM's whole tasks run as aos_gemm_kernel).
  * Workgroups of one GEMM that land on one XCD take consecutive (piece, weight block, token tile)
  * triples, token tile fastest, so that a weight block's token tiles share an L2. */
 template <bool SW, int D, bool DBT, bool APF, int WV, int OCC, int LC, int NS>
@@ -2045,7 +2046,7 @@ __global__ void __launch_bounds__(64 * WV, OCC) aos_gemm_multi_kernel(aos_gemm_m
   if (k > 0) b -= q.wg_end[k - 1];
   const aos_gemm_params &p = q.g[k];
   int mbi, nbk;
-  if (q.S == 1) {
+  if (!SW && q.S == 1) {
     gemm_tile_of(b, p.mb, p.nb, mbi, nbk);
     gemm_task<SW, D, DBT, APF, WV, OCC, LC, NS>(p, smem, mbi, nbk, 0, p.w0.G, GEMM_WHOLE, SkCtx{0u, 0u, 0u});
     return;
@@ -2472,7 +2473,7 @@ extern "C" int aos_launch_gemm(const aos_gemm_params *p, int swiglu, const aos_l
 /* Grids of a multi-GEMM launch and its finish launch for the kernel shape of WV waves. */
 template <int WV>
 static int multi_grids(const aos_gemm_multi_params *p, int swiglu, aos_gemm_multi_params &q) {
-  if (p->n < 1 || p->n > 3 || p->S < 1 || (swiglu && p->n != 1)) return (int)hipErrorInvalidValue;
+  if (p->n < 1 || p->n > 3 || p->S < 1 || (swiglu && (p->n != 1 || p->S < 2))) return (int)hipErrorInvalidValue;
   q = *p;
   int wg = 0, fin = 0;
   for (int k = 0; k < 3; ++k) {

@@ -542,7 +542,7 @@ typedef struct {
 } aos_gemm_params;
 
 /* One launch over up to three GEMMs of one kernel shape (SwiGLU or single-matrix; n > 1: the
- * projections that share x), each task's K groups cut into S pieces. S = 1: every task runs whole,
+ * projections that share x), each task's K groups cut into S pieces. S = 1 (single-matrix): every task runs whole,
  * expand and epilogue included. S > 1: piece s of a task stores its partial sums in slot
  * (s * mb + mbi) * nb + nbk of its GEMM's sk_part (a slot: aos_gemm_sk_slot_floats floats), and the
  * finish launch adds the pieces in order, then the expand, and writes y. */
