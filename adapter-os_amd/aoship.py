@@ -146,6 +146,8 @@ def lib():
         L.aoship_internal_layer_workspace.argtypes = [_P]
         L.aoship_internal_layer_last_perm.restype = C.c_int
         L.aoship_internal_layer_last_perm.argtypes = [_P, _P, C.c_int]
+        L.aoship_internal_prefill_rule.restype = C.c_int
+        L.aoship_internal_prefill_rule.argtypes = [C.c_int] * 5
         L.aoship_internal_route_tokens.restype = C.c_int
         L.aoship_internal_route_tokens.argtypes = [C.c_int, C.c_int, C.c_int]
         L.aoship_internal_model_workspace.restype = C.c_int
@@ -179,6 +181,17 @@ def decode_geometry(kind: int, out: int, inp: int, T: int, wr_pin: int = 0, ks_p
     """(waves, K splits, row blocks per workgroup, fewest K groups of any wave) of a decode launch
     shape, optionally with a GEMV shape pinned as Layer.set_gemv_geometry pins it."""
     return decode_launch(kind, out, inp, T, wr_pin, ks_pin, n, rpad)[1:]
+
+
+PREFILL_RULES = ("gate_up_pieces", "single_pieces", "qkv_pieces")
+
+
+def prefill_rule(rule: str, tasks: int, G: int, cols: int, slots: int) -> int:
+    """A prompt GEMM rule's choice (see aoship_internal_prefill_rule)."""
+    r = lib().aoship_internal_prefill_rule(PREFILL_RULES.index(rule), tasks, G, cols, slots)
+    if r < 0:
+        raise AosError(last_error())
+    return r
 
 
 def route_tokens(T: int, n: int, d: int) -> int:

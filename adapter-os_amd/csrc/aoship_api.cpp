@@ -1905,28 +1905,57 @@ static void plan_sk(aoship_layer *l, Carve &cv, aos_gemm_params &g, bool swiglu)
 }
 
 /* K pieces of each of a launch's `tasks` (token tile, weight block) tasks of G groups: as many as keep
- * the launch in one round of the device's resident workgroups, at least AOS_SPLIT_MIN_GROUPS groups a
+ * the launch in one round of the device's resident workgroups (slots), at least AOS_SPLIT_MIN_GROUPS groups a
  * piece, 1 below `least` pieces. A task runs its groups one after the other (1 to 1.5 us each however
  * idle the chip is), so a launch of few tasks takes G times that: the 7B-shaped down GEMM of one token
  * tile, 14 tasks of 296 groups, 284 us whole and 25 + 12 us in 18 pieces; gate/up, 148 tasks of 56
  * groups, 83 us whole and 44 + 21 us in 3. least is 2, and 3 for a single matrix alone: stream-K
  * serves two pieces as well (126 tasks on 256 slots) and moves fewer partial sums. */
 #define AOS_SPLIT_MIN_GROUPS 8
-static int gemm_pieces(long tasks, int G, bool swiglu, int least) {
-  const long slots = aos_gemm_sk_slots(swiglu ? 1 : 0);
+static int gemm_pieces(long tasks, int G, long slots, int least) {
   if (tasks < 1) return 1;
   const long s = std::min(slots / tasks, (long)(G / AOS_SPLIT_MIN_GROUPS));
   return s < least ? 1 : (int)s;
+}
+
+/* The same for the gate/up GEMM. In pieces it loses the x shrink (over cols columns of a tile's union) that whole
+ * tasks carry in their launch's idle slots, and needs a finish launch; both grow with the tasks, so that beyond
+ * slots / 7 tasks (slots / 5 over few columns) the groups taken off each task's chain must pay for them. MLP of
+ * (hidden, intermediate), whole / in pieces:
+ *   44 tasks of 16 groups in 2 (1024, 2816; 256 tokens) 129 / 112 us, 176 tasks in 2 (1024 tokens) 137 / 165 us;
+ *   88 tasks in 2 over 64 columns (450 tokens) 106 / 94, 154 tasks (800 tokens) 100 / 107 us;
+ *   88 tasks of 32 in 4 (2048, 5632; 200 tokens) 134 / 122, 132 in 3 (384 tokens) 156 / 168 us;
+ *   128 tasks of 48 in 4 (3072, 8192; 256 tokens) 154 / 148, 192 in 2 (384 tokens) 180 / 202 us;
+ *   172 tasks of 64 in 2 (4096, 11008; 256 tokens) 192 / 215 us;
+ *   148 tasks of 56 in 3 (7B, 96 tokens) 159 / 158, 216 of 80 in 2 (32B, 96 tokens) 241 / 232 us. */
+#define AOS_NARROW_COLS 64      /* few columns, up to */
+#define AOS_SPLIT_GU_GROUPS4 24 /* groups off a task's chain, at least, in 4 or more pieces */
+#define AOS_SPLIT_GU_GROUPS 37  /* ... in fewer */
+static int gate_up_pieces(long tasks, int G, int cols, long slots) {
+  const int s = gemm_pieces(tasks, G, slots, 2);
+  if (s == 1 || tasks * (cols > AOS_NARROW_COLS ? 7 : 5) <= slots) return s;
+  return G - (G + s - 1) / s >= (s >= 4 ? AOS_SPLIT_GU_GROUPS4 : AOS_SPLIT_GU_GROUPS) ? s : 1;
 }
 
 /* Whether a down GEMM of these tasks leaves over 45% of its grid's last round idle and stream-K could
  * share it: then its shrink takes a launch of its own rather than that round. The 7B-shaped MLP with
  * the shrink in the launch and with stream-K: 700 tokens (84 tasks on 256 slots, in pieces) 554 and
  * 439 us, 1100 tokens (126 tasks) 658 and 618 us, 1500 tokens (168 tasks) 731 and 768 us. */
-static bool down_mostly_idle(long tasks, int G) {
-  const long slots = aos_gemm_sk_slots(0);
+static bool down_mostly_idle(long tasks, int G, long slots) {
   if (slots < 1 || tasks * G / slots < AOS_SK_MIN_GROUPS) return false;
   return tasks * 20 < (tasks + slots - 1) / slots * slots * 11;
+}
+
+/* Diagnostic (no counterpart in the reference): the prompt GEMMs' rules above for `tasks` tasks of G groups on
+ * `slots` resident workgroups. rule 0: gate/up pieces (cols columns); 1: a single matrix's pieces; 2: q/k/v's pieces. */
+extern "C" int aoship_internal_prefill_rule(int rule, int tasks, int G, int cols, int slots) {
+  if (tasks < 1 || G < 1 || cols < 0 || slots < 1) return set_err("aoship_internal_prefill_rule: bad arguments");
+  switch (rule) {
+    case 0: return gate_up_pieces(tasks, G, cols, slots);
+    case 1: return gemm_pieces(tasks, G, slots, 3);
+    case 2: return gemm_pieces(tasks, G, slots, 2);
+  }
+  return set_err("aoship_internal_prefill_rule: unknown rule");
 }
 
 static long gemm_tasks(int T, int RB, bool swiglu) {
@@ -2029,12 +2058,13 @@ static void plan_mlp_prefill(aoship_layer *l, int T, const uint16_t *x, const ao
   /* each shrink in its GEMM's launch when its workgroups fit in the idle slots of that grid's
    * last round, else a launch of its own (K split into slices) */
   M.fused_x = M.fused_h = false;
-  const int s1 = gemm_pieces(gemm_tasks(T, Wg.RB, true), Wg.G, true, 2);
-  const int s2 = gemm_pieces(gemm_tasks(T, Wd.RB, false), Wd.G, false, 3);
+  const long slots = aos_gemm_sk_slots(0), tasks_dn = gemm_tasks(T, Wd.RB, false);
+  const int tc = M.P.tu_cap, rd = tall[2].rpad, cols_gu = tc * std::max(tall[0].rpad, tall[1].rpad);
+  const int s1 = gate_up_pieces(gemm_tasks(T, Wg.RB, true), Wg.G, cols_gu, aos_gemm_sk_slots(1));
+  const int s2 = gemm_pieces(tasks_dn, Wd.G, slots, 3);
   if (M.P.lora && l->prefill_fused_shrink) {
-    const int tc = M.P.tu_cap, rg = tall[0].rpad, ru = tall[1].rpad, rd = tall[2].rpad;
-    M.fused_x = s1 == 1 && aos_gemm_shrink_fits(T, Wg.RB, tc * (rg > ru ? rg : ru), 1) != 0;
-    M.fused_h = s2 == 1 && !((l->prefill_sk & 2) && down_mostly_idle(gemm_tasks(T, Wd.RB, false), Wd.G)) &&
+    M.fused_x = s1 == 1 && aos_gemm_shrink_fits(T, Wg.RB, cols_gu, 1) != 0;
+    M.fused_h = s2 == 1 && !((l->prefill_sk & 2) && down_mostly_idle(tasks_dn, Wd.G, slots)) &&
                 aos_gemm_shrink_fits(T, Wd.RB, tc * rd, 0) != 0;
   }
   plan_tshrink(l, cv, M.P, x, perm, T, H, 0, 2, M.sx, M.fused_x);
@@ -2744,9 +2774,9 @@ extern "C" int aoship_route_mlp_forward(aoship_router_t *r, const float *feature
 }
 
 /* Prefill chunk of projections sharing x: the group plan, one tile shrink over every module, one
- * launch over the matrices' GEMMs. The same code sizes the workspace (a Carve over nullptr) and fills
- * it. The k and v GEMMs of grouped-query attention are a few tasks each, which take as long alone as
- * q's: a 7B-shaped layer's q, k and v at 1531 tokens, 190 us as three launches. A single matrix
+ * launch over the matrices' GEMMs. The same code sizes the workspace (a Carve
+ * over nullptr) and fills it. The k and v GEMMs of grouped-query attention are a few tasks each, which take as
+ * long alone as q's: a 7B-shaped layer's q, k and v at 1531 tokens, 190 us as three launches. A single matrix
  * whose grid leaves part of its last round idle runs as stream-K. */
 struct ProjPrefill {
   PrefillPlan P;
@@ -2763,9 +2793,10 @@ static void plan_proj_prefill(aoship_layer *l, Carve &cv, const int *mods, int n
   plan_prefill_common(l, cv, rc, Tc, tabs, nm, Q.P);
   const uint16_t *perm = Q.P.lora ? Q.P.gp.perm : nullptr;
   plan_tshrink(l, cv, Q.P, xc, perm, Tc, in, 0, nm, Q.sp);
+  const long slots = aos_gemm_sk_slots(0);
   long tasks = 0;
   for (int i = 0; i < nm; ++i) tasks += gemm_tasks(Tc, l->mats[mods[i]].RB, false);
-  const int S = gemm_pieces(tasks, l->mats[mods[0]].G, false, nm > 1 ? 2 : 3);
+  const int S = gemm_pieces(tasks, l->mats[mods[0]].G, slots, nm > 1 ? 2 : 3);
   for (int i = 0; i < nm; ++i)
     plan_gemm(l, Q.P, Q.sp, l->mats[mods[i]], nullptr, xc, perm, perm, Tc, i, i, yc ? yc[i] : nullptr, Q.gp[i]);
   if (S == 1 && nm == 1) plan_sk(l, cv, Q.gp[0], false);

@@ -1,0 +1,29 @@
+"""The prompt GEMMs' launch rules (CPU): which launches are cut into K pieces, leave their shrink, or run as
+stream-K, on MI355X's resident workgroups (512 of the gate/up kernel, 256 of the single-matrix kernel)."""
+import pytest
+
+import aoship
+
+
+def _tasks(T, rows, per):
+    """Tasks of T tokens and `rows` weight rows: 128-token tiles times blocks of `per` 32-row blocks."""
+    return -(-T // 128) * -(-rows // (32 * per))
+
+
+# (tokens, hidden, intermediate, columns of the union, pieces): whole where pieces measured slower
+@pytest.mark.parametrize("T,H,I,cols,want", [
+    (75, 3584, 18944, 256, 3), (128, 5120, 27648, 4096, 2), (200, 2048, 5632, 256, 4), (256, 3072, 8192, 256, 4),
+    (256, 1024, 2816, 512, 2), (450, 1024, 2816, 64, 2),
+    (450, 1024, 2816, 512, 1), (800, 1024, 2816, 64, 1), (1024, 1024, 2816, 512, 1), (384, 2048, 5632, 256, 1),
+    (384, 3072, 8192, 256, 1), (256, 4096, 11008, 768, 1), (2048, 3584, 18944, 256, 1), (75, 448, 512, 64, 1)])
+def test_gate_up_pieces(T, H, I, cols, want):
+    assert aoship.prefill_rule("gate_up_pieces", _tasks(T, I, 4), H // 64, cols, 512) == want
+
+
+@pytest.mark.parametrize("rule,slots", [("gate_up_pieces", 512), ("single_pieces", 256), ("qkv_pieces", 256)])
+def test_pieces_fit_one_round_and_keep_their_groups(rule, slots):
+    for tasks in range(1, 700):
+        for G in (4, 7, 8, 14, 16, 31, 56, 80, 296, 432):
+            for cols in (0, 64, 512):
+                s = aoship.prefill_rule(rule, tasks, G, cols, slots)
+                assert s == 1 or (s * tasks <= slots and G // s >= 8), (tasks, G, cols, s)
