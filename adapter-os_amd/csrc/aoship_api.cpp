@@ -1937,23 +1937,41 @@ static int gate_up_pieces(long tasks, int G, int cols, long slots) {
   return G - (G + s - 1) / s >= (s >= 4 ? AOS_SPLIT_GU_GROUPS4 : AOS_SPLIT_GU_GROUPS) ? s : 1;
 }
 
+/* K groups per workgroup for which the last round of a plain grid leaves a slot idle, on average. */
+static double idle_groups(long tasks, int G, long slots) {
+  const long last = tasks % slots;
+  return last ? (double)(slots - last) * G / slots : 0.0;
+}
+
 /* Whether a down GEMM of these tasks leaves over 45% of its grid's last round idle and stream-K could
- * share it: then its shrink takes a launch of its own rather than that round. The 7B-shaped MLP with
- * the shrink in the launch and with stream-K: 700 tokens (84 tasks on 256 slots, in pieces) 554 and
- * 439 us, 1100 tokens (126 tasks) 658 and 618 us, 1500 tokens (168 tasks) 731 and 768 us. */
-static bool down_mostly_idle(long tasks, int G, long slots) {
+ * share it: then its shrink (over cols columns of a tile's union) takes a launch of its own rather than that
+ * round. That launch and the sharing cost as much as 45 to 70 groups of the chain, less over few columns. MLP of
+ * (hidden, intermediate) with the shrink in the launch / with stream-K:
+ *   7B, 1100 tokens (126 tasks on 256 slots, 150 idle groups) 640 / 623 us, 800 tokens (183) 576 / 518 us;
+ *   (3072, 8192), 1024 tokens (80) 307 / 291, 1100 tokens (74) 307 / 305, 1300 tokens (62) 335 / 342 us;
+ *   (2048, 5632), 256 columns, 1300 tokens (58) 253 / 241, 1800 tokens (47) 266 / 281 us; 64 columns, 2048
+ *   tokens (44) 242 / 234 us;
+ *   (896, 4864), 4096 tokens (38) 254 / 273, over 64 columns 235 / 231; (1024, 2816), 3000 tokens (28) 187 / 204,
+ *   over 64 columns 171 / 163 us. */
+#define AOS_IDLE_DOWN_GROUPS 55
+#define AOS_IDLE_DOWN_GROUPS_NARROW 20
+static bool down_mostly_idle(long tasks, int G, int cols, long slots) {
   if (slots < 1 || tasks * G / slots < AOS_SK_MIN_GROUPS) return false;
-  return tasks * 20 < (tasks + slots - 1) / slots * slots * 11;
+  if (tasks * 20 >= (tasks + slots - 1) / slots * slots * 11) return false;
+  return idle_groups(tasks, G, slots) >=
+         (cols > AOS_NARROW_COLS ? AOS_IDLE_DOWN_GROUPS : AOS_IDLE_DOWN_GROUPS_NARROW);
 }
 
 /* Diagnostic (no counterpart in the reference): the prompt GEMMs' rules above for `tasks` tasks of G groups on
- * `slots` resident workgroups. rule 0: gate/up pieces (cols columns); 1: a single matrix's pieces; 2: q/k/v's pieces. */
+ * `slots` resident workgroups. rule 0: gate/up pieces (cols columns); 1: a single matrix's pieces; 2: q/k/v's pieces; 3: whether
+ * the down GEMM's shrink (cols columns) leaves its launch. */
 extern "C" int aoship_internal_prefill_rule(int rule, int tasks, int G, int cols, int slots) {
   if (tasks < 1 || G < 1 || cols < 0 || slots < 1) return set_err("aoship_internal_prefill_rule: bad arguments");
   switch (rule) {
     case 0: return gate_up_pieces(tasks, G, cols, slots);
     case 1: return gemm_pieces(tasks, G, slots, 3);
     case 2: return gemm_pieces(tasks, G, slots, 2);
+    case 3: return down_mostly_idle(tasks, G, cols, slots) ? 1 : 0;
   }
   return set_err("aoship_internal_prefill_rule: unknown rule");
 }
@@ -2064,7 +2082,7 @@ static void plan_mlp_prefill(aoship_layer *l, int T, const uint16_t *x, const ao
   const int s2 = gemm_pieces(tasks_dn, Wd.G, slots, 3);
   if (M.P.lora && l->prefill_fused_shrink) {
     M.fused_x = s1 == 1 && aos_gemm_shrink_fits(T, Wg.RB, cols_gu, 1) != 0;
-    M.fused_h = s2 == 1 && !((l->prefill_sk & 2) && down_mostly_idle(tasks_dn, Wd.G, slots)) &&
+    M.fused_h = s2 == 1 && !((l->prefill_sk & 2) && down_mostly_idle(tasks_dn, Wd.G, tc * rd, slots)) &&
                 aos_gemm_shrink_fits(T, Wd.RB, tc * rd, 0) != 0;
   }
   plan_tshrink(l, cv, M.P, x, perm, T, H, 0, 2, M.sx, M.fused_x);
