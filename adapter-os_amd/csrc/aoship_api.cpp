@@ -1962,9 +1962,19 @@ static bool down_mostly_idle(long tasks, int G, int cols, long slots) {
          (cols > AOS_NARROW_COLS ? AOS_IDLE_DOWN_GROUPS : AOS_IDLE_DOWN_GROUPS_NARROW);
 }
 
+/* Whether a projection alone gains from stream-K: its idle groups must pay for the partial sums' way through
+ * memory (about 20 groups; o of hidden = out, plain / stream-K):
+ *   5120: 900 tokens (30 idle groups) 112 / 109, 1100 tokens (24) 117 / 119, 1300 tokens (11) 125 / 132 us;
+ *   3584: 1300 tokens (22) 95 / 94, 1531 tokens (19) 94 / 98, 2048 tokens (7) 102 / 110, 2600 tokens (48) 168 /
+ *   144 us; 3072: 1531 tokens (21) 87 / 87, 2300 tokens (8) 97 / 104 us; 2048: 3000 tokens (8) 81 / 87 us. */
+#define AOS_SK_PROJ_GROUPS 20
+static bool proj_stream_k(long tasks, int G, long slots) {
+  return slots > 0 && idle_groups(tasks, G, slots) >= AOS_SK_PROJ_GROUPS;
+}
+
 /* Diagnostic (no counterpart in the reference): the prompt GEMMs' rules above for `tasks` tasks of G groups on
  * `slots` resident workgroups. rule 0: gate/up pieces (cols columns); 1: a single matrix's pieces; 2: q/k/v's pieces; 3: whether
- * the down GEMM's shrink (cols columns) leaves its launch. */
+ * the down GEMM's shrink (cols columns) leaves its launch; 4: whether a projection alone runs as stream-K. */
 extern "C" int aoship_internal_prefill_rule(int rule, int tasks, int G, int cols, int slots) {
   if (tasks < 1 || G < 1 || cols < 0 || slots < 1) return set_err("aoship_internal_prefill_rule: bad arguments");
   switch (rule) {
@@ -1972,6 +1982,7 @@ extern "C" int aoship_internal_prefill_rule(int rule, int tasks, int G, int cols
     case 1: return gemm_pieces(tasks, G, slots, 3);
     case 2: return gemm_pieces(tasks, G, slots, 2);
     case 3: return down_mostly_idle(tasks, G, cols, slots) ? 1 : 0;
+    case 4: return proj_stream_k(tasks, G, slots) ? 1 : 0;
   }
   return set_err("aoship_internal_prefill_rule: unknown rule");
 }
@@ -2795,7 +2806,7 @@ extern "C" int aoship_route_mlp_forward(aoship_router_t *r, const float *feature
  * launch over the matrices' GEMMs. The same code sizes the workspace (a Carve
  * over nullptr) and fills it. The k and v GEMMs of grouped-query attention are a few tasks each, which take as
  * long alone as q's: a 7B-shaped layer's q, k and v at 1531 tokens, 190 us as three launches. A single matrix
- * whose grid leaves part of its last round idle runs as stream-K. */
+ * whose grid leaves enough of its last round idle runs as stream-K (proj_stream_k). */
 struct ProjPrefill {
   PrefillPlan P;
   aos_tshrink_params sp;
@@ -2817,7 +2828,7 @@ static void plan_proj_prefill(aoship_layer *l, Carve &cv, const int *mods, int n
   const int S = gemm_pieces(tasks, l->mats[mods[0]].G, slots, nm > 1 ? 2 : 3);
   for (int i = 0; i < nm; ++i)
     plan_gemm(l, Q.P, Q.sp, l->mats[mods[i]], nullptr, xc, perm, perm, Tc, i, i, yc ? yc[i] : nullptr, Q.gp[i]);
-  if (S == 1 && nm == 1) plan_sk(l, cv, Q.gp[0], false);
+  if (S == 1 && nm == 1 && proj_stream_k(tasks, l->mats[mods[0]].G, slots)) plan_sk(l, cv, Q.gp[0], false);
   size_t floats = 0;
   for (int i = 0; i < nm; ++i) floats += piece_floats(Q.gp[i], S, false);
   plan_multi(Q.gp, nm, S, false, cv.b.take<float>(floats), Q.mu);

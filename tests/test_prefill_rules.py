@@ -36,3 +36,12 @@ def test_pieces_fit_one_round_and_keep_their_groups(rule, slots):
     (1800, 2048, 5632, 256, 0), (4096, 896, 4864, 256, 0), (3000, 1024, 2816, 512, 0), (1500, 3584, 18944, 256, 0)])
 def test_idle_down(T, H, I, cols, want):
     assert aoship.prefill_rule("idle_down", _tasks(T, H, 8), I // 64, cols, 256) == want
+
+
+# (tokens, out, in): o as stream-K where its idle groups pay for the partial sums
+@pytest.mark.parametrize("T,out,inp,want", [
+    (900, 5120, 5120, 1), (1300, 3584, 3584, 1), (2600, 3584, 3584, 1), (1531, 3072, 3072, 1),
+    (1300, 5120, 5120, 0), (1531, 3584, 3584, 0), (2048, 3584, 3584, 0), (2300, 3072, 3072, 0), (3000, 2048, 2048, 0),
+    (2048, 4096, 4096, 0)])
+def test_projection_stream_k(T, out, inp, want):
+    assert aoship.prefill_rule("proj_stream_k", _tasks(T, out, 8), inp // 64, 0, 256) == want
