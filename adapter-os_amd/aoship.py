@@ -183,7 +183,7 @@ def decode_geometry(kind: int, out: int, inp: int, T: int, wr_pin: int = 0, ks_p
     return decode_launch(kind, out, inp, T, wr_pin, ks_pin, n, rpad)[1:]
 
 
-PREFILL_RULES = ("gate_up_pieces", "single_pieces", "qkv_pieces", "idle_down", "proj_stream_k")
+PREFILL_RULES = ("gate_up_pieces", "single_pieces", "qkv_pieces", "idle_down", "proj_stream_k", "one_launch")
 
 
 def prefill_rule(rule: str, tasks: int, G: int, cols: int, slots: int) -> int:

@@ -1972,17 +1972,35 @@ static bool proj_stream_k(long tasks, int G, long slots) {
   return slots > 0 && idle_groups(tasks, G, slots) >= AOS_SK_PROJ_GROUPS;
 }
 
+/* Whether whole tasks of projections sharing x (tasks[0, n)) run as one launch: unless that saves no round of
+ * the resident workgroups and leaves its own last round at most half full, where each matrix in a launch of its
+ * own spreads its tasks more evenly (q, k and v of 192 tasks each, hidden 4096, 1531 tokens: 278 us as one launch of
+ * 2 1/4 rounds, 269 us as three of 3/4; of 240 tasks each, 1800 tokens: 304 and 307 us). */
+static bool proj_one_launch(const long *tasks, int n, long slots) {
+  if (slots < 1 || n < 2) return true;
+  long sum = 0, rounds = 0;
+  for (int i = 0; i < n; ++i) {
+    sum += tasks[i];
+    rounds += (tasks[i] + slots - 1) / slots;
+  }
+  const long last = sum % slots;
+  return (sum + slots - 1) / slots < rounds || last == 0 || 2 * last > slots;
+}
+
 /* Diagnostic (no counterpart in the reference): the prompt GEMMs' rules above for `tasks` tasks of G groups on
  * `slots` resident workgroups. rule 0: gate/up pieces (cols columns); 1: a single matrix's pieces; 2: q/k/v's pieces; 3: whether
- * the down GEMM's shrink (cols columns) leaves its launch; 4: whether a projection alone runs as stream-K. */
+ * the down GEMM's shrink (cols columns) leaves its launch; 4: whether a projection alone runs as stream-K; 5:
+ * whether q, k and v of `tasks`, G and cols tasks run as one launch. */
 extern "C" int aoship_internal_prefill_rule(int rule, int tasks, int G, int cols, int slots) {
   if (tasks < 1 || G < 1 || cols < 0 || slots < 1) return set_err("aoship_internal_prefill_rule: bad arguments");
+  const long t3[3] = {tasks, G, cols};
   switch (rule) {
     case 0: return gate_up_pieces(tasks, G, cols, slots);
     case 1: return gemm_pieces(tasks, G, slots, 3);
     case 2: return gemm_pieces(tasks, G, slots, 2);
     case 3: return down_mostly_idle(tasks, G, cols, slots) ? 1 : 0;
     case 4: return proj_stream_k(tasks, G, slots) ? 1 : 0;
+    case 5: return proj_one_launch(t3, 3, slots) ? 1 : 0;
   }
   return set_err("aoship_internal_prefill_rule: unknown rule");
 }
@@ -2803,7 +2821,7 @@ extern "C" int aoship_route_mlp_forward(aoship_router_t *r, const float *feature
 }
 
 /* Prefill chunk of projections sharing x: the group plan, one tile shrink over every module, one
- * launch over the matrices' GEMMs. The same code sizes the workspace (a Carve
+ * launch over the matrices' GEMMs (or one each: proj_one_launch). The same code sizes the workspace (a Carve
  * over nullptr) and fills it. The k and v GEMMs of grouped-query attention are a few tasks each, which take as
  * long alone as q's: a 7B-shaped layer's q, k and v at 1531 tokens, 190 us as three launches. A single matrix
  * whose grid leaves enough of its last round idle runs as stream-K (proj_stream_k). */
@@ -2812,6 +2830,7 @@ struct ProjPrefill {
   aos_tshrink_params sp;
   aos_gemm_params gp[3];
   aos_gemm_multi_params mu;
+  bool one; /* mu's launch (and its finish launch), else a launch per matrix */
 };
 
 static void plan_proj_prefill(aoship_layer *l, Carve &cv, const int *mods, int nm, const uint16_t *xc, int Tc,
@@ -2823,12 +2842,16 @@ static void plan_proj_prefill(aoship_layer *l, Carve &cv, const int *mods, int n
   const uint16_t *perm = Q.P.lora ? Q.P.gp.perm : nullptr;
   plan_tshrink(l, cv, Q.P, xc, perm, Tc, in, 0, nm, Q.sp);
   const long slots = aos_gemm_sk_slots(0);
-  long tasks = 0;
-  for (int i = 0; i < nm; ++i) tasks += gemm_tasks(Tc, l->mats[mods[i]].RB, false);
-  const int S = gemm_pieces(tasks, l->mats[mods[0]].G, slots, nm > 1 ? 2 : 3);
+  long tasks[3] = {0, 0, 0}, sum = 0;
+  for (int i = 0; i < nm; ++i) {
+    tasks[i] = gemm_tasks(Tc, l->mats[mods[i]].RB, false);
+    sum += tasks[i];
+  }
+  const int S = gemm_pieces(sum, l->mats[mods[0]].G, slots, nm > 1 ? 2 : 3);
   for (int i = 0; i < nm; ++i)
     plan_gemm(l, Q.P, Q.sp, l->mats[mods[i]], nullptr, xc, perm, perm, Tc, i, i, yc ? yc[i] : nullptr, Q.gp[i]);
-  if (S == 1 && nm == 1 && proj_stream_k(tasks, l->mats[mods[0]].G, slots)) plan_sk(l, cv, Q.gp[0], false);
+  if (S == 1 && nm == 1 && proj_stream_k(sum, l->mats[mods[0]].G, slots)) plan_sk(l, cv, Q.gp[0], false);
+  Q.one = S > 1 || (nm > 1 && proj_one_launch(tasks, nm, slots));
   size_t floats = 0;
   for (int i = 0; i < nm; ++i) floats += piece_floats(Q.gp[i], S, false);
   plan_multi(Q.gp, nm, S, false, cv.b.take<float>(floats), Q.mu);
@@ -2927,12 +2950,14 @@ static int proj_multi(aoship_layer *l, const int *mods, int nm, const uint16_t *
       plan_proj_prefill(l, cv, mods, nm, x + (size_t)t0 * in, Tc, rings + t0, yc, Q);
       if (launch_gplan(l, Q.P)) return -1;
       if (launch_tshrink(l, Q.sp, KS_PSHRINK_X)) return -1;
-      if (nm == 1 && Q.mu.S == 1) {
-        if (Q.gp[0].sk_nwg) Q.gp[0].gen = next_gen(&l->gen);
+      if (Q.one) {
+        if (launch_multi(l, Q.mu, 0, KS_GEMM_PROJ, KS_GEMM_PROJF, "q4 gemm")) return -1;
+        continue;
+      }
+      for (int i = 0; i < nm; ++i) {
+        if (Q.gp[i].sk_nwg) Q.gp[i].gen = next_gen(&l->gen);
         aos_launch_ctx cg = launch_ctx(l, KS_GEMM_PROJ);
-        if (launch_err(aos_launch_gemm(&Q.gp[0], 0, &cg), "q4 gemm")) return -1;
-      } else if (launch_multi(l, Q.mu, 0, KS_GEMM_PROJ, KS_GEMM_PROJF, "q4 gemm")) {
-        return -1;
+        if (launch_err(aos_launch_gemm(&Q.gp[i], 0, &cg), "q4 gemm")) return -1;
       }
     }
     return 0;

@@ -45,3 +45,11 @@ def test_idle_down(T, H, I, cols, want):
     (2048, 4096, 4096, 0)])
 def test_projection_stream_k(T, out, inp, want):
     assert aoship.prefill_rule("proj_stream_k", _tasks(T, out, 8), inp // 64, 0, 256) == want
+
+
+# (q, k and v tasks): one launch unless that saves no round and leaves its own last one at most half full
+@pytest.mark.parametrize("q,k,v,want", [
+    (168, 24, 24, 1), (240, 32, 32, 1), (240, 240, 240, 1), (256, 256, 256, 1), (384, 384, 384, 1),
+    (192, 192, 192, 0), (448, 448, 448, 0)])
+def test_qkv_one_launch(q, k, v, want):
+    assert aoship.prefill_rule("one_launch", q, k, v, 256) == want
