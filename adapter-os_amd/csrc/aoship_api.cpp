@@ -1974,8 +1974,8 @@ static bool proj_stream_k(long tasks, int G, long slots) {
 
 /* Whether whole tasks of projections sharing x (tasks[0, n)) run as one launch: unless that saves no round of
  * the resident workgroups and leaves its own last round at most half full, where each matrix in a launch of its
- * own spreads its tasks more evenly (q, k and v of 192 tasks each, hidden 4096, 1531 tokens: 278 us as one launch of
- * 2 1/4 rounds, 269 us as three of 3/4; of 240 tasks each, 1800 tokens: 304 and 307 us). */
+ * own spreads its tasks more evenly (q, k and v of 192 tasks each, hidden 4096, 1531 tokens: 273 us as one launch of
+ * 2 1/4 rounds, 259 us as three of 3/4; of 240 tasks each, 1800 tokens: 304 and 307 us). */
 static bool proj_one_launch(const long *tasks, int n, long slots) {
   if (slots < 1 || n < 2) return true;
   long sum = 0, rounds = 0;

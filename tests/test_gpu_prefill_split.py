@@ -116,3 +116,28 @@ def test_projections(hip, T, finish):
         ref = oracle_proj(cid, name, xf[sample], rings[sample])
         ratio = assert_parity(f"split {name} T={T}", W.bf16_bits_to_f32(got).reshape(T, -1)[sample], ref)
         assert ratio <= REL_TOL, f"{name}: {ratio:.4g}"
+
+
+def test_qkv_in_launches_of_their_own(hip):
+    """q, k and v of 192 tasks each (2 1/4 rounds of 256 as one launch): a launch per matrix, against 64-bit
+    arithmetic (two roundings to bfloat16: the scaled shrink and the result) and run to run."""
+    import torch
+
+    from test_gpu_decode_direct import TOL, _bf16, _build, _err, _linear, _rings
+
+    rng = np.random.default_rng(17)
+    T, inp, out = 1531, 512, 4096
+    layer, ads, base, lora = _build(hip, rng, {m: (out, inp) for m in ("q_proj", "k_proj", "v_proj")}, 5, 16)
+    rings, coef = _rings(hip, rng, T, 5, 3)
+    x = _bf16(rng.standard_normal((T, inp))).cuda()
+    r = _dev(rings.view(np.uint8))
+    layer.set_profiling(True)
+    outs = [[torch.empty((T, out), dtype=torch.bfloat16, device="cuda") for _ in range(3)] for _ in range(2)]
+    for o in outs:
+        layer.qkv_forward(x, r, *o)
+    torch.cuda.synchronize()
+    assert _launches(layer, "q4_gemm_proj") == 6
+    assert all(torch.equal(a, b) for a, b in zip(*outs)), "run-to-run outputs differ"
+    xf = x.double().cpu().numpy()
+    for m, o in zip(("q_proj", "k_proj", "v_proj"), outs[0]):
+        assert _err(o, _linear(base, lora, m, xf, coef)) <= TOL, m
