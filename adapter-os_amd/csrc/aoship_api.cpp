@@ -1240,9 +1240,8 @@ static int gemv_splits(int RB, int G, int T, int W, int waves_target) {
  * reduction's LDS. */
 static size_t gemv_lds_x(int T, int G, int ks) { return 128 + (size_t)T * ceil_div(G, ks) * 136; }
 
-/* Row-split geometry (3 or more tokens with x staged: a gate/up launch of at most 8 tokens over a wide adapter
- * table, fewer than AOS_GEMV_DX_MIN_G K groups, and pinned shapes; the 8-wave rule serves pinned shapes
- * alone): the waves of a workgroup take different row blocks over
+/* Row-split geometry (3 or more tokens with x staged: wide or large launches of at most 8 tokens, fewer than
+ * AOS_GEMV_DX_MIN_G K groups, and pinned shapes; see gemv_direct_waves): the waves of a workgroup take different row blocks over
  * one K split, so the x slice staged in LDS serves WR row blocks instead of one (x staged over a
  * whole launch scales with RB / WR). The rules below are the best of sweeps over (WR, ks) on
  * MI355X (the 7B MLP at 4, 8 and 32 tokens, the 3B projections at 32): the fewest K splits that
@@ -1309,8 +1308,18 @@ static void gemv_geometry_rows(int RB, int G, int T, bool swiglu, int W, aos_gem
  *   down, 32B shape at 3, 8 and 16 tokens: 61, 115, 205 / 58, 100, 140 / 66, 109, 145 us (20 adapters, 7B shape
  *   at 12 tokens: 61 / 46 / 43 us, hence its wider line);
  *   gate/up, hidden 4096, intermediate 11008, at 12 and 16 tokens: 202, 242 / 140, 157 / 218, 251 us.
- * A gate/up launch of at most 8 tokens over a wide table stays staged: the 7B and 32B shapes at 8 tokens take
- * 167 and 246 us staged, 185 and 308 us here. */
+ * Projections of at most 8 tokens whose waves would be a single split of each row block take the wide launch from
+ * AOS_GEMV_DX_COLS_PROJ8 columns on (o of hidden 4096, 128 row blocks, 12 adapters of rank 64, 8 tokens: 20 us
+ * staged, 16 / 21 us here; at 32 tokens the q/k/v launch would lose, 41 / 37 us).
+ * A wave streams at most AOS_GEMV_DX_MAX_GROUPS groups (down of the 32B shape, 54 groups a wave else, at 9 and 16
+ * tokens: 36, 47 us staged / 34, 39 / 37, 51 us).
+ * At most 8 tokens stay staged
+ *  - in a gate/up launch over a wide table: the 7B and 32B shapes at 8 tokens take 167 and 246 us staged, 185 and
+ *    308 us here;
+ *  - in large launches, where x, re-read for every row block, is the bound (about 2.5 K groups of row blocks per
+ *    ns, against 3.2 staged): down of the 32B shape (69k groups) at 3 and 8 tokens 29 and 31 us staged, 31 and 34 us
+ *    here, of hidden 8192 and intermediate 28672 (115k) 36 and 38 us staged, 47 and 50 us here, its gate/up
+ *    launch at 3 tokens 84 and 87 us; of hidden 6144 (49k) 20 us both. */
 #define AOS_GEMV_DX_MIN_T 3
 #define AOS_GEMV_DX_MIN_G 8
 #define AOS_GEMV_DX_WAVES 1024
@@ -1319,24 +1328,40 @@ static void gemv_geometry_rows(int RB, int G, int T, bool swiglu, int W, aos_gem
 #define AOS_GEMV_DX_COLS_DOWN 1280
 #define AOS_GEMV_DX_WAVES_WIDE 2048
 #define AOS_GEMV_DX_WAVES_WIDE_DOWN 1536
+#define AOS_GEMV_DX_COLS_PROJ8 512
+#define AOS_GEMV_DX_MAX_GROUPS 48
+#define AOS_GEMV_DX_LARGE_DOWN 60000     /* row blocks times K groups */
+#define AOS_GEMV_DX_LARGE_GATE_UP 100000 /* ... of each of the two matrices */
+#define AOS_GEMV_DX_LARGE_MAX 200000     /* past it (hidden 16384) the staged launch's 19 splits outgrow the scratch */
 
 /* The decode GEMV launches, as the diagnostics number them. */
 enum { GV_GATE_UP = 0, GV_DOWN = 1, GV_PROJ = 2 };
 
-/* Waves of a decode GEMV launch that reads x itself, 0 for one that stages x in LDS. n, rpad: the adapter
- * table's size and the widest padded rank of the launch's modules; wr_force, ks_force: a pinned (staged)
- * shape. */
-static int gemv_direct_waves(int kind, int G, int T, int n, int rpad, int wr_force, int ks_force) {
+/* Waves of a decode GEMV launch that reads x itself, 0 for one that stages x in LDS. RB: the row blocks of its
+ * matrices (of one of the pair); n, rpad: the adapter table's size and the widest padded rank of the launch's
+ * modules; wr_force, ks_force: a pinned (staged) shape. */
+static int gemv_direct_waves(int kind, int RB, int G, int T, int n, int rpad, int wr_force, int ks_force) {
   if (T < AOS_GEMV_DX_MIN_T || G < AOS_GEMV_DX_MIN_G || wr_force > 0 || ks_force > 0) return 0;
-  if (kind == GV_GATE_UP && T <= 8 && n * rpad > AOS_GEMV_DX_COLS) return 0;
   const int cols = std::min(n, 8 * T) * rpad;
-  if (kind == GV_DOWN) return cols > AOS_GEMV_DX_COLS_DOWN ? AOS_GEMV_DX_WAVES_WIDE_DOWN : AOS_GEMV_DX_WAVES;
-  if (cols > AOS_GEMV_DX_COLS) return AOS_GEMV_DX_WAVES_WIDE;
-  return kind == GV_PROJ ? AOS_GEMV_DX_WAVES_PROJ : AOS_GEMV_DX_WAVES;
+  const long groups = (long)RB * G;
+  const bool large = T <= 8 && groups <= AOS_GEMV_DX_LARGE_MAX &&
+                     groups > (kind == GV_DOWN ? AOS_GEMV_DX_LARGE_DOWN : AOS_GEMV_DX_LARGE_GATE_UP);
+  if (kind == GV_GATE_UP) {
+    if ((T <= 8 && n * rpad > AOS_GEMV_DX_COLS) || large) return 0;
+    return cols > AOS_GEMV_DX_COLS ? AOS_GEMV_DX_WAVES_WIDE : AOS_GEMV_DX_WAVES;
+  }
+  if (kind == GV_DOWN) {
+    if (cols > AOS_GEMV_DX_COLS_DOWN) return AOS_GEMV_DX_WAVES_WIDE_DOWN;
+    return large ? 0 : AOS_GEMV_DX_WAVES;
+  }
+  const bool one_split = 4 * RB >= AOS_GEMV_DX_WAVES_PROJ;
+  if (cols > (T <= 8 && one_split ? AOS_GEMV_DX_COLS_PROJ8 : AOS_GEMV_DX_COLS)) return AOS_GEMV_DX_WAVES_WIDE;
+  return AOS_GEMV_DX_WAVES_PROJ;
 }
 
 static void gemv_geometry_direct(int RB, int G, int T, bool swiglu, bool lora, aos_gemv_params &g, int waves) {
   int ks = ceil_div(waves, 4 * RB);
+  if ((long)RB * G <= AOS_GEMV_DX_LARGE_MAX) ks = std::max(ks, ceil_div(G, 4 * AOS_GEMV_DX_MAX_GROUPS));
   if (ks > G / 8) ks = G / 8;
   g.dx = 1;
   g.wr = 1;
@@ -1391,7 +1416,7 @@ static void gemv_geometry(int RB, int G, int T, bool swiglu, bool lora, aos_gemv
  * grid, in 4-wave workgroups like the rest of that grid. */
 static void gemv_launch_geometry(int kind, int RB, int G, int T, int n, int rpad, int wr_force, int ks_force,
                                  aos_gemv_params &g) {
-  const int dx = gemv_direct_waves(kind, G, T, n, rpad, wr_force, ks_force);
+  const int dx = gemv_direct_waves(kind, RB, G, T, n, rpad, wr_force, ks_force);
   if (dx > 0) {
     gemv_geometry_direct(RB, G, T, kind == GV_GATE_UP, rpad > 0, g, dx);
     return;
