@@ -3253,7 +3253,8 @@ static size_t attn_part_rows(const aoship_model_config_t &c, int T) {
 /* Prompts take the matrix-core attention from AOS_ATTN_PREFILL_ROWS (token, head) rows on: below, its
  * 128-token workgroups are too few to fill the chip and the wave per (token, head) is as fast. Measured on a
  * whole one-layer call, 28 heads of 128, fresh cache: 64 tokens 288 against 286 us, 96 tokens 324 against
- * 338, 256 tokens 363 against 413, 1900 tokens 528 against 2710. */
+ * 338, 256 tokens 363 against 413, 1900 tokens 528 against 2710. Long caches only widen it (the launch alone, 74
+ * tokens after 8000 positions: 421 against 1334 us), and so do few heads (1 head of 2048 tokens: 112 against 186). */
 static bool attn_prefill(const aoship_model *m, int T) {
   return T > 1 && (long long)T * m->cfg.num_heads >= AOS_ATTN_PREFILL_ROWS &&
          aos_attn_prefill_fits(m->cfg.head_dim, m->cfg.max_seq);

@@ -560,9 +560,9 @@ __global__ void __launch_bounds__(64) aos_attn_merge_kernel(aos_attn_params p) {
  * by the two row bits a transposed read spans.
  *
  * Bound by the matrix cores (three MFMAs for each of the plain bfloat16 products) and the float32
- * exponentials and splits between them. One layer of 1900 tokens, 28 heads of 128, 4 key/value heads: 132 us
+ * exponentials and splits between them. One layer of 1900 tokens, 28 heads of 128, 4 key/value heads: 128 us
  * (26 GFLOP of products over the causal half; 82 GFLOP executed, with the pieces and the masked parts of the
- * edge tiles: 620 TFLOP/s) against 2452 us for the wave per (token, head), which reads every visible key and
+ * edge tiles: 640 TFLOP/s) against 2452 us for the wave per (token, head), which reads every visible key and
  * value row once per token. */
 constexpr int PA_BQ = 128; /* tokens per workgroup */
 constexpr int PA_BK = 64;  /* positions per tile */

@@ -273,8 +273,9 @@ int aoship_mlp_forward(aoship_layer_t *layer, const aoship_bf16_t *x, int T,
  * of 33 MiB (28.75 MiB of workspace) that each GPU holds until the process ends; a layer and
  * token count whose workspace does not fit is rejected with an error (-1), as is T > 32. Makes no
  * hipMalloc, hipFree or other allocating call. The array keeps the last call's contents; calls that
- * overlap on one GPU (on different streams) share it and race: serialise them. Output equals
- * aoship_mlp_forward's bit for bit. Returns 0 / -1. */
+ * overlap on one GPU (on different streams) share it and race: serialise them. The stamps that order
+ * the workgroups of a launch are launch arguments: a captured call is good for one replay, since a second
+ * would find the first one's stamps. Output equals aoship_mlp_forward's bit for bit. Returns 0 / -1. */
 int aoship_mlp_forward_noalloc(aoship_layer_t *layer, const aoship_bf16_t *x, int T,
                                const aoship_ring_t *rings, aoship_bf16_t *y);
 
