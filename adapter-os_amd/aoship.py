@@ -147,7 +147,7 @@ def lib():
         L.aoship_internal_layer_last_perm.restype = C.c_int
         L.aoship_internal_layer_last_perm.argtypes = [_P, _P, C.c_int]
         L.aoship_internal_prefill_rule.restype = C.c_int
-        L.aoship_internal_prefill_rule.argtypes = [C.c_int] * 5
+        L.aoship_internal_prefill_rule.argtypes = [C.c_int] * 7
         L.aoship_internal_route_tokens.restype = C.c_int
         L.aoship_internal_route_tokens.argtypes = [C.c_int, C.c_int, C.c_int]
         L.aoship_internal_model_workspace.restype = C.c_int
@@ -186,9 +186,9 @@ def decode_geometry(kind: int, out: int, inp: int, T: int, wr_pin: int = 0, ks_p
 PREFILL_RULES = ("gate_up_pieces", "single_pieces", "qkv_pieces", "idle_down", "proj_stream_k", "one_launch")
 
 
-def prefill_rule(rule: str, tasks: int, G: int, cols: int, slots: int) -> int:
+def prefill_rule(rule: str, tasks: int, G: int, cols: int, slots: int, tiles: int = 1, rpad: int = 0) -> int:
     """A prompt GEMM rule's choice (see aoship_internal_prefill_rule)."""
-    r = lib().aoship_internal_prefill_rule(PREFILL_RULES.index(rule), tasks, G, cols, slots)
+    r = lib().aoship_internal_prefill_rule(PREFILL_RULES.index(rule), tasks, G, cols, slots, tiles, rpad)
     if r < 0:
         raise AosError(last_error())
     return r

@@ -1943,24 +1943,30 @@ static int gemm_pieces(long tasks, int G, long slots, int least) {
   return s < least ? 1 : (int)s;
 }
 
-/* The same for the gate/up GEMM. In pieces it loses the x shrink (over cols columns of a tile's union) that whole
- * tasks carry in their launch's idle slots, and needs a finish launch; both grow with the tasks, so that beyond
- * slots / 7 tasks (slots / 5 over few columns) the groups taken off each task's chain must pay for them. MLP of
- * (hidden, intermediate), whole / in pieces:
- *   44 tasks of 16 groups in 2 (1024, 2816; 256 tokens) 129 / 112 us, 176 tasks in 2 (1024 tokens) 137 / 165 us;
- *   88 tasks in 2 over 64 columns (450 tokens) 106 / 94, 154 tasks (800 tokens) 100 / 107 us;
- *   88 tasks of 32 in 4 (2048, 5632; 200 tokens) 134 / 122, 132 in 3 (384 tokens) 156 / 168 us;
- *   128 tasks of 48 in 4 (3072, 8192; 256 tokens) 154 / 148, 192 in 2 (384 tokens) 180 / 202 us;
- *   172 tasks of 64 in 2 (4096, 11008; 256 tokens) 192 / 215 us;
- *   148 tasks of 56 in 3 (7B, 96 tokens) 159 / 158, 216 of 80 in 2 (32B, 96 tokens) 241 / 232 us. */
-#define AOS_NARROW_COLS 64      /* few columns, up to */
-#define AOS_SPLIT_GU_GROUPS4 24 /* groups off a task's chain, at least, in 4 or more pieces */
-#define AOS_SPLIT_GU_GROUPS 37  /* ... in fewer */
-static int gate_up_pieces(long tasks, int G, int cols, long slots) {
+/* The same for the gate/up GEMM of `tiles` token tiles. In pieces it loses the x shrink (over cols columns of a
+ * tile's union, rpad each adapter) that whole tasks carry in their launch's idle slots, and needs a finish launch.
+ * Both grow with the tiles and the weight blocks while the second piece is all that their tasks leave room for, so
+ * that from 3 tiles on tasks of two pieces run whole; but not over many or long adapters, whose expand the finish
+ * launch spreads better. MLP of (hidden, intermediate), whole / in pieces:
+ *   16 adapters of rank 16 in 6 sets: (1024, 2816) at 700 tokens (132 tasks) 139 / 154, 1000 tokens (176) 137 / 156,
+ *   (1536, 4096) at 1000 tokens (256) 152 / 183 us; each token its own set: 140 / 135, 142 / 146, 162 / 178 us;
+ *   100 of rank 16: (2048, 5632) at 640 tokens (220 tasks) 306 / 418 us; 20 of rank 32: 211 / 212 us;
+ *   24 of rank 48: (2048, 5632) at 512 tokens (176 tasks) 228 / 217 us; 150 of rank 16: 352 / 293 us;
+ *   2 tiles: 16 adapters of rank 16, (2048, 11008) at 200 tokens (172 tasks) 156 / 156, 16 of rank 64 209 / 194 us;
+ *   1 tile: (5120, 27648) at 75 tokens (216 tasks) 246 / 241 us, 148 tasks of 56 groups 169 / 166 us.
+ * Of 1472 calls measured (14 shapes, 40 to 1400 tokens, 1 to 200 adapters) one is over 1% slower than in pieces (3%,
+ * 20 adapters of rank 32). */
+#define AOS_GU_WHOLE_TILES 3
+#define AOS_GU_WHOLE_COLS 2048
+#define AOS_GU_WHOLE_COLS_LONG 768 /* adapters of more than 32 columns */
+static int gate_up_pieces(long tasks, int tiles, int G, int cols, int rpad, long slots) {
   const int s = gemm_pieces(tasks, G, slots, 2);
-  if (s == 1 || tasks * (cols > AOS_NARROW_COLS ? 7 : 5) <= slots) return s;
-  return G - (G + s - 1) / s >= (s >= 4 ? AOS_SPLIT_GU_GROUPS4 : AOS_SPLIT_GU_GROUPS) ? s : 1;
+  const bool whole = tiles >= AOS_GU_WHOLE_TILES && 3 * tasks > slots &&
+                     cols <= (rpad > 32 ? AOS_GU_WHOLE_COLS_LONG : AOS_GU_WHOLE_COLS);
+  return whole ? 1 : s;
 }
+
+#define AOS_NARROW_COLS 64 /* few columns of a union, up to */
 
 /* K groups per workgroup for which the last round of a plain grid leaves a slot idle, on average. */
 static double idle_groups(long tasks, int G, long slots) {
@@ -2013,14 +2019,15 @@ static bool proj_one_launch(const long *tasks, int n, long slots) {
 }
 
 /* Diagnostic (no counterpart in the reference): the prompt GEMMs' rules above for `tasks` tasks of G groups on
- * `slots` resident workgroups. rule 0: gate/up pieces (cols columns); 1: a single matrix's pieces; 2: q/k/v's pieces; 3: whether
+ * `slots` resident workgroups. rule 0: gate/up pieces (tiles token tiles,
+ * cols columns, rpad an adapter); 1: a single matrix's pieces; 2: q/k/v's pieces; 3: whether
  * the down GEMM's shrink (cols columns) leaves its launch; 4: whether a projection alone runs as stream-K; 5:
  * whether q, k and v of `tasks`, G and cols tasks run as one launch. */
-extern "C" int aoship_internal_prefill_rule(int rule, int tasks, int G, int cols, int slots) {
-  if (tasks < 1 || G < 1 || cols < 0 || slots < 1) return set_err("aoship_internal_prefill_rule: bad arguments");
+extern "C" int aoship_internal_prefill_rule(int rule, int tasks, int G, int cols, int slots, int tiles, int rpad) {
+  if (tasks < 1 || G < 1 || cols < 0 || slots < 1 || tiles < 1 || rpad < 0) return set_err("aoship_internal_prefill_rule: bad arguments");
   const long t3[3] = {tasks, G, cols};
   switch (rule) {
-    case 0: return gate_up_pieces(tasks, G, cols, slots);
+    case 0: return gate_up_pieces(tasks, tiles, G, cols, rpad, slots);
     case 1: return gemm_pieces(tasks, G, slots, 3);
     case 2: return gemm_pieces(tasks, G, slots, 2);
     case 3: return down_mostly_idle(tasks, G, cols, slots) ? 1 : 0;
@@ -2131,8 +2138,8 @@ static void plan_mlp_prefill(aoship_layer *l, int T, const uint16_t *x, const ao
    * last round, else a launch of its own (K split into slices) */
   M.fused_x = M.fused_h = false;
   const long slots = aos_gemm_sk_slots(0), tasks_dn = gemm_tasks(T, Wd.RB, false);
-  const int tc = M.P.tu_cap, rd = tall[2].rpad, cols_gu = tc * std::max(tall[0].rpad, tall[1].rpad);
-  const int s1 = gate_up_pieces(gemm_tasks(T, Wg.RB, true), Wg.G, cols_gu, aos_gemm_sk_slots(1));
+  const int tc = M.P.tu_cap, rd = tall[2].rpad, rgu = std::max(tall[0].rpad, tall[1].rpad), cols_gu = tc * rgu;
+  const int s1 = gate_up_pieces(gemm_tasks(T, Wg.RB, true), M.P.mtiles, Wg.G, cols_gu, rgu, aos_gemm_sk_slots(1));
   const int s2 = gemm_pieces(tasks_dn, Wd.G, slots, 3);
   if (M.P.lora && l->prefill_fused_shrink) {
     M.fused_x = s1 == 1 && aos_gemm_shrink_fits(T, Wg.RB, cols_gu, 1) != 0;

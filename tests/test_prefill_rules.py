@@ -10,14 +10,16 @@ def _tasks(T, rows, per):
     return -(-T // 128) * -(-rows // (32 * per))
 
 
-# (tokens, hidden, intermediate, columns of the union, pieces): whole where pieces measured slower
-@pytest.mark.parametrize("T,H,I,cols,want", [
-    (75, 3584, 18944, 256, 3), (128, 5120, 27648, 4096, 2), (200, 2048, 5632, 256, 4), (256, 3072, 8192, 256, 4),
-    (256, 1024, 2816, 512, 2), (450, 1024, 2816, 64, 2),
-    (450, 1024, 2816, 512, 1), (800, 1024, 2816, 64, 1), (1024, 1024, 2816, 512, 1), (384, 2048, 5632, 256, 1),
-    (384, 3072, 8192, 256, 1), (256, 4096, 11008, 768, 1), (2048, 3584, 18944, 256, 1), (75, 448, 512, 64, 1)])
-def test_gate_up_pieces(T, H, I, cols, want):
-    assert aoship.prefill_rule("gate_up_pieces", _tasks(T, I, 4), H // 64, cols, 512) == want
+# (tokens, hidden, intermediate, adapters, rank, pieces): whole where pieces measured slower
+@pytest.mark.parametrize("T,H,I,n,r,want", [
+    (75, 3584, 18944, 16, 16, 3), (128, 5120, 27648, 64, 64, 2), (105, 1280, 9600, 37, 16, 2), (200, 2048, 11008, 16, 64, 2),
+    (256, 3072, 8192, 16, 16, 4), (450, 1024, 2816, 200, 16, 2), (700, 1024, 2816, 16, 16, 2), (512, 2048, 5632, 64, 64, 2),
+    (512, 2048, 5632, 24, 48, 2), (640, 2048, 5632, 150, 16, 2),
+    (1000, 1024, 2816, 16, 16, 1), (1000, 1536, 4096, 37, 16, 1), (640, 2048, 5632, 100, 16, 1), (640, 2048, 5632, 128, 8, 1),
+    (350, 3072, 8192, 12, 64, 1), (1000, 1024, 4096, 8, 8, 1), (2048, 3584, 18944, 16, 16, 1), (75, 448, 512, 8, 8, 1)])
+def test_gate_up_pieces(T, H, I, n, r, want):
+    got = aoship.prefill_rule("gate_up_pieces", _tasks(T, I, 4), H // 64, n * r, 512, -(-T // 128), r)
+    assert got == want
 
 
 @pytest.mark.parametrize("rule,slots", [("gate_up_pieces", 512), ("single_pieces", 256), ("qkv_pieces", 256)])
