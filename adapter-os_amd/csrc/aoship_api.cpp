@@ -1966,8 +1966,6 @@ static int gate_up_pieces(long tasks, int tiles, int G, int cols, int rpad, long
   return whole ? 1 : s;
 }
 
-#define AOS_NARROW_COLS 64 /* few columns of a union, up to */
-
 /* K groups per workgroup for which the last round of a plain grid leaves a slot idle, on average. */
 static double idle_groups(long tasks, int G, long slots) {
   const long last = tasks % slots;
@@ -1975,22 +1973,15 @@ static double idle_groups(long tasks, int G, long slots) {
 }
 
 /* Whether a down GEMM of these tasks leaves over 45% of its grid's last round idle and stream-K could
- * share it: then its shrink (over cols columns of a tile's union) takes a launch of its own rather than that
- * round. That launch and the sharing cost as much as 45 to 70 groups of the chain, less over few columns. MLP of
- * (hidden, intermediate) with the shrink in the launch / with stream-K:
- *   7B, 1100 tokens (126 tasks on 256 slots, 150 idle groups) 640 / 623 us, 800 tokens (183) 576 / 518 us;
- *   (3072, 8192), 1024 tokens (80) 307 / 291, 1100 tokens (74) 307 / 305, 1300 tokens (62) 335 / 342 us;
- *   (2048, 5632), 256 columns, 1300 tokens (58) 253 / 241, 1800 tokens (47) 266 / 281 us; 64 columns, 2048
- *   tokens (44) 242 / 234 us;
- *   (896, 4864), 4096 tokens (38) 254 / 273, over 64 columns 235 / 231; (1024, 2816), 3000 tokens (28) 187 / 204,
- *   over 64 columns 171 / 163 us. */
-#define AOS_IDLE_DOWN_GROUPS 55
-#define AOS_IDLE_DOWN_GROUPS_NARROW 20
-static bool down_mostly_idle(long tasks, int G, int cols, long slots) {
+ * share it: then its shrink takes a launch of its own rather than that round. Measured both ways on 2174 MLPs (hidden
+ * 768 to 4096, intermediate 2048 to 18944, 700 to 4100 tokens in 1 to 24 sets of 2 to 64 adapters, 20 idle groups or
+ * more): stream-K is faster by over 1% in 1772 (mean 7%, at most 47%; 7B, 16 adapters of rank 16, 800 tokens
+ * 576 / 518 us), slower in 192 (at most 12%), all of them prompts of many tiles over 8 adapters or more whose tokens
+ * share few of them, which the host cannot see ((896, 4864), 16 adapters in 6 sets, 4076 tokens 250 / 269 us; each
+ * token its own set 324 / 308 us). Asking for 55 idle groups instead left up to 20% in 295 calls. */
+static bool down_mostly_idle(long tasks, int G, long slots) {
   if (slots < 1 || tasks * G / slots < AOS_SK_MIN_GROUPS) return false;
-  if (tasks * 20 >= (tasks + slots - 1) / slots * slots * 11) return false;
-  return idle_groups(tasks, G, slots) >=
-         (cols > AOS_NARROW_COLS ? AOS_IDLE_DOWN_GROUPS : AOS_IDLE_DOWN_GROUPS_NARROW);
+  return tasks * 20 < (tasks + slots - 1) / slots * slots * 11;
 }
 
 /* Whether a projection alone gains from stream-K: its idle groups must pay for the partial sums' way through
@@ -2021,7 +2012,7 @@ static bool proj_one_launch(const long *tasks, int n, long slots) {
 /* Diagnostic (no counterpart in the reference): the prompt GEMMs' rules above for `tasks` tasks of G groups on
  * `slots` resident workgroups. rule 0: gate/up pieces (tiles token tiles,
  * cols columns, rpad an adapter); 1: a single matrix's pieces; 2: q/k/v's pieces; 3: whether
- * the down GEMM's shrink (cols columns) leaves its launch; 4: whether a projection alone runs as stream-K; 5:
+ * the down GEMM's shrink leaves its launch; 4: whether a projection alone runs as stream-K; 5:
  * whether q, k and v of `tasks`, G and cols tasks run as one launch. */
 extern "C" int aoship_internal_prefill_rule(int rule, int tasks, int G, int cols, int slots, int tiles, int rpad) {
   if (tasks < 1 || G < 1 || cols < 0 || slots < 1 || tiles < 1 || rpad < 0) return set_err("aoship_internal_prefill_rule: bad arguments");
@@ -2030,7 +2021,7 @@ extern "C" int aoship_internal_prefill_rule(int rule, int tasks, int G, int cols
     case 0: return gate_up_pieces(tasks, tiles, G, cols, rpad, slots);
     case 1: return gemm_pieces(tasks, G, slots, 3);
     case 2: return gemm_pieces(tasks, G, slots, 2);
-    case 3: return down_mostly_idle(tasks, G, cols, slots) ? 1 : 0;
+    case 3: return down_mostly_idle(tasks, G, slots) ? 1 : 0;
     case 4: return proj_stream_k(tasks, G, slots) ? 1 : 0;
     case 5: return proj_one_launch(t3, 3, slots) ? 1 : 0;
   }
@@ -2143,7 +2134,7 @@ static void plan_mlp_prefill(aoship_layer *l, int T, const uint16_t *x, const ao
   const int s2 = gemm_pieces(tasks_dn, Wd.G, slots, 3);
   if (M.P.lora && l->prefill_fused_shrink) {
     M.fused_x = s1 == 1 && aos_gemm_shrink_fits(T, Wg.RB, cols_gu, 1) != 0;
-    M.fused_h = s2 == 1 && !((l->prefill_sk & 2) && down_mostly_idle(tasks_dn, Wd.G, tc * rd, slots)) &&
+    M.fused_h = s2 == 1 && !((l->prefill_sk & 2) && down_mostly_idle(tasks_dn, Wd.G, slots)) &&
                 aos_gemm_shrink_fits(T, Wd.RB, tc * rd, 0) != 0;
   }
   plan_tshrink(l, cv, M.P, x, perm, T, H, 0, 2, M.sx, M.fused_x);

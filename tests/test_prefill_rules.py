@@ -31,13 +31,12 @@ def test_pieces_fit_one_round_and_keep_their_groups(rule, slots):
                 assert s == 1 or (s * tasks <= slots and G // s >= 8), (tasks, G, cols, s)
 
 
-# (tokens, hidden, intermediate, columns): the down GEMM's shrink leaves its launch for stream-K, or stays
-@pytest.mark.parametrize("T,H,I,cols,want", [
-    (800, 3584, 18944, 256, 1), (1100, 3584, 18944, 256, 1), (1024, 3072, 8192, 256, 1), (1024, 4096, 11008, 768, 1),
-    (1300, 2048, 5632, 256, 1), (2048, 2048, 5632, 64, 1), (4096, 1024, 2816, 64, 1),
-    (1800, 2048, 5632, 256, 0), (4096, 896, 4864, 256, 0), (3000, 1024, 2816, 512, 0), (1500, 3584, 18944, 256, 0)])
-def test_idle_down(T, H, I, cols, want):
-    assert aoship.prefill_rule("idle_down", _tasks(T, H, 8), I // 64, cols, 256) == want
+# (tokens, hidden, intermediate): the down GEMM's shrink leaves its launch for stream-K, or stays
+@pytest.mark.parametrize("T,H,I,want", [
+    (800, 3584, 18944, 1), (1100, 3584, 18944, 1), (986, 2624, 4480, 1), (1800, 2048, 5632, 1), (4096, 896, 4864, 1),
+    (3000, 1024, 2816, 1), (1500, 3584, 18944, 0), (2048, 3584, 18944, 0), (2300, 2048, 5632, 0), (2048, 1024, 256, 0)])
+def test_idle_down(T, H, I, want):
+    assert aoship.prefill_rule("idle_down", _tasks(T, H, 8), I // 64, 256, 256) == want
 
 
 # (tokens, out, in): o as stream-K where its idle groups pay for the partial sums
