@@ -1305,12 +1305,12 @@ static void gemv_geometry_rows(int RB, int G, int T, bool swiglu, int W, aos_gem
  * splits of a row block). 64 adapters of rank 64, staged before / these waves / the waves above:
  *   q/k/v, 7B shape (144 row blocks) at 4, 8 and 16 tokens: 43, 57, 83 / 40, 50, 63 / 50, 63, 81 us;
  *   o, hidden 5120 (160 row blocks): 39, 44, 79 / 35, 38, 52 / 43, 52, 69 us;
- *   down, 32B shape at 3, 8 and 16 tokens: 61, 115, 205 / 58, 100, 140 / 66, 109, 145 us (20 adapters, 7B shape
- *   at 12 tokens: 61 / 46 / 43 us, hence its wider line);
+ *   down, 32B shape (69k K groups of row blocks) at 3, 8 and 16 tokens: 61, 115, 205 / 58, 100, 140 / 66, 109,
+ *   145 us; smaller ones measure the same in both (30 random calls) and keep their waves;
  *   gate/up, hidden 4096, intermediate 11008, at 12 and 16 tokens: 202, 242 / 140, 157 / 218, 251 us.
- * Projections of at most 8 tokens whose waves would be a single split of each row block take the wide launch from
- * AOS_GEMV_DX_COLS_PROJ8 columns on (o of hidden 4096, 128 row blocks, 12 adapters of rank 64, 8 tokens: 20 us
- * staged, 16 / 21 us here; at 32 tokens the q/k/v launch would lose, 41 / 37 us).
+ * Projections of at most 8 tokens over more than AOS_GEMV_DX_COLS_PROJ8 columns whose 128 to 159 row blocks would be
+ * as many workgroups, half of the chip, take two splits (85 random calls of 520: 5% less with 3 adapters a token
+ * or more, 2% more with 1 or 2; from 160 row blocks on 2% less and 5% more. Four splits: 4% less and 10% more).
  * A wave streams at most AOS_GEMV_DX_MAX_GROUPS groups (down of the 32B shape, 54 groups a wave else, at 9 and 16
  * tokens: 36, 47 us staged / 34, 39 / 37, 51 us).
  * At most 8 tokens stay staged
@@ -1329,6 +1329,7 @@ static void gemv_geometry_rows(int RB, int G, int T, bool swiglu, int W, aos_gem
 #define AOS_GEMV_DX_WAVES_WIDE 2048
 #define AOS_GEMV_DX_WAVES_WIDE_DOWN 1536
 #define AOS_GEMV_DX_COLS_PROJ8 512
+#define AOS_GEMV_DX_FULL_PROJ 160
 #define AOS_GEMV_DX_MAX_GROUPS 48
 #define AOS_GEMV_DX_LARGE_DOWN 60000     /* row blocks times K groups */
 #define AOS_GEMV_DX_LARGE_GATE_UP 100000 /* ... of each of the two matrices */
@@ -1351,11 +1352,12 @@ static int gemv_direct_waves(int kind, int RB, int G, int T, int n, int rpad, in
     return cols > AOS_GEMV_DX_COLS ? AOS_GEMV_DX_WAVES_WIDE : AOS_GEMV_DX_WAVES;
   }
   if (kind == GV_DOWN) {
-    if (cols > AOS_GEMV_DX_COLS_DOWN) return AOS_GEMV_DX_WAVES_WIDE_DOWN;
+    if (cols > AOS_GEMV_DX_COLS_DOWN && groups > AOS_GEMV_DX_LARGE_DOWN) return AOS_GEMV_DX_WAVES_WIDE_DOWN;
     return large ? 0 : AOS_GEMV_DX_WAVES;
   }
-  const bool one_split = 4 * RB >= AOS_GEMV_DX_WAVES_PROJ;
-  if (cols > (T <= 8 && one_split ? AOS_GEMV_DX_COLS_PROJ8 : AOS_GEMV_DX_COLS)) return AOS_GEMV_DX_WAVES_WIDE;
+  if (cols > AOS_GEMV_DX_COLS) return AOS_GEMV_DX_WAVES_WIDE;
+  if (T <= 8 && cols > AOS_GEMV_DX_COLS_PROJ8 && 4 * RB >= AOS_GEMV_DX_WAVES_PROJ && RB < AOS_GEMV_DX_FULL_PROJ)
+    return AOS_GEMV_DX_WAVES;
   return AOS_GEMV_DX_WAVES_PROJ;
 }
 
@@ -1976,7 +1978,7 @@ static double idle_groups(long tasks, int G, long slots) {
  * share it: then its shrink takes a launch of its own rather than that round. Measured both ways on 2174 MLPs (hidden
  * 768 to 4096, intermediate 2048 to 18944, 700 to 4100 tokens in 1 to 24 sets of 2 to 64 adapters, 20 idle groups or
  * more): stream-K is faster by over 1% in 1772 (mean 7%, at most 47%; 7B, 16 adapters of rank 16, 800 tokens
- * 576 / 518 us), slower in 192 (at most 12%), all of them prompts of many tiles over 8 adapters or more whose tokens
+ * 576 / 518 us), slower in 192 (at most 12%), nearly all prompts of many tiles over 8 adapters or more whose tokens
  * share few of them, which the host cannot see ((896, 4864), 16 adapters in 6 sets, 4076 tokens 250 / 269 us; each
  * token its own set 324 / 308 us). Asking for 55 idle groups instead left up to 20% in 295 calls. */
 static bool down_mostly_idle(long tasks, int G, long slots) {

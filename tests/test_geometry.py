@@ -63,6 +63,16 @@ def test_wide_unions_get_more_waves(kind, rb, G, T):
     assert narrow == line and (2 * wide >= 3 * narrow or -(-G // (4 * wide)) <= 48), (narrow, line, wide)
 
 
+# (kind, row blocks, K groups, tokens, adapters, rank, splits): more splits only where they were measured to pay
+@pytest.mark.parametrize("kind,rb,G,T,n,r,ks", [
+    (2, 128, 64, 8, 12, 64, 2), (2, 159, 64, 3, 24, 32, 2), (2, 160, 64, 8, 12, 64, 1), (2, 234, 26, 3, 19, 32, 1),
+    (2, 322, 18, 7, 60, 16, 1), (2, 127, 64, 8, 12, 64, 2), (2, 128, 64, 8, 8, 64, 1), (2, 128, 64, 9, 12, 64, 1),
+    (1, 112, 296, 16, 64, 64, 3), (1, 32, 147, 20, 49, 32, 8), (1, 160, 432, 16, 64, 64, 3), (1, 160, 432, 16, 16, 16, 3)])
+def test_splits_of_launches_over_wide_tables(kind, rb, G, T, n, r, ks):
+    direct, _, got, _, _ = aoship.decode_launch(kind, 32 * rb, 64 * G, T, n=n, rpad=r)
+    assert direct and got == ks
+
+
 @pytest.mark.parametrize("T", range(3, 33))
 def test_every_wave_of_a_pinned_staged_launch_gets_a_group(T):
     """Pinned to any one row split, the launches stage x: 8 waves over a long K with up to 64 KB of it."""
